@@ -1,0 +1,448 @@
+"""The work a user of simdyolo_amd has it do, as cases that can be timed: single
+layers through the op entry points (convolutions, depthwise, pooling,
+attention, head decode, top-k) and whole YOLOv8n forwards.  Shapes are those of
+the YOLOv8 / YOLO11 / YOLO26 families at network inputs between 320 and 640
+pixels, batches from one camera frame to the 32-image batch of bench.py.
+"""
+import math
+
+import numpy as np
+import torch
+import torch.nn.functional as F
+
+from simdyolo_amd import Tensor, synth
+from simdyolo_amd import _native as N
+from simdyolo_amd.detector import YoloDetector
+from simdyolo_amd.device import HipContext
+
+
+def listed():
+    return [
+        # A bottleneck convolution of one frame: latency, a handful of workgroups.
+        dict(name="conv3x3 64 40x40 b1", kind="conv", k=3, stride=1, n=1, ic=64, oc=64, h=40, w=40, residual=True),
+        # The class branch of the detect head at stride 8 for 600x360 frames: 80 channels, odd height.
+        dict(name="conv3x3 80 45x75 b4", kind="conv", k=3, stride=1, n=4, ic=80, oc=80, h=45, w=75, residual=False),
+        # The detect head's box branch at stride 8 for a full batch, the largest 3x3 layer of YOLOv8n.
+        dict(name="conv3x3 64 80x80 b32", kind="conv", k=3, stride=1, n=32, ic=64, oc=64, h=80, w=80, residual=False),
+        # A downsampling layer of the backbone for a full batch.
+        dict(name="conv3x3 s2 64-128 80x80 b32", kind="conv", k=3, stride=2, n=32, ic=64, oc=128, h=80, w=80,
+             residual=False),
+        # A C2f's closing 1x1 over its concatenated parts, a part-filled batch of 4:3 frames.
+        dict(name="conv1x1 192-128 30x40 b7", kind="conv", k=1, stride=1, n=7, ic=192, oc=128, h=30, w=40,
+             residual=False),
+        # The same layer family for a full batch at stride 16.
+        dict(name="conv1x1 384-128 40x40 b32", kind="conv", k=1, stride=1, n=32, ic=384, oc=128, h=40, w=40,
+             residual=False),
+        # The depthwise layer of YOLO11's class branch.
+        dict(name="depthwise 64 80x80 b32", kind="depthwise", n=32, c=64, h=80, w=80),
+        # C2PSA attention of YOLO11n at 640x640 (400 tokens).
+        dict(name="attention 2x64 20x20 b16", kind="attention", n=16, heads=2, kd=32, hd=64, h=20, w=20),
+        # Joined head decode of YOLOv8n, half a batch.
+        dict(name="decode 640x640 b16", kind="decode", n=16, h=640, w=640, bins=16, nc=80),
+        # YOLO26's end-to-end selection, one frame.
+        dict(name="topk 8400 b1", kind="topk", n=1, anchors=8400, nc=80, extra=0, keep=300),
+        # One frame from host memory and back, the call of an interactive program.
+        dict(name="yolov8n 640x640 b1 host", kind="model", n=1, h=640, w=640, host=True),
+        # The headline workload: a resident 32-image batch.
+        dict(name="yolov8n 640x640 b32", kind="model", n=32, h=640, w=640, host=False),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    """One more case: mostly convolutions, as in the networks."""
+    kind = rng.choices(["conv3", "down", "conv1", "depthwise", "attention", "decode", "topk", "model"],
+                       [4, 2, 4, 1, 1, 1, 1, 1])[0]
+    while True:
+        n, h, w = _log(rng, 1, 32), _log(rng, 10, 160), _log(rng, 10, 160)
+        if kind in ("conv3", "down", "conv1"):
+            # Channel counts of the n, s and m scales, and the 80 classes.
+            widths = [16, 24, 32, 48, 64, 80, 96, 128, 192, 256]
+            ic, oc = rng.choice(widths), rng.choice(widths)
+            if kind == "conv3" and rng.random() < 0.6:
+                oc = ic
+            if kind == "conv1":
+                ic *= rng.choice([1, 2, 3])
+            case = dict(kind="conv", k=1 if kind == "conv1" else 3, stride=2 if kind == "down" else 1, n=n, ic=ic,
+                        oc=oc, h=h, w=w, residual=kind == "conv3" and ic == oc and rng.random() < 0.5)
+        elif kind == "depthwise":
+            case = dict(kind=kind, n=n, c=rng.choice([16, 32, 64, 80, 128, 256]), h=h, w=w)
+        elif kind == "attention":
+            case = dict(kind=kind, n=n, heads=rng.choice([2, 4]), kd=32, hd=64, h=_log(rng, 7, 40),
+                        w=_log(rng, 7, 40))
+        elif kind == "decode":
+            case = dict(kind=kind, n=n, h=32 * rng.randint(3, 20), w=32 * rng.randint(3, 20),
+                        bins=rng.choice([1, 16]), nc=rng.choice([1, 20, 80]))
+        elif kind == "topk":
+            case = dict(kind=kind, n=n, anchors=_log(rng, 400, 33600), nc=rng.choice([1, 20, 80]),
+                        extra=rng.choice([0, 32]), keep=rng.choice([100, 300]))
+        else:
+            case = dict(kind=kind, n=n, h=32 * rng.randint(10, 20), w=32 * rng.randint(10, 20),
+                        host=rng.random() < 0.3)
+        cost = work(case)
+        if cost["bytes"] < 1.0e9 and cost["flops"] < (300e9 if kind == "model" else 60e9):
+            return case
+
+
+# ------------------------------------------------------------------ inputs
+
+_context = None
+
+
+def _ctx():
+    """One context for the process, as a program has."""
+    global _context
+    if _context is None:
+        _context = HipContext(0)
+    return _context
+
+
+class _State:
+    def __init__(self, **kw):
+        self.__dict__.update(kw)
+
+    def __del__(self):
+        det = self.__dict__.get("det")
+        if det is not None:
+            torch.cuda.synchronize()
+            det.close()
+
+
+def _gen(seed):
+    return torch.Generator(device="cuda").manual_seed(seed)
+
+
+def _normal(seed, *shape):
+    return torch.randn(shape, generator=_gen(seed), device="cuda")
+
+
+def _view(t):
+    """The NHWC view of a torch [n, h, w, c] tensor whose channels are contiguous."""
+    n, h, w, c = t.shape
+    return Tensor(t.data_ptr(), n, c, h, w, t.stride(2), N.LAYOUT_NHWC)
+
+
+def _weights(case, seed):
+    """OIHW weights (Kaiming) and a bias, as folded from a trained layer."""
+    icg = 1 if case["kind"] == "depthwise" else case["ic"]
+    oc = case["c"] if case["kind"] == "depthwise" else case["oc"]
+    k = 3 if case["kind"] == "depthwise" else case["k"]
+    w = _normal(seed + 1000003, oc, icg, k, k) * math.sqrt(2.0 / (icg * k * k))
+    b = _normal(seed + 2000003, oc) * 0.1
+    return w, b
+
+
+def _feature(seed, n, h, w, c):
+    """Activations behind a SiLU, as every layer but the first reads."""
+    return F.silu(_normal(seed, n, h, w, c))
+
+
+def _levels(case, seed):
+    """Raw NHWC heads of the three detect levels: box logits, then class logits around the usual prior."""
+    c = 4 * case["bins"]
+    got = []
+    for i, s in enumerate((8, 16, 32)):
+        t = _normal(seed + 17 * i, case["n"], case["h"] // s, case["w"] // s, c + case["nc"])
+        t[..., c:] = t[..., c:] * 1.5 - 4.6
+        got.append(t)
+    return got
+
+
+def _anchors(case):
+    return sum((case["h"] // s) * (case["w"] // s) for s in (8, 16, 32))
+
+
+def _images(case, seed):
+    u8 = torch.randint(0, 256, (case["n"], 3, case["h"], case["w"]), generator=_gen(seed), device="cuda",
+                       dtype=torch.uint8)
+    return u8.float() / 255.0
+
+
+class _Borrowed:
+    """Device memory of the library, as torch.as_tensor takes it."""
+
+    def __init__(self, ptr, shape):
+        self.__cuda_array_interface__ = dict(data=(ptr, False), shape=tuple(shape), typestr="<f4", version=2)
+
+
+def _params(seed):
+    cfg = synth.config("n")
+    return cfg, synth.params(cfg, seed)
+
+
+def prepare(case, seed):
+    ctx, kind = _ctx(), case["kind"]
+    s = _State(case=case)
+    if kind == "conv":
+        w, b = _weights(case, seed)
+        k, st, n, ic, oc = case["k"], case["stride"], case["n"], case["ic"], case["oc"]
+        s.conv = ctx.conv_create(w.cpu().numpy(), b.cpu().numpy(), (st, st), (k // 2,) * 4, silu=True)
+        oh, ow = ctx.conv_out_size(s.conv, case["h"], case["w"])
+        if case["residual"]:
+            # A C2f's bottleneck: input, shortcut and output are slices of its concat buffer.
+            s.buffer = torch.zeros((n, oh, ow, 3 * oc), device="cuda")
+            s.x, s.y = s.buffer[..., oc:2 * oc], s.buffer[..., 2 * oc:]
+            s.x.copy_(_feature(seed, n, oh, ow, oc))
+        else:
+            s.x = _feature(seed, n, case["h"], case["w"], ic)
+            s.y = torch.zeros((n, oh, ow, oc), device="cuda")
+        s.vx, s.vy = _view(s.x), _view(s.y)
+        s.vres = s.vx if case["residual"] else None
+    elif kind == "depthwise":
+        w, b = _weights(case, seed)
+        s.conv = ctx.conv_create(w.cpu().numpy(), b.cpu().numpy(), (1, 1), (1, 1, 1, 1), groups=case["c"], silu=True)
+        s.x = _feature(seed, case["n"], case["h"], case["w"], case["c"])
+        s.y = torch.zeros_like(s.x)
+        s.vx, s.vy, s.vres = _view(s.x), _view(s.y), None
+    elif kind == "attention":
+        heads, kd, hd = case["heads"], case["kd"], case["hd"]
+        s.x = _normal(seed, case["n"], case["h"], case["w"], heads * (2 * kd + hd))
+        s.o = torch.zeros((case["n"], case["h"], case["w"], heads * hd), device="cuda")
+        s.v = torch.zeros_like(s.o)
+        s.vx, s.vo, s.vv = _view(s.x), _view(s.o), _view(s.v)
+    elif kind == "decode":
+        s.levels = _levels(case, seed)
+        s.views = [_view(t) for t in s.levels]
+        s.y = torch.zeros((case["n"], 4 + case["nc"], _anchors(case)), device="cuda")
+    elif kind == "topk":
+        g = _normal(seed, case["n"], 4 + case["nc"] + case["extra"], case["anchors"])
+        g[:, :4] = g[:, :4].abs() * 100.0
+        g[:, 4:4 + case["nc"]] = torch.sigmoid(g[:, 4:4 + case["nc"]] * 1.5 - 4.6)
+        s.x = g
+        s.y = torch.zeros((case["n"], min(case["keep"], case["anchors"]), 6 + case["extra"]), device="cuda")
+    else:
+        n, h, w = case["n"], case["h"], case["w"]
+        cfg, params = _params(seed)
+        s.det = YoloDetector(cfg, params, ctx=ctx)
+        s.x = _images(case, seed)
+        if case["host"]:
+            s.x = s.x.cpu().numpy()
+            for _ in range(2):
+                s.det.predict_raw(s.x)
+        else:
+            inp, out = s.det.buffers(n, h, w)
+            torch.as_tensor(_Borrowed(inp, s.x.shape), device="cuda").copy_(s.x)
+            s.y = torch.as_tensor(_Borrowed(out, s.det.output_shape(n, h, w)), device="cuda")
+    torch.cuda.synchronize()
+    if kind != "model" or not case["host"]:
+        # Warm, as a program's layers and plans are: a shape's first calls time its candidates.
+        for _ in range(2):
+            run(s)
+        ctx.flush()
+    return s
+
+
+# -------------------------------------------------------------------- pass
+
+def run(s):
+    case, kind, ctx = s.case, s.case["kind"], _context
+    if kind in ("conv", "depthwise"):
+        ctx.conv(s.conv, s.vx, s.vy, s.vres)
+        return s.y
+    if kind == "attention":
+        ctx.attention(s.vx, case["heads"], case["kd"], case["hd"], case["kd"] ** -0.5, s.vo, s.vv)
+        return s.o, s.v
+    if kind == "decode":
+        ctx.detect_decode(s.views, (8.0, 16.0, 32.0), case["bins"], case["nc"], False, s.y.data_ptr(), s.y.shape[2])
+        return s.y
+    if kind == "topk":
+        ctx.e2e_topk(s.x.data_ptr(), case["n"], s.x.shape[1], case["anchors"], case["nc"], case["keep"], False,
+                     s.y.data_ptr())
+        return s.y
+    if case["host"]:
+        return s.det.predict_raw(s.x)
+    s.det.run(case["n"], case["h"], case["w"])
+    return s.y
+
+
+def _out_hw(case):
+    k, st = case["k"], case["stride"]
+    return tuple((case[d] + 2 * (k // 2) - k) // st + 1 for d in ("h", "w"))
+
+
+def work(case):
+    kind, n = case["kind"], case["n"]
+    px = n * case.get("h", 1) * case.get("w", 1)
+    if kind == "conv":
+        oh, ow = _out_hw(case)
+        k2, ic, oc = case["k"] ** 2, case["ic"], case["oc"]
+        return {"bytes": 4 * (px * ic + n * oh * ow * oc + k2 * ic * oc + oc), "flops": 2 * n * oh * ow * oc * ic * k2}
+    if kind == "depthwise":
+        return {"bytes": 4 * (2 * px * case["c"] + 10 * case["c"]), "flops": 18 * px * case["c"]}
+    if kind == "attention":
+        heads, kd, hd, t = case["heads"], case["kd"], case["hd"], case["h"] * case["w"]
+        return {"bytes": 4 * n * t * heads * (2 * kd + 3 * hd), "flops": 2 * n * heads * t * t * (kd + hd)}
+    if kind == "decode":
+        a = n * _anchors(case)
+        return {"bytes": 4 * a * (4 * case["bins"] + 2 * case["nc"] + 4), "flops": 4 * a * (4 * case["bins"] + case["nc"])}
+    if kind == "topk":
+        k = min(case["keep"], case["anchors"])
+        return {"bytes": 4 * n * (case["anchors"] * case["nc"] + 2 * k * (6 + case["extra"])),
+                "flops": n * case["anchors"] * case["nc"]}
+    # YOLOv8n: 8.743 GFLOP and 8400 anchors for each 640x640 image, 12.58 MB of weights; input and head move once.
+    area = px / 409600.0
+    return {"bytes": 12.58e6 + 4 * (3 * px + area * 84 * 8400), "flops": 8.743e9 * area}
+
+
+def tolerance(case):
+    """Four times what float32 arithmetic in another order was measured to give."""
+    kind = case["kind"]
+    if kind == "topk":
+        return "exact"  # rows are copies of the input
+    if kind == "conv" and case["k"] == 3 and case["stride"] == 1:
+        return {"rel": 8e-6}  # Winograd F(4x4, 3x3) may be taken
+    return {"rel": 2e-5 if kind == "model" else 4e-6}
+
+
+# -------------------------------------------------- the same in 64 bits
+
+def _conv64(x, w, b, stride=1, act=True):
+    """x [n, c, h, w] and w in float64; one image at a time, as one matrix product."""
+    oc, ic, k, _ = w.shape
+    oh, ow = ((d + 2 * (k // 2) - k) // stride + 1 for d in x.shape[2:])
+    y = torch.empty((x.shape[0], oc, oh, ow), dtype=torch.float64, device=x.device)
+    for i in range(x.shape[0]):
+        cols = F.unfold(x[i:i + 1], k, padding=k // 2, stride=stride)[0] if k > 1 or stride > 1 else x[i].flatten(1)
+        y[i] = (w.reshape(oc, -1) @ cols + b[:, None]).reshape(oc, oh, ow)
+    return y * torch.sigmoid(y) if act else y
+
+
+def _decode64(levels, bins):
+    """[n, 4 + nc, anchors] from NCHW float64 heads at strides 8, 16, 32."""
+    parts = []
+    for t, s in zip(levels, (8, 16, 32)):
+        n, _, h, w = t.shape
+        box = t[:, :4 * bins].reshape(n, 4, bins, h, w)
+        if bins > 1:
+            grid = torch.arange(bins, dtype=torch.float64, device=t.device)[:, None, None]
+            box = (torch.softmax(box, 2) * grid).sum(2)
+        else:
+            box = box[:, :, 0]
+        gy = torch.arange(h, dtype=torch.float64, device=t.device)[:, None] + 0.5
+        gx = torch.arange(w, dtype=torch.float64, device=t.device)[None, :] + 0.5
+        x1, y1, x2, y2 = gx - box[:, 0], gy - box[:, 1], gx + box[:, 2], gy + box[:, 3]
+        xywh = torch.stack([(x1 + x2) / 2, (y1 + y2) / 2, x2 - x1, y2 - y1], 1) * s
+        parts.append(torch.cat([xywh, torch.sigmoid(t[:, 4 * bins:])], 1).flatten(2))
+    return torch.cat(parts, 2)
+
+
+class _Parameters:
+    """Walks YOLOv8n's tensors in state_dict order."""
+
+    def __init__(self, flat, eps):
+        self.flat, self.at, self.eps = flat, 0, eps
+
+    def take(self, *shape):
+        n = math.prod(shape)
+        v = torch.from_numpy(self.flat[self.at:self.at + n].astype(np.float64)).cuda().reshape(shape)
+        self.at += n
+        return v
+
+    def conv(self, oc, ic, k):
+        """Conv2d without bias, then BatchNorm; folded."""
+        w = self.take(oc, ic, k, k)
+        g, b, m, v = (self.take(oc) for _ in range(4))
+        f = g / torch.sqrt(v + self.eps)
+        return w * f[:, None, None, None], b - m * f
+
+
+def _yolov8n64(flat, eps, x, nc=80):
+    P = _Parameters(flat, eps)
+    ops = []  # parameters are taken in module order, so the layers are read first
+
+    def conv(oc, ic, k, s=1):
+        w, b = P.conv(oc, ic, k)
+        return lambda t: _conv64(t, w, b, s)
+
+    def c2f(ic, oc, n, shortcut):
+        c = oc // 2
+        cv1, cv2 = conv(oc, ic, 1), conv(oc, (2 + n) * c, 1)
+        m = [(conv(c, c, 3), conv(c, c, 3)) for _ in range(n)]
+
+        def f(t):
+            y = list(cv1(t).chunk(2, 1))
+            for a, b in m:
+                z = b(a(y[-1]))
+                y.append(y[-1] + z if shortcut else z)
+            return cv2(torch.cat(y, 1))
+        return f
+
+    def sppf(c):
+        cv1, cv2 = conv(c // 2, c, 1), conv(c, 2 * c, 1)
+
+        def f(t):
+            y = [cv1(t)]
+            for _ in range(3):
+                y.append(F.max_pool2d(y[-1].cpu(), 5, 1, 2).to(t.device))
+            return cv2(torch.cat(y, 1))
+        return f
+
+    for layer in [(conv, 16, 3, 3, 2), (conv, 32, 16, 3, 2), (c2f, 32, 32, 1, True), (conv, 64, 32, 3, 2),
+                  (c2f, 64, 64, 2, True), (conv, 128, 64, 3, 2), (c2f, 128, 128, 2, True), (conv, 256, 128, 3, 2),
+                  (c2f, 256, 256, 1, True), (sppf, 256), (c2f, 384, 128, 1, False), (c2f, 192, 64, 1, False),
+                  (conv, 64, 64, 3, 2), (c2f, 192, 128, 1, False), (conv, 128, 128, 3, 2), (c2f, 384, 256, 1, False)]:
+        ops.append(layer[0](*layer[1:]))
+
+    def branch(ic, mid, out):
+        a, b = conv(mid, ic, 3), conv(mid, mid, 3)
+        w, bias = P.take(out, mid, 1, 1), P.take(out)
+        return lambda t: _conv64(b(a(t)), w, bias, act=False)
+
+    box = [branch(c, 64, 64) for c in (64, 128, 256)]
+    cls = [branch(c, 80, nc) for c in (64, 128, 256)]
+
+    def up(t):
+        return t.repeat_interleave(2, 2).repeat_interleave(2, 3)
+
+    t, saved = x, {}
+    for i in range(10):
+        t = ops[i](t)
+        saved[i] = t
+    p4 = ops[10](torch.cat([up(saved[9]), saved[6]], 1))
+    p3 = ops[11](torch.cat([up(p4), saved[4]], 1))
+    q4 = ops[13](torch.cat([ops[12](p3), p4], 1))
+    q5 = ops[15](torch.cat([ops[14](q4), saved[9]], 1))
+    return _decode64([torch.cat([b(q), c(q)], 1) for b, c, q in zip(box, cls, (p3, q4, q5))], 16)
+
+
+def _nchw64(t):
+    return t.permute(0, 3, 1, 2).double()
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "conv":
+        w, b = _weights(case, seed)
+        x = _feature(seed, case["n"], case["h"], case["w"], case["ic"])
+        y = torch.cat([_conv64(_nchw64(x[i:i + 1]), w.double(), b.double(), case["stride"]).permute(0, 2, 3, 1)
+                       for i in range(case["n"])])
+        return y + x.double() if case["residual"] else y
+    if kind == "depthwise":
+        w, b = _weights(case, seed)
+        x = F.pad(_nchw64(_feature(seed, case["n"], case["h"], case["w"], case["c"])), (1, 1, 1, 1))
+        h, wd = case["h"], case["w"]
+        y = b.double()[:, None, None] + sum(w[:, 0, i, j].double()[:, None, None] * x[:, :, i:i + h, j:j + wd]
+                                            for i in range(3) for j in range(3))
+        return (y * torch.sigmoid(y)).permute(0, 2, 3, 1)
+    if kind == "attention":
+        n, heads, kd, hd, t = case["n"], case["heads"], case["kd"], case["hd"], case["h"] * case["w"]
+        x = _normal(seed, n, case["h"], case["w"], heads * (2 * kd + hd)).double().reshape(n, t, heads, 2 * kd + hd)
+        q, k, v = x.split([kd, kd, hd], 3)
+        o = torch.empty((n, t, heads, hd), dtype=torch.float64, device="cuda")
+        for i in range(n):
+            for j in range(heads):
+                a = torch.softmax(q[i, :, j] @ k[i, :, j].T.contiguous() * float(np.float32(kd ** -0.5)), 1)
+                o[i, :, j] = a @ v[i, :, j]
+        shape = (n, case["h"], case["w"], heads * hd)
+        return o.reshape(shape), v.reshape(shape)
+    if kind == "decode":
+        return _decode64([_nchw64(t) for t in _levels(case, seed)], case["bins"])
+    if kind == "topk":
+        return None  # rows are copies of the input
+    if case["n"] * case["h"] * case["w"] > 8 * 640 * 640:
+        return None  # minutes in float64
+    cfg, params = _params(seed)
+    return _yolov8n64(params, cfg.bn_eps, _images(case, seed).double())
