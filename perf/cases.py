@@ -104,11 +104,16 @@ class _State:
     def __init__(self, **kw):
         self.__dict__.update(kw)
 
+
+class _Model:
+    """A detector that closes when neither a state nor a returned output refers to it."""
+
+    def __init__(self, det):
+        self.det = det
+
     def __del__(self):
-        det = self.__dict__.get("det")
-        if det is not None:
-            torch.cuda.synchronize()
-            det.close()
+        torch.cuda.synchronize()
+        self.det.close()
 
 
 def _gen(seed):
@@ -162,9 +167,10 @@ def _images(case, seed):
 
 
 class _Borrowed:
-    """Device memory of the library, as torch.as_tensor takes it."""
+    """Device memory of a model, as torch.as_tensor takes it; the tensor keeps this object, and so the model."""
 
-    def __init__(self, ptr, shape):
+    def __init__(self, ptr, shape, model):
+        self.model = model
         self.__cuda_array_interface__ = dict(data=(ptr, False), shape=tuple(shape), typestr="<f4", version=2)
 
 
@@ -217,6 +223,7 @@ def prepare(case, seed):
         n, h, w = case["n"], case["h"], case["w"]
         cfg, params = _params(seed)
         s.det = YoloDetector(cfg, params, ctx=ctx)
+        s.model = _Model(s.det)
         s.x = _images(case, seed)
         if case["host"]:
             s.x = s.x.cpu().numpy()
@@ -224,8 +231,8 @@ def prepare(case, seed):
                 s.det.predict_raw(s.x)
         else:
             inp, out = s.det.buffers(n, h, w)
-            torch.as_tensor(_Borrowed(inp, s.x.shape), device="cuda").copy_(s.x)
-            s.y = torch.as_tensor(_Borrowed(out, s.det.output_shape(n, h, w)), device="cuda")
+            torch.as_tensor(_Borrowed(inp, s.x.shape, s.model), device="cuda").copy_(s.x)
+            s.y = torch.as_tensor(_Borrowed(out, s.det.output_shape(n, h, w), s.model), device="cuda")
     torch.cuda.synchronize()
     if kind != "model" or not case["host"]:
         # Warm, as a program's layers and plans are: a shape's first calls time its candidates.
