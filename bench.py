@@ -57,6 +57,7 @@ SYMBOLS = {"wino_input": "sy::wino_in_kernel<4>", "wino_input_blk": "sy::wino_in
 def symbol(name):
     """rocprofv3 symbol of a library profile name: igemm_m<mode>_<bm>x<bn>_<wm><wn>_k<bk>[_p<pf>] or
     wino_gemm_<bm>x<bn>_<wm><wn>_k<bk>[_p<pf>] (pf: K tiles loaded ahead, 1 when absent),
+    igemm_m<mode>_x3_<bm>x<bn>_<wm><wn> and conv3_x3_<pixels>x<channels>_<waves> (f16-split kernels),
     pw_gemm_n<32*NW> / wino_pw_n<32*NW> (the K-chunk template argument depends on the layer,
     written *), or a fixed kernel."""
     m = re.fullmatch(r"(igemm_m(\d)|wino_gemm)_(\d+)x(\d+)_(\d)(\d)_k(\d+)(?:_p(\d))?", name)
@@ -65,6 +66,11 @@ def symbol(name):
         pf = m.group(8) or "1"
         return (f"sy::igemm_kernel<{kind}, {mode}, {m.group(3)}, {m.group(4)}, {m.group(5)}, {m.group(6)}, "
                 f"{m.group(7)}, {pf}>")
+    m = re.fullmatch(r"igemm_m(\d)_x3_(\d+)x(\d+)_(\d)(\d)", name)
+    if m:
+        return "sy::x3_kernel<" + ", ".join(m.groups()) + ">"
+    if name.startswith("conv3_x3_"):
+        return "sy::conv3_kernel<*>"
     m = re.fullmatch(r"(pw_gemm|wino_pw)_n(\d+)", name)
     if m:
         return f"sy::pw_kernel<{int(m.group(2)) // 32}, *>"

@@ -21,135 +21,10 @@
 #include <string>
 #include <utility>
 
+#include "igemm.h"
 #include "sy_internal.h"
 
 namespace sy {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ float silu_f(float v) { return v / (1.0f + __expf(-v)); }
-// SiLU with the hardware reciprocal (within 1 ulp of the division) for GEMM
-// epilogues, where the IEEE division sequence is a large share of the VALU.
-__device__ __forceinline__ float silu_fast(float v) { return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v)); }
-
-// ------------------------------------------------------------ implicit GEMM
-
-struct IgemmArgs {
-  const float* x;
-  int N, H, W, IC, ldx;
-  const float* w;
-  int Kp;
-  const float* bias;
-  const float* res;
-  int ldr;
-  float* y;
-  int OH, OW, OC, ldy;
-  int KH, KW, SH, SW, PH, PW, DH, DW;
-  int K, M, silu;
-  long long xb, wb, yb;  // per-blockIdx.z strides (floats) for batched GEMMs
-  int Nb, bguard;        // B rows present; check B reads against Nb and K
-  int shuf = 0;          // > 0: column q * shuf + o goes to pixel (2y + q/2, 2x + q%2), channel o
-  // Split K: workgroup z sums k in [z * kchunk, (z + 1) * kchunk) and stores
-  // the raw partial tile to part[z][m][ldp]; splitk_reduce_kernel finishes.
-  float* part = nullptr;
-  int kchunk = 0, ldp = 0;
-  // MODE 3 (1x1 over concat(upsample2x(xu), x)): K columns [0, ku) of row
-  // (n, oy, ox) come from xu's pixel (n, oy / 2, ox / 2) of an (H/2) x (W/2)
-  // image, columns [ku, K) from x's row (x points at that part's first
-  // channel).  ku is a whole number of K tiles.
-  const float* xu = nullptr;
-  int ldxu = 0, ku = 0;
-};
-
-// Epilogue of a GEMM tile: y = [res +] act(acc + bias) for the 32x32 MFMA
-// blocks of one wave.  rbase is the wave's first output row (plus the lane
-// half's 4-row offset), col0 its first column plus the lane's column.  D
-// layout of the 32x32 MFMA: lane holds column (lane & 31) and rows
-// 8*(r/4) + 4*(lane/32) + (r%4) for r = 0..15.  Every bias and residual
-// value is loaded before the first store: a wait for a load also waits for
-// the stores issued before it, so interleaving them would serialise the
-// stores' round trips.
-template <int TM, int TN>
-__device__ __forceinline__ void store_acc(const IgemmArgs& a, float* __restrict__ y, const f32x16 (&acc)[TM][TN],
-                                          int rbase, int col0) {
-  float bv[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) bv[j] = (a.bias && col0 + j * 32 < a.OC) ? a.bias[col0 + j * 32] : 0.f;
-  // A wave tile wholly inside the output (every row below M, every column
-  // below OC) stores without per-element tests: one branch for the tile
-  // instead of one per store.
-  const bool inner = rbase - 4 * ((threadIdx.x & 63) >> 5) + TM * 32 <= a.M &&
-                     col0 - (threadIdx.x & 31) + TN * 32 <= a.OC;
-  if (__builtin_amdgcn_readfirstlane((int)inner)) {
-    float v[TM][TN][16];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float t = acc[i][j][r] + bv[j];
-          v[i][j][r] = a.silu ? silu_fast(t) : t;
-        }
-    if (a.res) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const float* rr = a.res + (long long)(rbase + i * 32) * a.ldr + col0 + j * 32;
-          float rv[16];
-#pragma unroll
-          for (int r = 0; r < 16; ++r) rv[r] = rr[(8 * (r >> 2) + (r & 3)) * a.ldr];
-#pragma unroll
-          for (int r = 0; r < 16; ++r) v[i][j][r] = rv[r] + v[i][j][r];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        float* yr = y + (long long)(rbase + i * 32) * a.ldy + col0 + j * 32;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) yr[(8 * (r >> 2) + (r & 3)) * a.ldy] = v[i][j][r];
-      }
-    return;
-  }
-  float rv[TM][TN][16];
-  if (a.res) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int col = col0 + j * 32, row0 = rbase + i * 32;
-        const float* rr = a.res + (long long)row0 * a.ldr + col;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int dr = 8 * (r >> 2) + (r & 3);
-          rv[i][j][r] = (col < a.OC && row0 + dr < a.M) ? rr[dr * a.ldr] : 0.f;
-        }
-      }
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int col = col0 + j * 32;
-    if (col >= a.OC) continue;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int row0 = rbase + i * 32;
-      float* yr = y + (long long)row0 * a.ldy + col;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int dr = 8 * (r >> 2) + (r & 3);
-        if (row0 + dr >= a.M) continue;
-        float v = acc[i][j][r] + bv[j];
-        if (a.silu) v = silu_fast(v);
-        if (a.res) v = rv[i][j][r] + v;
-        yr[dr * a.ldy] = v;
-      }
-    }
-  }
-}
 
 // KIND only separates the instantiations by caller (0 convolution, 1 Winograd
 // plane GEMM, 2 plain GEMM) so that profilers report them apart.  MODE picks
@@ -401,29 +276,7 @@ __global__ __launch_bounds__(WM* WN * 64, (BM * BN <= 64 * 64 && WM * WN == 4)  
     return;
   }
   if (MODE == 2 && a.shuf > 0) {
-    // Transposed 2x2 stride-2 conv: scatter each column to its sub-pixel.
-    const int hw = a.H * a.W;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = n0 + wn * (BN / WN) + j * 32 + r32;
-      if (col >= a.OC) continue;
-      const float bv = a.bias ? a.bias[col] : 0.f;
-      const int q = col / a.shuf, o = col - q * a.shuf;
-      const int dy = q >> 1, dx = q & 1;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = rbase + i * 32 + 8 * (r >> 2) + (r & 3);
-          if (row >= a.M) continue;
-          const int n = row / hw, rem = row - n * hw;
-          const int yy = rem / a.W, xx = rem - yy * a.W;
-          const long long pix = ((long long)n * 2 * a.H + 2 * yy + dy) * (2 * a.W) + 2 * xx + dx;
-          float v = acc[i][j][r] + bv;
-          if (a.silu) v = silu_fast(v);
-          y[pix * a.ldy + o] = v;
-        }
-    }
+    store_shuf<TM, TN>(a, y, acc, rbase, n0 + wn * (BN / WN) + r32);
     return;
   }
   store_acc<TM, TN>(a, y, acc, rbase, n0 + wn * (BN / WN) + r32);
@@ -1208,6 +1061,15 @@ static int launch_igemm(sy_ctx* ctx, const IgemmArgs& a, int batch, bool wino, d
                                : (a.OC == 16 ? "conv3x3_c16_oc16_s2" : "conv3x3_c16_oc32_s2");
     ProfScope prof(ctx, pn, flops, bytes);
     SY_TRY(launch_c16(ctx, a));
+    return check_launch(pn);
+  }
+  if (is_x3_tile(ft) && batch == 1 && !name && !wino) {
+    const int mode = rows ? (a.ku > 0 ? 3 : 2) : (a.IC % 32 == 0 && (long long)a.H * a.W * a.ldx < (1LL << 31) ? 1 : 0);
+    SY_CHECK(a.ku == 0 || (rows && a.ku % 32 == 0), SY_EINVAL,
+             "an upsampled input part needs a plain 1x1 GEMM whose K tile divides it");
+    const char* pn = x3_name(ft, mode);
+    ProfScope prof(ctx, pn, flops, bytes);
+    SY_TRY(launch_x3(ctx, ft, mode, a));
     return check_launch(pn);
   }
   if (is_ks_tile(ft) && batch == 1 && !name && !wino && a.ku == 0) {
@@ -2799,13 +2661,17 @@ static bool fused_wino_fits(const sy_tensor* x) {
   return 4 * img * (31 / tpi + 2) < kFxOob;
 }
 
+// 3x3 stride-1 pad-1 undilated ungrouped convolution on whole float4s.
+static bool conv3x3_s1(const ConvPlan* p) {
+  return p->groups == 1 && p->kh == 3 && p->kw == 3 && p->sh == 1 && p->sw == 1 && p->dh == 1 && p->dw == 1 &&
+         p->pt == 1 && p->pl == 1 && p->pb == 1 && p->pr == 1 && p->ic % 4 == 0;
+}
+
 bool conv_supports(const ConvPlan* p, int algo) {
   const bool g1 = p->groups == 1;
   switch (algo) {
     case kIgemm: return g1 && p->ic % 4 == 0;
-    case kWinograd:
-      return g1 && p->kh == 3 && p->kw == 3 && p->sh == 1 && p->sw == 1 && p->dh == 1 && p->dw == 1 && p->pt == 1 &&
-             p->pl == 1 && p->pb == 1 && p->pr == 1 && p->ic % 4 == 0 && p->oc % 4 == 0;
+    case kWinograd: return conv3x3_s1(p) && p->oc % 4 == 0;
     case kDirect: return g1 && p->kh * p->kw * p->ic <= 1024;
     case kWinograd3: return conv_supports(p, kWinograd);
     case kDepthwise: return p->groups == p->ic && p->ic == p->oc;
@@ -2834,8 +2700,11 @@ static int auto_algo(const ConvPlan* p) {
 }
 
 // Packs (once) the device weights the given algorithm reads.
-static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo) {
-  SY_CHECK(!ctx->capturing || (algo == kIgemm ? p->w_gemm != nullptr
+static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo, int tile) {
+  const bool x3 = algo == kIgemm && is_x3_tile(tile), c3 = algo == kIgemm && is_c3_tile(tile);
+  SY_CHECK(!ctx->capturing || (x3 ? p->w_x3 != nullptr
+                               : c3 ? p->w_c3 != nullptr
+                               : algo == kIgemm ? p->w_gemm != nullptr
                                : algo == kDirect ? p->w_direct != nullptr
                                : algo == kDepthwise ? p->w_dw != nullptr
                                : algo == kWinograd2 || algo == kWinograd ? p->w_wino_b != nullptr
@@ -2843,7 +2712,36 @@ static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo) {
            SY_ESTATE, "weight packing during graph capture");
   const int oc = p->oc, ic = p->ic, kh = p->kh, kw = p->kw;
   const float* W = p->host_w.data();
-  if (algo == kIgemm && !p->w_gemm) {
+  if ((x3 && !p->w_x3) || (c3 && !p->w_c3)) {
+    // Split weights in the GEMM's or the 3x3 patch kernel's operand order
+    // (igemm.h), then the channels' inverse scales.
+    const int taps = kh * kw, K = taps * ic, nkt = (K + 31) / 32, ng = (ic + 15) / 16, ocp = oc_pad(oc);
+    const size_t units = x3 ? (size_t)(ocp / 32) * nkt * kX3Units : (size_t)(ocp / 32) * ng * taps * 128;
+    std::vector<float> h(units * 4 + ocp, 0.f);
+    uint16_t* q = (uint16_t*)h.data();
+    for (int o = 0; o < oc; ++o) {
+      const float* g = W + (size_t)o * K;
+      float big = 0.f;
+      for (int i = 0; i < K; ++i)
+        if (std::isfinite(g[i])) big = std::max(big, std::fabs(g[i]));
+      const float scale = x3_weight_scale(big);
+      h[units * 4 + o] = 1.f / scale;
+      for (int c = 0; c < ic; ++c)
+        for (int t = 0; t < taps; ++t) {
+          const int k = x3 ? t * ic + c : c;
+          const size_t unit = x3 ? ((size_t)(o >> 5) * nkt + (k >> 5)) * kX3Units + ((k >> 4) & 1) * 128
+                                 : (((size_t)(o >> 5) * ng + (c >> 4)) * taps + t) * 128;
+          uint16_t part[2];
+          x3_split(g[(size_t)c * taps + t], scale, part);
+          for (int i = 0; i < 2; ++i) q[(unit + 64 * i + ((k >> 3) & 1) * 32 + (o & 31)) * 8 + (k & 7)] = part[i];
+        }
+    }
+    float* d = nullptr;
+    SY_TRY(upload(ctx, h, &d));
+    (x3 ? p->w_x3 : p->w_c3) = d;
+    (x3 ? p->w_x3s : p->w_c3s) = d + units * 4;
+  }
+  if (algo == kIgemm && !x3 && !c3 && !p->w_gemm) {
     const int K = kh * kw * ic;
     p->kp = round_up(K, 32);  // the deepest K tile
     p->ocp = oc_pad(oc);
@@ -2941,7 +2839,7 @@ int conv_prepare(sy_ctx* ctx, ConvPlan* p) {
            "convolution oc=%d ic=%d k=%dx%d groups=%d is not supported by the HIP backend", p->oc, p->ic, p->kh,
            p->kw, p->groups);
   p->algo = algo;
-  return pack_weights(ctx, p, algo);
+  return pack_weights(ctx, p, algo, -1);
 }
 
 void conv_out_size(const ConvPlan* p, int h, int w, int* oh, int* ow) {
@@ -3022,7 +2920,7 @@ static int conv_exec(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tens
              "residual shape does not match the conv output");
   const bool nchw = x->layout == SY_LAYOUT_NCHW;
   const int algo = ch.algo;
-  SY_TRY(pack_weights(ctx, p, algo));
+  SY_TRY(pack_weights(ctx, p, algo, ch.tile >= 0 ? ch.tile : env_tile()));
   ForceTile force(ctx, ch.tile, ch.split);
   ProfTag tag_scope(ctx);
   if (ctx->profile_shapes) {
@@ -3137,10 +3035,32 @@ static int conv_exec(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tens
   // float4 gathers need 16-byte aligned channel groups.
   SY_CHECK(((uintptr_t)x->data & 15) == 0 && (x->ldc & 3) == 0, SY_EINVAL,
            "conv input view must be 16-byte aligned with ldc %% 4 == 0");
+  const int et = ch.tile >= 0 ? ch.tile : env_tile();
+  if (algo == kIgemm && is_c3_tile(et)) {
+    C3Args a{};
+    a.x = x->data; a.N = x->n; a.H = x->h; a.W = x->w; a.IC = x->c; a.ldx = x->ldc;
+    a.w = p->w_c3; a.ws = p->w_c3s; a.bias = p->bias;
+    a.res = res ? res->data : nullptr; a.ldr = res ? res->ldc : 0;
+    a.y = y->data; a.ldy = y->ldc; a.OC = p->oc; a.silu = p->silu; a.ng = (p->ic + 15) / 16;
+    if (!conv3x3_s1(p) || ctx->up_src || !c3_fits(a)) {
+      // Views past the kernel's 32-bit offsets (the tuned choice is kept by
+      // shape, not by pitch) take the routing rule.
+      SY_CHECK(ch.tile >= 0, SY_EUNSUPPORTED,
+               "the 3x3 patch kernel needs a 3x3 stride-1 pad-1 convolution of 32-bit extent");
+      return conv_exec(ctx, p, x, y, res, ConvChoice{p->algo, -1});
+    }
+    const double px = (double)x->n * oh * ow;
+    const char* pn = c3_name(et - kC3Base);
+    ProfScope prof(ctx, pn, 2.0 * 9 * px * p->ic * p->oc,
+                   4.0 * (px * p->ic + px * p->oc * (res ? 2 : 1) + 9.0 * p->ic * p->oc));
+    SY_TRY(launch_c3(ctx, et - kC3Base, a));
+    return check_launch(pn);
+  }
   if (algo == kIgemm) {
     IgemmArgs a;
     a.x = x->data; a.N = x->n; a.H = x->h; a.W = x->w; a.IC = x->c; a.ldx = x->ldc;
     a.w = p->w_gemm; a.Kp = p->kp; a.bias = p->bias;
+    a.w3 = p->w_x3; a.w3s = p->w_x3s; a.nkt = (p->kh * p->kw * p->ic + 31) / 32;
     a.res = res ? res->data : nullptr; a.ldr = res ? res->ldc : 0;
     a.y = y->data; a.OH = oh; a.OW = ow; a.OC = p->oc; a.ldy = y->ldc;
     a.KH = p->kh; a.KW = p->kw; a.SH = p->sh; a.SW = p->sw; a.PH = p->pt; a.PW = p->pl; a.DH = p->dh; a.DW = p->dw;
@@ -3342,6 +3262,20 @@ static std::vector<ConvChoice> conv_candidates_all(const ConvPlan* p, const sy_t
   conv_out_size(p, x->h, x->w, &oh, &ow);
   const long long M = (long long)x->n * oh * ow;
   const int K = p->kh * p->kw * p->ic;
+  // The f16-split kernels.  Where 64 x 64 output tiles fill the CUs twice over
+  // they are the fastest of all at every layer shape of the YOLO families with
+  // at least 64 multiplied channels (1x1 384 -> 128 at 40 x 40, batch 32: 30 us
+  // against 58; 3x3 64 -> 64 at 80 x 80: 57 against 73; 3x3 stride 2 64 -> 128:
+  // 38 against 82) and no other candidate is timed; smaller grids and shallow
+  // products, where the in-workgroup split-K and row kernels can win, time all.
+  if (conv_supports(p, kIgemm) && M * p->oc < (1LL << 40)) {
+    for (int i = 0; i < x3_num_tiles(); ++i) cand.push_back(ConvChoice{kIgemm, kX3Base + i});
+    const long long wide = (M + 63) / 64 * ((p->oc + 63) / 64);
+    if (conv3x3_s1(p)) {
+      for (int i = 0; i < c3_num_forms(); ++i) cand.push_back(ConvChoice{kIgemm, kC3Base + i});
+    }
+    if (wide >= 512 && K >= 64 && p->ic >= 32) return cand;
+  }
   for (int algo : {(int)kIgemm, (int)kWinograd3}) {
     if (!conv_supports(p, algo)) continue;
     for (int t = 0; t < kNumTiles; ++t) {
@@ -3405,7 +3339,9 @@ static std::vector<ConvChoice> conv_candidates(const ConvPlan* p, const sy_tenso
   if (ku == 0) return cand;
   std::vector<ConvChoice> keep;
   for (const ConvChoice& c : cand)
-    if (c.algo == kIgemm && c.tile >= 0 && c.tile < kNumTiles && ku % kTiles[c.tile].bk == 0) keep.push_back(c);
+    if (c.algo == kIgemm && (is_x3_tile(c.tile) ? ku % 32 == 0
+                                                : c.tile >= 0 && c.tile < kNumTiles && ku % kTiles[c.tile].bk == 0))
+      keep.push_back(c);
   return keep;
 }
 

@@ -1,0 +1,386 @@
+// 3x3 stride-1 convolution on the f16 matrix cores, from an LDS patch.
+//
+// The arithmetic is split_gemm.hip's (float32 as scaled f16 pairs, three
+// products).  Its implicit GEMM stages and splits every input value once per
+// tap; here a workgroup stages the input patch of its output tile (TH x TW
+// outputs, (TH + 2) x (TW + 2) inputs) once, up to 64 channels at a time, and
+// the nine taps read it at shifted pixels.  All of a chunk's loads are issued
+// together: 16 channels at a time left too few bytes in flight, and every
+// wait for weights behind them (loads return in order) cost a memory latency.  Weights stream from L2 straight into MFMA
+// operands: their packed order makes each read of a wave 1 KiB contiguous, and
+// the workgroup's waves read the same ones.
+//
+// A wave owns TM 32-pixel blocks x TN 32-channel blocks.  Per (tap, 16
+// channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
+// MFMAs of 32 cycles.
+//
+// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 57 us,
+// against 73 us for the fastest float32 Winograd form.  The matrix cores are
+// busy for a third of it at the 1.8 GHz the GPU holds under this load; a
+// 128-pixel workgroup's 31,000 cycles are 14,000 of taps, 8,000 of patch loads
+// and 7,000 of epilogue, and 1,600 of them on 256 CUs leave a thin last round.
+// Workgroups that run through several tiles with the next patch loaded behind
+// the last taps measured the same, 16-channel double buffering 57 - 60 us.
+//
+// LDS holds the patch as planes of 8 channels, [split][8-channel block][pixel]
+// [8].  ds_read_b128 serves 16 lanes a cycle over 64 banks, lanes 0-3, 12-15,
+// 20-23, 24-27 together and the other 16 of each half wave together (measured:
+// 232 B/clk per CU without conflicts, 126 with 32 consecutive pixels on 32
+// consecutive lanes); c3_row gives the lanes of one such group 16 consecutive
+// pixels.  The planes' pitch spreads a staged pixel's 8-byte writes over the
+// banks.
+#include <cmath>
+#include <cstring>
+#include <string>
+
+#include "igemm.h"
+#include "split.h"
+
+namespace sy {
+
+constexpr int kC3Oob = 0x40000000;       // buffer offset past every record: the load returns zero
+constexpr int kC3BufWord3 = 0x00020000;  // raw buffer resource, word 3 (gfx9 family)
+
+// LDS pixels a patch may take for a tile of BM outputs.
+constexpr int c3_patch(int bm) { return bm == 64 ? 112 : 192; }
+
+// Pixel of a 32-pixel block that MFMA row r (lane r of a half wave) holds.
+__device__ __forceinline__ int c3_row(int r) { return ((0x73261540 >> (r & 28)) & 7) * 4 + (r & 3); }
+
+__device__ __forceinline__ float c3_weight(const C3Args& a, int col, int ic, int tap) {
+  const _Float16* e = (const _Float16*)a.w +
+                      ((((long long)(col >> 5) * a.ng + (ic >> 4)) * 9 + tap) * 128 + ((ic >> 3) & 1) * 32 +
+                       (col & 31)) * 8 + (ic & 7);
+  const float hi = (float)e[0], lo = (float)e[512];
+  return (lo == 0.f ? hi : __builtin_fmaf(lo, 1.f / 2048, hi)) * a.ws[col];
+}
+
+// Epilogue of a wave whose sums are not all finite: its elements again in
+// float32, from the input and the packed weights.
+__device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int pixels, int col0, int cols, int lane) {
+  for (int i = lane; i < pixels * cols; i += 64) {
+    const int pix = opix[i / cols], col = col0 + i % cols;
+    if (pix < 0 || col >= a.OC) continue;
+    const int ox = pix % a.W, t = pix / a.W, oy = t % a.H, n = t / a.H;
+    float v = 0.f;
+    for (int tap = 0; tap < 9; ++tap) {
+      const int iy = oy - 1 + tap / 3, ix = ox - 1 + tap % 3;
+      if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
+      const float* x = a.x + (((long long)n * a.H + iy) * a.W + ix) * a.ldx;
+      for (int c = 0; c < a.IC; ++c) v = __builtin_fmaf(x[c], c3_weight(a, col, c, tap), v);
+    }
+    v += a.bias[col];
+    if (a.silu) v = silu_fast(v);
+    if (a.res) v = a.res[(long long)pix * a.ldr + col] + v;
+    a.y[(long long)pix * a.ldy + col] = v;
+  }
+}
+
+// G: 16-channel groups per chunk.
+template <int G, int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G == 4 && WM * WN == 2) ? 2 : 4) void conv3_kernel(
+    const C3Args a) {
+  constexpr int NW = WM * WN, NT = NW * 64, BM = WM * TM * 32, NPX = c3_patch(BM);
+  constexpr int PL = (NPX * 8 + 127) / 128 * 128 + 64 / G;  // halves per plane
+  constexpr int L_IT = (NPX * 4 * G + NT - 1) / NT;         // float4 loads per thread and chunk
+  __shared__ __attribute__((aligned(16))) _Float16 P[G * 4 * PL];
+  __shared__ __attribute__((aligned(16))) int opix[BM];
+  __shared__ float red[NW];  // the waves' largest magnitudes
+
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wid / WN, wn = wid % WN;
+  const int half = lane >> 5, r32 = lane & 31;
+  // Each XCD (workgroups L, L + 8, ...) takes a contiguous run of tiles, a
+  // tile's channel blocks next to each other (they read the same patch) and
+  // neighbouring tiles after it.
+  const int grid = gridDim.x, L = blockIdx.x;
+  const int xcd = L & 7, q8 = grid >> 3, rem = grid & 7;
+  const int T = xcd * q8 + (xcd < rem ? xcd : rem) + (L >> 3);
+  const int tile = T / a.nblk, ob0 = (T - tile * a.nblk) * (WN * TN) + wn * TN;
+  const int trow = tile / a.ntx, ox0 = (tile - trow * a.ntx) * a.TW;
+  // Tile rows run over virtual rows, rpi per image: H + 1 with tiles that may
+  // span images (the row past H is the zero row between two images), or a
+  // multiple of TH with tiles inside one image.
+  const int v0 = trow * a.TH, nb = v0 / a.rpi, y0 = v0 - nb * a.rpi;
+  const int PW = a.TW + 2, npx = (a.TH + 2) * PW;
+
+  // Patch values this thread stages: its i-th float4 is channels 4 q4 .. + 3 of
+  // the chunk, of patch pixel px0 + i NT / 4G.  Byte offsets from the tile's
+  // first image; pixels outside their image read as zero.
+  const long long img = (long long)a.H * a.W * a.ldx;
+  const long long span = 4 * ((a.N - nb) * img - a.ldx + a.IC);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(a.x + nb * img), (short)0, (int)min(span, (long long)kC3Oob), kC3BufWord3);
+  const int q4 = tid % (4 * G), px0 = tid / (4 * G);
+  f32x4 d[L_IT];
+  auto xload = [&](int ch) {
+    const bool cok = ch * (16 * G) + 4 * q4 < a.IC;
+#pragma unroll
+    for (int i = 0; i < L_IT; ++i) {
+      const int px = px0 + i * (NT / (4 * G)), pr = (px * a.inv_pw) >> 16, ix = ox0 - 1 + px - pr * PW;
+      const bool wrap = a.rpi > a.H && y0 - 1 + pr >= a.rpi;  // into the next image
+      const int y = wrap ? y0 - 1 + pr - a.rpi : y0 - 1 + pr;
+      const bool ok =
+          cok && px < npx && nb + wrap < a.N && (unsigned)y < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+      const int off = ok ? 4 * ((wrap ? (int)img : 0) + (y * a.W + ix) * a.ldx + 4 * q4) : kC3Oob;
+      d[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, ch * (64 * G), 0));
+    }
+  };
+  auto stage = [&](float s) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < L_IT; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m = fmaxf(m, __builtin_fabsf(d[i][e]));
+      const int px = px0 + i * (NT / (4 * G));
+      u32x2 hi, lo;
+      split4(d[i], s, hi, lo);
+      if (L_IT * NT == NPX * 4 * G || px < NPX) {
+        _Float16* dst = P + (q4 >> 1) * PL + px * 8 + (q4 & 1) * 4;
+        *(u32x2*)dst = hi;
+        *(u32x2*)(dst + 2 * G * PL) = lo;
+      }
+    }
+    m = wave_max63(m);
+    if (lane == 63) red[wid] = m;
+  };
+  // Weights run kRing taps ahead of their use, across groups and chunks (the
+  // last group loads its own first taps again): uniform base of the wave's
+  // channel blocks, 32-bit lane offset.
+  constexpr int kRing = 3;
+  f16x8 bv[kRing][TN][2];
+  const int wob = a.ng * (9 * 128 * 16);  // bytes per 32-channel block
+  const char* wbase = (const char*)a.w + (long long)ob0 * wob;
+  const unsigned wlane = lane * 16;
+  auto wload = [&](int g, int tap) {
+    const char* wg = wbase + min(g, a.ng - 1) * (9 * 128 * 16);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        bv[tap % kRing][j][p] = *(const f16x8*)(wg + (j * wob + (tap * 2 + p) * 1024) + wlane);
+  };
+
+  xload(0);
+  // The epilogue's operands, loaded before they are waited for.
+  const int col0 = ob0 * 32 + r32;
+  float bias[TN], ws[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    bias[j] = col0 + j * 32 < a.OC ? a.bias[col0 + j * 32] : 0.f;
+    ws[j] = a.ws[col0 + j * 32];
+  }
+  // This tile's output pixels, by MFMA row.
+  for (int p = tid; p < BM; p += NT) {
+    const int q = (p & ~31) + c3_row(p & 31), py = (q * a.inv_tw) >> 16, ox = ox0 + q - py * a.TW;
+    const bool wrap = y0 + py >= a.rpi;
+    const int n = wrap ? nb + 1 : nb, oy = wrap ? y0 + py - a.rpi : y0 + py;
+    opix[p] = py < a.TH && n < a.N && oy < a.H && ox < a.W ? (n * a.H + oy) * a.W + ox : -1;
+  }
+  // LDS offset (halves) of this lane's operand rows at tap (0, 0).
+  int arow[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int p = (wm * TM + i) * 32 + c3_row(r32), py = (p * a.inv_tw) >> 16;
+    arow[i] = (min(py, a.TH - 1) * PW + p - py * a.TW) * 8 + half * PL;
+  }
+  f32x16 acc[TM][TN], crs[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = crs[i][j][r] = 0.f;
+  int se = kSplitExpGuess;
+  float big = 0.f;  // largest magnitude so far
+
+  for (int g = 0; g < a.ng; ++g) {
+    if (g % G == 0) {
+      if (g > 0) {
+        xload(g / G);
+        __syncthreads();  // the last chunk's operand reads are done
+      }
+      stage(exp_float(se));
+      if (g == 0) {
+#pragma unroll
+        for (int t = 0; t < kRing; ++t) wload(0, t);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < NW; ++w) big = fmaxf(big, red[w]);
+      int ne;
+      if (!scale_fits(big, se, &ne)) {  // rare: the chunk again with another scale
+        if (g > 0) rescale<TM, TN>(se, ne, acc, crs);
+        se = ne;
+        xload(g / G);
+        __syncthreads();  // every wave has read the maxima
+        stage(exp_float(se));
+        __syncthreads();
+      }
+    }
+    const _Float16* pg = P + (g % G) * (2 * PL);
+    f16x8 av[2][TM][2];
+    auto aload = [&](int tap) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          av[tap & 1][i][p] =
+              *(const f16x8*)(pg + p * (2 * G * PL) + arow[i] + (tap / 3) * PW * 8 + (tap % 3) * 8);
+    };
+    aload(0);
+    // The barriers pin the order: operands of the next tap, this tap's MFMAs,
+    // the weights three taps on.
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+      if (tap + 1 < 9) aload(tap + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const auto& w = bv[tap % kRing];
+      const auto& x = av[tap & 1];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          crs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i][1], w[j][0], crs[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i][0], w[j][0], acc[i][j], 0, 0, 0);
+        }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          crs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i][0], w[j][1], crs[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      wload(tap + kRing < 9 ? g : g + 1, (tap + kRing) % 9);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  const bool bad = unscale<TM, TN>(ws, se, acc, crs);
+  const int* po = opix + wm * TM * 32;
+  if (__any(bad) || big >= kSplitHuge) {
+    c3_exact(a, po, TM * 32, col0 - r32, TN * 32, lane);
+    return;
+  }
+  // D layout: lane holds column r32 of rows 8 (r / 4) + 4 half + r % 4.
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    int px[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) px[r] = po[i * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = col0 + j * 32;
+      if (col >= a.OC) continue;
+      float v[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        v[r] = acc[i][j][r] + bias[j];
+        if (a.silu) v[r] = silu_fast(v[r]);
+      }
+      if (a.res) {
+        float rv[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) rv[r] = a.res[(unsigned)(max(px[r], 0) * a.ldr + col)];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = rv[r] + v[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (px[r] >= 0) a.y[(unsigned)(px[r] * a.ldy + col)] = v[r];
+    }
+  }
+}
+
+// Wave grid (pixels x channels) and 32 x 32 blocks per wave.
+#define SY_C3_LIST(X) \
+  X(0, 2, 2, 2, 1) X(1, 4, 1, 1, 1) X(2, 2, 1, 1, 1) X(3, 2, 2, 1, 1) X(4, 2, 3, 1, 1)
+
+struct C3Form {
+  int wm, wn, tm, tn;
+};
+#define SY_C3_CFG(i, wm, wn, tm, tn) {wm, wn, tm, tn},
+static const C3Form kC3Forms[] = {SY_C3_LIST(SY_C3_CFG)};
+#undef SY_C3_CFG
+static constexpr int kNumC3 = sizeof(kC3Forms) / sizeof(kC3Forms[0]);
+int c3_num_forms() { return kNumC3; }
+
+const char* c3_name(int f) {
+  struct Names {
+    std::string n[kNumC3];
+    Names() {
+      for (int i = 0; i < kNumC3; ++i) {
+        char buf[48];
+        snprintf(buf, sizeof buf, "conv3_x3_%dx%d_%d%d", kC3Forms[i].wm * kC3Forms[i].tm * 32,
+                 kC3Forms[i].wn * kC3Forms[i].tn * 32, kC3Forms[i].wm, kC3Forms[i].wn);
+        n[i] = buf;
+      }
+    }
+  };
+  static const Names names;
+  return names.n[f].c_str();
+}
+
+// Output tile of at most bm pixels whose patch fits, with the fewest tiles:
+// TW from 4 to bm columns (a multiple of 16 among equals: its operand reads are
+// free of bank conflicts), tiles inside one image or over virtual rows.
+static bool pick_tile_shape(int bm, int N, int H, int W, int* th, int* tw, int* rpi, long long* tiles, int* ntx) {
+  long long best = -1;
+  int best_px = 0;
+  for (int w = 4; w <= bm && w <= ((W + 3) & ~3); ++w) {
+    int h = std::min(bm / w, c3_patch(bm) / (w + 2) - 2);
+    if (h < 1) continue;
+    const int tx = (W + w - 1) / w;
+    for (int span = 0; span < 2; ++span) {
+      // A tile spans at most two images.
+      const int hh = span ? std::min(h, H - 1) : std::min(h, H);
+      if (hh < 1) continue;
+      const int r = span ? H + 1 : (H + hh - 1) / hh * hh;
+      const long long t = ((long long)N * r + hh - 1) / hh * tx;
+      const int px = (hh + 2) * (w + 2);
+      if (best < 0 || t < best || (t == best && (w % 16 == 0 || (*tw % 16 && px <= best_px)))) {
+        best = t;
+        best_px = px;
+        *th = hh;
+        *tw = w;
+        *rpi = r;
+        *ntx = tx;
+      }
+    }
+  }
+  *tiles = best;
+  return best > 0;
+}
+
+bool c3_fits(const C3Args& a) {
+  // 32-bit offsets: the two images a tile may span below the zero-read
+  // offset, every output and residual element below 2^31.
+  const long long img = 4LL * a.H * a.W * a.ldx, M = (long long)a.N * a.H * a.W;
+  return 2 * img < kC3Oob && M * a.ldy < (1LL << 31) && M * a.ldr < (1LL << 31) &&
+         (long long)a.N * (a.H + 64) < (1LL << 31) && (long long)a.ng * (9 * 128 * 16 * 4) < (1LL << 31);
+}
+
+int launch_c3(sy_ctx* ctx, int f, C3Args a) {
+  const C3Form& c = kC3Forms[f];
+  const int bm = c.wm * c.tm * 32;
+  long long tiles = 0;
+  SY_CHECK(pick_tile_shape(bm, a.N, a.H, a.W, &a.TH, &a.TW, &a.rpi, &tiles, &a.ntx), SY_EUNSUPPORTED,
+           "no tile for a %dx%d image", a.H, a.W);
+  a.nblk = ((a.OC + 31) / 32 + c.wn * c.tn - 1) / (c.wn * c.tn);
+  a.inv_tw = 65536 / a.TW + 1;
+  a.inv_pw = 65536 / (a.TW + 2) + 1;
+  SY_CHECK(tiles * a.nblk < (1LL << 31), SY_EUNSUPPORTED, "convolution grid too large");
+  void (*k)(const C3Args) = nullptr;
+#define SY_C3_CASE(i, wm, wn, tm, tn)                 \
+  if (f == i)                                         \
+    k = a.ng == 1   ? conv3_kernel<1, wm, wn, tm, tn> \
+        : a.ng == 2 ? conv3_kernel<2, wm, wn, tm, tn> \
+                    : conv3_kernel<4, wm, wn, tm, tn>;
+  SY_C3_LIST(SY_C3_CASE)
+#undef SY_C3_CASE
+  SY_CHECK(k != nullptr, SY_EINVAL, "no split 3x3 form %d", f);
+  hipLaunchKernelGGL(k, dim3((unsigned)(tiles * a.nblk)), dim3(c.wm * c.wn * 64), 0, ctx->stream, a);
+  return SY_OK;
+}
+
+}  // namespace sy

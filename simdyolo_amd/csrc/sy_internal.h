@@ -217,6 +217,11 @@ struct ConvPlan {
   // implicit GEMM: weights [ocp][kp], K ordered (ky, kx, ic)
   float* w_gemm = nullptr;
   int kp = 0, ocp = 0;
+  // implicit GEMM on f16 splits: packed as igemm.h describes, then per output
+  // channel the inverse of its scale
+  float *w_x3 = nullptr, *w_x3s = nullptr;
+  // the same for the 3x3 patch kernel
+  float *w_c3 = nullptr, *w_c3s = nullptr;
   // Winograd: U [36][ocw][kpw] (ocw = oc rounded to the GEMM tile, kpw = ic
   // rounded to the deepest K tile)
   float* w_wino = nullptr;

@@ -1,0 +1,211 @@
+"""The f16-split matrix kernels (float32 values as scaled f16 pairs): every
+tile of the implicit GEMM and every form of the 3x3 patch kernel, pinned
+through SIMDYOLO_HIP_TILE, against float64.
+
+Bound: a value's pair is within 2^-23 of it, the product left out below 2^-22
+of the product, so a sum of products is within 2^-20.5 of the sum of their
+magnitudes before the accumulators round; these add at most 2^-24 of the
+running sum per 16 terms and product.  2^-19 covers both up to K = 1152.  A
+value below 2^-15 of the workgroup's largest has an absolute error of 2^-38 of
+that largest instead.
+"""
+import numpy as np
+import pytest
+
+from simdyolo_amd import CONV_IGEMM, synth
+
+pytestmark = pytest.mark.gpu
+
+X3_BASE, C3_BASE = 64, 96
+X3_TILES = [(128, 128, 2, 2), (64, 64, 2, 2), (64, 128, 2, 2), (128, 32, 4, 1), (64, 32, 2, 1)]
+C3_FORMS = [(128, 64, 2, 2), (128, 32, 4, 1), (64, 32, 2, 1), (64, 64, 2, 2), (64, 96, 2, 3)]
+
+
+def conv64(x, w, b, stride, silu, res):
+    """(result, sum of the products' magnitudes) in float64, NCHW."""
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    n, ic, h, wd = x.shape
+    oc, _, k, _ = w.shape
+    p = k // 2
+    oh, ow = (h + 2 * p - k) // stride + 1, (wd + 2 * p - k) // stride + 1
+    y = np.zeros((n, oc, oh, ow)) + b.astype(np.float64)[None, :, None, None]
+    mag = np.abs(y)
+    xp = np.pad(x, ((0, 0), (0, 0), (p, p), (p, p)))
+    with np.errstate(invalid="ignore", over="ignore"):
+        for i in range(k):
+            for j in range(k):
+                t = xp[:, :, i:i + stride * (oh - 1) + 1:stride, j:j + stride * (ow - 1) + 1:stride]
+                y += np.einsum("nchw,oc->nohw", t, w[:, :, i, j])
+                mag += np.einsum("nchw,oc->nohw", np.abs(t), np.abs(w[:, :, i, j]))
+        if silu:
+            y = y / (1.0 + np.exp(-y))
+    if res is not None:
+        y = y + res
+        mag = mag + np.abs(res)
+    return y, mag
+
+
+def run(hip, monkeypatch, tile, x, w, b, stride=1, silu=True, res=None):
+    """The conv on channel slices of wider buffers; (result, kernel names)."""
+    monkeypatch.setenv("SIMDYOLO_HIP_TILE", str(tile))
+    n, ic, h, wd = x.shape
+    oc, _, k, _ = w.shape
+    hip.begin_frame()
+    try:
+        conv = hip.conv_create(w, b, (stride, stride), (k // 2,) * 4, silu=silu)
+        hip.conv_set_algo(conv, CONV_IGEMM)
+        oh, ow = hip.conv_out_size(conv, h, wd)
+        xv = hip.alloc(n, ic + 4, h, wd).slice(4, ic)
+        hip.upload(x, xv)
+        yv = hip.alloc(n, oc + 13, oh, ow).slice(9, oc)
+        rv = None
+        if res is not None:
+            rv = hip.alloc(n, oc + 7, oh, ow).slice(3, oc)
+            hip.upload(res, rv)
+        hip.profile_enable(True)
+        hip.profile_read()
+        try:
+            hip.conv(conv, xv, yv, rv)
+            hip.flush()
+            names = set(hip.profile_read())
+        finally:
+            hip.profile_enable(False)
+        return hip.download(yv), names
+    finally:
+        hip.end_frame()
+
+
+def data(n, ic, h, w, oc, k, seed):
+    return (synth.activations((n, ic, h, w), seed), synth.kaiming((oc, ic, k, k), seed + 1),
+            synth.activations((oc,), seed + 2) * np.float32(0.1))
+
+
+def near(got, exp, mag, floor=0.0):
+    off = np.abs(got.astype(np.float64) - exp)
+    allowed = 2.0 ** -19 * mag + floor
+    assert np.isfinite(got).all() and (off <= allowed).all(), (off / allowed).max()
+
+
+# (n, ic, h, w, oc, k, stride), mode: ragged pixels, channels and depth.
+GEMM = [((2, 40, 13, 11, 72, 1, 1), 2), ((1, 4, 1, 1, 1, 1, 1), 2), ((1, 512, 9, 7, 132, 1, 1), 2),
+        ((1, 64, 19, 21, 40, 3, 2), 1), ((2, 20, 11, 9, 24, 3, 1), 0), ((1, 16, 33, 18, 32, 3, 2), 0)]
+
+
+@pytest.mark.parametrize("res", [False, True], ids=["plain", "res"])
+@pytest.mark.parametrize("form,mode", GEMM, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+@pytest.mark.parametrize("tile", range(len(X3_TILES)))
+def test_gemm_tiles(hip, monkeypatch, tile, form, mode, res):
+    n, ic, h, w, oc, k, s = form
+    x, wt, b = data(n, ic, h, w, oc, k, 100 + tile)
+    r = synth.activations((n, oc, (h - 1) // s + 1, (w - 1) // s + 1), 7) if res else None
+    exp, mag = conv64(x, wt, b, s, True, r)
+    got, names = run(hip, monkeypatch, X3_BASE + tile, x, wt, b, s, True, r)
+    assert names == {"igemm_m%d_x3_%dx%d_%d%d" % ((mode,) + X3_TILES[tile])}
+    near(got, exp, mag)
+
+
+# (n, ic, h, w, oc): one pixel, images smaller than a tile, tiles across images, ragged edges; input channels of one
+# partial group to three chunks.
+PATCH = [(1, 4, 1, 1, 1), (3, 16, 2, 5, 33), (5, 20, 20, 20, 24), (2, 32, 17, 33, 64), (1, 64, 45, 75, 80),
+         (2, 80, 9, 16, 96), (1, 144, 8, 8, 128)]
+
+
+@pytest.mark.parametrize("res", [False, True], ids=["plain", "res"])
+@pytest.mark.parametrize("shape", PATCH, ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("form", range(len(C3_FORMS)))
+def test_patch_forms(hip, monkeypatch, form, shape, res):
+    n, ic, h, w, oc = shape
+    x, wt, b = data(n, ic, h, w, oc, 3, 200 + form)
+    r = synth.activations((n, oc, h, w), 8) if res else None
+    exp, mag = conv64(x, wt, b, 1, True, r)
+    got, names = run(hip, monkeypatch, C3_BASE + form, x, wt, b, 1, True, r)
+    assert names == {"conv3_x3_%dx%d_%d%d" % C3_FORMS[form]}
+    near(got, exp, mag)
+
+
+@pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3], ids=["gemm", "patch"])
+@pytest.mark.parametrize("scale", [0.0, 1e-30, 1e-6, 3e4, 1e30], ids=str)
+def test_scales(hip, monkeypatch, tile, scale):
+    """Magnitudes outside the first guess of the scale, the second half of the
+    channels 2^12 times larger (the sums so far change scale), and one value
+    10^6 times the others."""
+    x, wt, b = data(1, 128, 12, 20, 40, 3, 300)
+    x = (x * np.float32(scale)).astype(np.float32)
+    x[:, 64:] *= np.float32(4096)
+    x[0, 5, 3, 4] *= np.float32(1e6)
+    b = b * np.float32(0)
+    exp, mag = conv64(x, wt, b, 1, False, None)
+    got, _ = run(hip, monkeypatch, tile, x, wt, b, 1, False)
+    near(got, exp, mag, 2.0 ** -38 * float(np.abs(x).max()) * np.abs(wt).sum(axis=(1, 2, 3)).max() + 1e-45)
+
+
+@pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3], ids=["gemm", "patch"])
+@pytest.mark.parametrize("where", ["input", "weight"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38], ids=str)
+def test_non_finite(hip, monkeypatch, tile, where, value):
+    """Infinities, NaN and the top of the float32 range give what float32
+    arithmetic gives, at the outputs that they reach and no others."""
+    x, wt, b = data(1, 32, 10, 19, 24, 3, 400)
+    (x if where == "input" else wt)[0, 3, 1, 1] = value
+    exp, mag = conv64(x, wt, b, 1, False, None)
+    exp = np.where(np.abs(exp) > np.finfo(np.float32).max, np.sign(exp) * np.inf, exp)
+    got, _ = run(hip, monkeypatch, tile, x, wt, b, 1, False)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(exp))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(exp))
+    fine = np.isfinite(exp)
+    # Elements of a tile that holds a non-finite sum are computed in float32.
+    assert (np.abs(got[fine] - exp[fine]) <= 2.0 ** -17 * mag[fine]).all()
+
+
+def test_transposed_conv(hip, monkeypatch):
+    """The 2x2 transposed conv's sub-pixel scatter behind a split GEMM tile."""
+    monkeypatch.setenv("SIMDYOLO_HIP_TILE", str(X3_BASE + 1))
+    ic, oc, h, w = 36, 20, 7, 9
+    x = synth.activations((2, ic, h, w), 500)
+    wt = synth.activations((ic, oc, 2, 2), 501)
+    b = synth.activations((oc,), 502)
+    exp = np.einsum("nchw,coij->nohiwj", x.astype(np.float64), wt).reshape(2, oc, 2 * h, 2 * w)
+    mag = np.einsum("nchw,coij->nohiwj", np.abs(x).astype(np.float64), np.abs(wt)).reshape(2, oc, 2 * h, 2 * w)
+    hip.begin_frame()
+    try:
+        conv = hip.conv_transpose2x2_create(wt, b)
+        hip.conv_set_algo(conv, CONV_IGEMM)
+        y = hip.alloc(2, oc, 2 * h, 2 * w)
+        hip.conv(conv, hip.upload(x), y)
+        got = hip.download(y)
+    finally:
+        hip.end_frame()
+    near(got, exp + b[None, :, None, None], mag + np.abs(b)[None, :, None, None])
+
+
+@pytest.mark.parametrize("tile", range(len(X3_TILES)))
+def test_upsampled_part(hip, monkeypatch, tile):
+    """A 1x1 conv whose first 64 channels come from a half-resolution view."""
+    monkeypatch.setenv("SIMDYOLO_HIP_AUTOTUNE", "0")
+    monkeypatch.setenv("SIMDYOLO_HIP_TILE", str(X3_BASE + tile))
+    n, cu, c, h, w, oc = 2, 64, 20, 14, 18, 40
+    xu, x = synth.activations((n, cu, h // 2, w // 2), 600), synth.activations((n, c, h, w), 601)
+    _, wt, b = data(n, cu + c, h, w, oc, 1, 602)
+    full = np.concatenate([xu.repeat(2, 2).repeat(2, 3), x], 1)
+    exp, mag = conv64(full, wt, b, 1, True, None)
+    hip.begin_frame()
+    try:
+        conv = hip.conv_create(wt, b, silu=True)
+        xv = hip.alloc(n, cu + c, h, w)
+        hip.upload(x, xv.slice(cu, c))
+        xuv = hip.upload(xu)
+        yv = hip.alloc(n, oc, h, w)
+        hip.profile_enable(True)
+        hip.profile_read()
+        try:
+            hip.conv_upsampled(conv, xuv, xv, yv)
+            hip.flush()
+            names = set(hip.profile_read())
+        finally:
+            hip.profile_enable(False)
+        got = hip.download(yv)
+    finally:
+        hip.end_frame()
+    assert names == {"igemm_m3_x3_%dx%d_%d%d" % X3_TILES[tile]}
+    near(got, exp, mag)
