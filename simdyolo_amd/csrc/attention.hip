@@ -6,13 +6,310 @@
 // this as DeviceMatMul + Scale (op 4) + Softmax (op 25) + DeviceMatMul
 // (VulkanExecution.cs:499-541, tensor.comp:62-68).
 //
-// Both products run on the FP32-MFMA GEMM (gemm_nt); S rows and V^T rows are
+// Key dims up to 32 and head dims up to 64 (every YOLO11 / YOLO26 block: 32 and
+// 64) run in one kernel that keeps the scores in registers.  Other geometries
+// run both products on the FP32-MFMA GEMM (gemm_nt); S rows and V^T rows are
 // padded to N4 = round_up(N, 4) with zeros so K stays a multiple of 4.
 #include <cmath>
 
+#include "split.h"
 #include "sy_internal.h"
 
 namespace sy {
+
+struct AttnArgs {
+  const float* qkv;
+  int ldq, N, heads, kd, hd, qtiles;
+  float scale;
+  float* o;
+  int ldo;
+  float* v;
+  int ldv;
+};
+
+// Rows of the workgroup's queries in plain float32, one wave per query: what a
+// workgroup does that met a non-finite or huge operand (kSplitHuge).
+__device__ __forceinline__ void attn_exact(const AttnArgs& a, const float* base, float* ob, int q0, int queries,
+                                           int wave, int lane) {
+  for (int q = wave; q < queries; q += 4) {
+    if (q0 + q >= a.N) continue;
+    const float* qr = base + (long long)(q0 + q) * a.ldq;
+    auto score = [&](int j) {
+      if (j >= a.N) return -INFINITY;
+      const float* kr = base + (long long)j * a.ldq + a.kd;
+      float s = 0.f;
+      for (int c = 0; c < a.kd; ++c) s = __builtin_fmaf(qr[c], kr[c], s);
+      return s * a.scale;
+    };
+    float mx = -INFINITY;
+    for (int j = lane; j < a.N; j += 64) mx = fmaxf(mx, score(j));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    float sum = 0.f, acc = 0.f;
+    for (int j0 = 0; j0 < a.N; j0 += 64) {
+      const float e = j0 + lane < a.N ? expf(score(j0 + lane) - mx) : 0.f;
+      sum += e;
+      for (int t = 0; t < min(64, a.N - j0); ++t) {
+        const float et = __shfl(e, t);
+        if (lane < a.hd) acc = __builtin_fmaf(et, base[(long long)(j0 + t) * a.ldq + 2 * a.kd + lane], acc);
+      }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    if (lane < a.hd) ob[(long long)(q0 + q) * a.ldo + lane] = acc / sum;
+  }
+}
+
+// 32 queries of one head and image per workgroup.  Wave w takes the 32-key
+// tiles w, w + 4, ... with a running maximum, sum and output of its own; the
+// four are joined through LDS at the end.  Nothing else is shared: operands go
+// from L2 straight into MFMA registers.
+//
+// Scores are computed as S^T = K Q^T, so that a lane holds one query's scores
+// (keys 8 (r / 4) + 4 half + r % 4): the maximum and sum over keys are in-lane
+// but for one exchange between the wave's halves, and the probabilities are
+// already the B operand of O^T = V^T P^T under the key order
+// 8 (e / 4) + 4 half + e % 4 of a 16-key step, in which V is loaded.
+//
+// Both products are f16 splits (split_gemm.hip): queries, each key tile and the
+// values under scales from their largest magnitudes, probabilities under 2^11.
+//
+// Bound by VALU work (splitting K, V and P, the exponentials: about 750
+// operations beside 18 MFMAs per tile) and, at 400 tokens, by the latency of its
+// few tiles.  Measured against two GEMMs, a softmax and a copy with the scores
+// in memory, us: 2 heads, 400 tokens, batch 16 74 -> 24, batch 1 25 -> 16;
+// 4 heads, 1,600 tokens, batch 8 858 -> 184.  64 queries per workgroup, which
+// would split each key tile for twice the work, spill registers: 214.
+__global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
+  constexpr int TQ = 1, NQ = 32 * TQ;  // 32-query blocks, queries
+  __shared__ float O[4][NQ][65];
+  __shared__ float M[4][NQ], Lsum[4][NQ];
+  __shared__ int wild[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, r32 = lane & 31;
+  const int qt = blockIdx.x % a.qtiles, bh = blockIdx.x / a.qtiles, head = bh % a.heads, b = bh / a.heads;
+  const int per = 2 * a.kd + a.hd, q0 = qt * NQ;
+  const float* base = a.qkv + (long long)b * a.N * a.ldq + head * per;
+  float* ob = a.o + (long long)b * a.N * a.ldo + head * a.hd;
+  float* vb = a.v + (long long)b * a.N * a.ldv + head * a.hd;
+
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // Row `row`'s channels 16 ks + 8 half + 4 i .. + 3 from `at`.
+  auto row4 = [&](int row, int at, int ks, int i) {
+    const int c = 16 * ks + 8 * half + 4 * i;
+    return c < a.kd ? *(const f32x4*)(base + min(row, a.N - 1) * a.ldq + at + c) : zero;
+  };
+  auto max4 = [](float m, const f32x4& v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = fmaxf(m, __builtin_fabsf(v[e]));
+    return m;
+  };
+  // Eight floats times s as operand halves.
+  auto split8 = [](const f32x4& x, const f32x4& y, float s, f16x8& hi, f16x8& lo) {
+    u32x2 h0, h1, l0, l1;
+    split4(x, s, h0, l0);
+    split4(y, s, h1, l1);
+    hi = __builtin_bit_cast(f16x8, u32x4{h0[0], h0[1], h1[0], h1[1]});
+    lo = __builtin_bit_cast(f16x8, u32x4{l0[0], l0[1], l1[0], l1[1]});
+  };
+
+  f16x8 qh[TQ][2], ql[TQ][2];
+  float huge = 0.f;
+  int sq;
+  {
+    f32x4 q[TQ][2][2];
+    float m = 0.f;
+#pragma unroll
+    for (int t = 0; t < TQ; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          q[t][ks][i] = row4(q0 + 32 * t + r32, 0, ks, i);
+          m = max4(m, q[t][ks][i]);
+        }
+    m = readlane63(wave_max63(m));
+    huge = m;
+    sq = scale_exp(m);
+#pragma unroll
+    for (int t = 0; t < TQ; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) split8(q[t][ks][0], q[t][ks][1], exp_float(sq), qh[t][ks], ql[t][ks]);
+  }
+
+  f32x16 acc[2][TQ], crs[2][TQ];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int t = 0; t < TQ; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][t][r] = crs[j][t][r] = 0.f;
+  float mrun[TQ], lrun[TQ];
+#pragma unroll
+  for (int t = 0; t < TQ; ++t) {
+    mrun[t] = -INFINITY;
+    lrun[t] = 0.f;
+  }
+  int sv = kSplitExpGuess;
+  float vbig = 0.f;
+
+  // A tile's keys and values; past the last key both read the last key's row.
+  f32x4 k[2][2];
+  float v[2][16];
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) k[ks][i] = row4(j0 + r32, a.kd, ks, i);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int j = min(j0 + 16 * (e >> 3) + 8 * ((e >> 2) & 1) + 4 * half + (e & 3), a.N - 1);
+      const float* vr = base + j * a.ldq + 2 * a.kd;
+#pragma unroll
+      for (int d = 0; d < 2; ++d) v[d][e] = vr[min(32 * d + r32, a.hd - 1)];
+    }
+  };
+  const int tiles = (a.N + 31) / 32;
+  load(min(wave, tiles - 1) * 32);
+  for (int kt = wave; kt < tiles; kt += 4) {
+    const int j0 = kt * 32;
+    float km = 0.f, vm = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) km = max4(km, k[ks][i]);
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) vm = fmaxf(vm, __builtin_fabsf(v[d][e]));
+    km = readlane63(wave_max63(km));
+    vbig = fmaxf(vbig, readlane63(wave_max63(vm)));
+    huge = fmaxf(huge, fmaxf(km, vbig));
+    const int sk = scale_exp(km);
+    f16x8 kh[2], kl[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) split8(k[ks][0], k[ks][1], exp_float(sk), kh[ks], kl[ks]);
+    int ne;
+    if (!scale_fits(vbig, sv, &ne)) {
+      rescale<2, TQ>(sv, ne, acc, crs);
+      sv = ne;
+    }
+    f16x8 vh[2][2], vl[2][2];  // [block of 32 dims][16-key step]
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+        split8(f32x4{v[d][8 * st], v[d][8 * st + 1], v[d][8 * st + 2], v[d][8 * st + 3]},
+               f32x4{v[d][8 * st + 4], v[d][8 * st + 5], v[d][8 * st + 6], v[d][8 * st + 7]}, exp_float(sv), vh[d][st],
+               vl[d][st]);
+    load(min(kt + 4, tiles - 1) * 32);  // the next tile (the last loads its own again)
+
+    // 2^-(sq + sk) in two factors: their sum may pass the exponent range.
+    const float us = exp_float(254 - sq), uk = exp_float(254 - sk);
+#pragma unroll
+    for (int t = 0; t < TQ; ++t) {
+      f32x16 s, c;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = c[r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[ks], qh[t][ks], c, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks], qh[t][ks], s, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks], ql[t][ks], c, 0, 0, 0);
+      }
+      float mx = mrun[t];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = j0 + 8 * (r >> 2) + 4 * half + (r & 3);
+        s[r] = key < a.N ? __builtin_fmaf(c[r], 1.f / 2048, s[r]) * us * uk * a.scale : -INFINITY;
+        mx = fmaxf(mx, s[r]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      // A maximum of -infinity: no weight yet, nothing to rescale.
+      const float alpha = mrun[t] == -INFINITY ? 0.f : expf(mrun[t] - mx);
+      mrun[t] = mx;
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[r] = s[r] == -INFINITY ? 0.f : expf(s[r] - mx);
+        sum += s[r];
+      }
+      lrun[t] = __builtin_fmaf(lrun[t], alpha, sum);
+      f16x8 ph[2], pl[2];
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+        split8(f32x4{s[8 * st], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3]},
+               f32x4{s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]}, 2048.f, ph[st], pl[st]);
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[d][t][r] *= alpha;
+          crs[d][t][r] *= alpha;
+        }
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          crs[d][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[d][st], ph[st], crs[d][t], 0, 0, 0);
+          acc[d][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[d][st], ph[st], acc[d][t], 0, 0, 0);
+          crs[d][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[d][st], pl[st], crs[d][t], 0, 0, 0);
+        }
+    }
+  }
+
+  const float uv = exp_float(254 - sv) * (1.f / 2048);
+#pragma unroll
+  for (int t = 0; t < TQ; ++t) {
+    const float l = lrun[t] + __shfl_xor(lrun[t], 32);
+    if (half == 0) {
+      M[wave][32 * t + r32] = mrun[t];
+      Lsum[wave][32 * t + r32] = l;
+    }
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        O[wave][32 * t + r32][32 * d + 8 * (r >> 2) + 4 * half + (r & 3)] =
+            __builtin_fmaf(crs[d][t][r], 1.f / 2048, acc[d][t][r]) * uv;
+  }
+  if (lane == 0) wild[wave] = huge >= kSplitHuge;
+  // v of these rows, dense, for the positional conv: thread (row q, dim lane).
+  float vd[NQ / 4];
+#pragma unroll
+  for (int i = 0; i < NQ / 4; ++i)
+    vd[i] = base[min(q0 + wave + 4 * i, a.N - 1) * a.ldq + 2 * a.kd + min(lane, a.hd - 1)];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NQ / 4; ++i)
+    if (q0 + wave + 4 * i < a.N && lane < a.hd) vb[(long long)(q0 + wave + 4 * i) * a.ldv + lane] = vd[i];
+  if (wild[0] | wild[1] | wild[2] | wild[3]) {
+    attn_exact(a, base, ob, q0, NQ, wave, lane);
+    return;
+  }
+  // Joins the waves' partial outputs; a wave without keys weighs nothing.
+#pragma unroll
+  for (int i = 0; i < NQ / 4; ++i) {
+    const int q = wave + 4 * i;
+    float mx = M[0][q];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) mx = fmaxf(mx, M[w][q]);
+    float l = 0.f, s = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float f = M[w][q] == -INFINITY ? 0.f : expf(M[w][q] - mx);
+      l = __builtin_fmaf(Lsum[w][q], f, l);
+      s = __builtin_fmaf(O[w][q][lane], f, s);
+    }
+    if (q0 + q < a.N && lane < a.hd) ob[(long long)(q0 + q) * a.ldo + lane] = s / l;
+  }
+}
+
+// The fused kernel's geometries: operands in its 32-channel steps, row offsets
+// within an image in 32 bits.
+static bool attention_fused(const sy_tensor* qkv, int kd, int hd) {
+  return kd <= 32 && hd <= 64 && (long long)qkv->h * qkv->w * qkv->ldc < (1LL << 31);
+}
 
 // One wavefront per row: y = softmax(x * scale) over n entries (max-subtracted),
 // zeroing the padding columns [n, ld).
@@ -76,6 +373,17 @@ int op_attention(sy_ctx* ctx, const sy_tensor* qkv, int heads, int kd, int hd, f
   SY_CHECK(qkv->ldc == qkv->c || qkv->ldc % 4 == 0, SY_EINVAL, "qkv view stride");
   SY_CHECK(kd % 4 == 0 && per % 4 == 0 && hd % 4 == 0, SY_EUNSUPPORTED,
            "attention needs key/head dims that are multiples of 4");
+  SY_CHECK(((uintptr_t)qkv->data & 15) == 0 && qkv->ldc % 4 == 0, SY_EINVAL,
+           "attention qkv view must be 16-byte aligned with ldc %% 4 == 0");
+  if (attention_fused(qkv, kd, hd)) {
+    AttnArgs a{qkv->data, qkv->ldc, N, heads, kd, hd, (N + 31) / 32, scale, o->data, o->ldc, v->data, v->ldc};
+    const long long grid = (long long)B * heads * a.qtiles;
+    SY_CHECK(grid < (1LL << 31), SY_EUNSUPPORTED, "attention grid too large");
+    ProfScope prof(ctx, "attention", 2.0 * B * heads * N * (double)N * (kd + hd),
+                   4.0 * (double)B * N * (heads * per + 2.0 * C));
+    hipLaunchKernelGGL(attention_kernel, dim3((unsigned)grid), dim3(256), 0, ctx->stream, a);
+    return check_launch("attention");
+  }
   const int N4 = (N + 3) / 4 * 4;
   const size_t s_floats = (size_t)B * heads * N * N4, vt_floats = (size_t)B * heads * hd * N4;
   SY_TRY(ensure_scratch(ctx, (s_floats + vt_floats) * sizeof(float) + 512));
@@ -107,7 +415,8 @@ int op_attention(sy_ctx* ctx, const sy_tensor* qkv, int heads, int kd, int hd, f
   return SY_OK;
 }
 
-size_t attention_scratch_bytes(int B, int H, int W, int heads, int hd) {
+size_t attention_scratch_bytes(int B, int H, int W, int heads, int kd, int hd) {
+  if (kd <= 32 && hd <= 64) return 0;  // the fused kernel
   const size_t N = (size_t)H * W, N4 = (N + 3) / 4 * 4;
   return ((size_t)B * heads * N * N4 + 64 + (size_t)B * heads * hd * N4) * sizeof(float) + 512;
 }

@@ -898,7 +898,7 @@ struct Planner {
     const float scale = blk.scale;
     op([ctx, qkv, heads, kd, hd, scale, o, v]() { return sy_attention(ctx, qkv, heads, kd, hd, scale, o, v); },
        {qkv, o, v});
-    reserve(attention_scratch_bytes(x->n, x->h, x->w, heads, hd));
+    reserve(attention_scratch_bytes(x->n, x->h, x->w, heads, kd, hd));
     sy_tensor* s = alloc(x->n, c, x->h, x->w);
     conv(blk.pe, v, s, o);  // attended + pe(v)
     sy_tensor* b1 = alloc(x->n, c, x->h, x->w);

@@ -54,12 +54,18 @@ __device__ __forceinline__ float readlane63(float m) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 63));
 }
 
+// Exponent field of the scale that takes a largest magnitude m into
+// [2^11, 2^12).
+__device__ __forceinline__ int scale_exp(float m) {
+  return min(265 - (int)(__builtin_bit_cast(unsigned, m) >> 23), kSplitExpMax);
+}
+
 // Whether the scale 2^(se - 127) suits operands whose largest magnitude so far
 // is m: the scaled maximum lies in [2^2, 2^15) (a zero maximum suits any).
 // Otherwise *ne is the one that takes m into [2^11, 2^12).
 __device__ __forceinline__ bool scale_fits(float m, int se, int* ne) {
   const int me = __builtin_amdgcn_readfirstlane((int)(__builtin_bit_cast(unsigned, m) >> 23));
-  *ne = min(265 - me, kSplitExpMax);
+  *ne = __builtin_amdgcn_readfirstlane(scale_exp(m));
   const int top = me + se - 127;
   return top < 127 + 15 && (top >= 127 + 2 || *ne == se || __builtin_amdgcn_readfirstlane(m == 0.f ? 1 : 0));
 }

@@ -283,7 +283,7 @@ int op_matmul(sy_ctx* ctx, const float* a, const float* b, float* c, int m, int 
               size_t b_len, size_t c_len);
 int op_attention(sy_ctx* ctx, const sy_tensor* qkv, int heads, int kd, int hd, float scale, const sy_tensor* o,
                  const sy_tensor* v);
-size_t attention_scratch_bytes(int B, int H, int W, int heads, int hd);
+size_t attention_scratch_bytes(int B, int H, int W, int heads, int kd, int hd);
 
 int64_t pool_out_size(int len, int k, int s, int before, int after, int ceil_mode);
 

@@ -1,0 +1,107 @@
+"""The fused attention kernel at the edges of its tiles (32 queries, 32-key
+tiles over four waves, key and head dims below its 32 and 64), with non-finite
+and far-scaled operands, and the geometry past it that keeps the GEMMs.
+
+Bound: scores carry at most 2^-19 of sum |q||k| scale (f16-split products, as
+in the convolutions), a probability e^(s - m) that error twice, and the output
+2^-19 of the weighted sum of |v| more.
+"""
+import numpy as np
+import pytest
+
+from simdyolo_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(qkv, heads, kd, hd, scale):
+    """(output, bound) in float64, [B, heads * hd, N]."""
+    b, _, h, w = qkv.shape
+    t = qkv.astype(np.float64).reshape(b, heads, 2 * kd + hd, h * w)
+    q, k, v = t[:, :, :kd], t[:, :, kd:2 * kd], t[:, :, 2 * kd:]
+    with np.errstate(invalid="ignore", over="ignore"):
+        s = np.matmul(q.transpose(0, 1, 3, 2), k) * float(scale)
+        off = np.matmul(np.abs(q).transpose(0, 1, 3, 2), np.abs(k)) * float(scale) * 2.0 ** -19 + 2.0 ** -21
+        p = np.exp(s - s.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        o = np.matmul(v, p.transpose(0, 1, 3, 2))
+        bound = np.matmul(np.abs(v), (p * (2 * off.max(-1, keepdims=True) + 2.0 ** -19)).transpose(0, 1, 3, 2))
+    return o.reshape(b, heads * hd, h, w), bound.reshape(b, heads * hd, h, w), v.reshape(b, heads * hd, h, w)
+
+
+def run(hip, qkv, heads, kd, hd, scale):
+    b, c, h, w = qkv.shape
+    hip.begin_frame()
+    try:
+        x = hip.alloc(b, c + 8, h, w).slice(4, c)
+        hip.upload(qkv, x)
+        o = hip.alloc(b, heads * hd + 3, h, w).slice(1, heads * hd)
+        v = hip.alloc(b, heads * hd + 5, h, w).slice(2, heads * hd)
+        hip.profile_enable(True)
+        hip.profile_read()
+        try:
+            hip.attention(x, heads, kd, hd, float(scale), o, v)
+            hip.flush()
+            names = set(hip.profile_read())
+        finally:
+            hip.profile_enable(False)
+        return hip.download(o), hip.download(v), names
+    finally:
+        hip.end_frame()
+
+
+# (batch, heads, key dim, head dim, h, w): one token, fewer key tiles than waves, one past a tile, ragged dims.
+CASES = [(1, 1, 32, 64, 1, 1), (2, 2, 4, 4, 3, 11), (1, 3, 20, 36, 8, 16), (2, 1, 32, 64, 3, 43), (1, 2, 32, 64, 20, 20),
+         (1, 2, 28, 60, 33, 31)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_fused(hip, case):
+    b, heads, kd, hd, h, w = case
+    qkv = synth.activations((b, heads * (2 * kd + hd), h, w), 31 * h + w)
+    scale = np.float32(kd ** -0.5)
+    exp, bound, vexp = reference(qkv, heads, kd, hd, scale)
+    got, v, names = run(hip, qkv, heads, kd, hd, scale)
+    assert names == {"attention"}
+    np.testing.assert_array_equal(v, vexp.astype(np.float32))
+    assert (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
+
+
+@pytest.mark.parametrize("scales", [(1e-6, 1e6, 1e-20), (30.0, 1.0, 1e4), (0.0, 1.0, 1.0), (1e-30, 1e-30, 1e-30)], ids=str)
+def test_operand_scales(hip, scales):
+    """q, k and v far from the first guess of their scales, values that grow by 2^14 over the key tiles."""
+    heads, kd, hd = 2, 32, 64
+    qkv = synth.activations((1, heads, 2 * kd + hd, 12, 16), 5)
+    qkv[:, :, :kd] *= np.float32(scales[0])
+    qkv[:, :, kd:2 * kd] *= np.float32(scales[1])
+    qkv[:, :, 2 * kd:] *= np.float32(scales[2])
+    qkv[:, :, 2 * kd:, 6:] *= np.float32(16384)
+    qkv = qkv.reshape(1, -1, 12, 16)
+    exp, bound, _ = reference(qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    got, _, _ = run(hip, qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    floor = 2.0 ** -38 * float(np.abs(qkv.reshape(1, heads, -1, 192)[:, :, 2 * kd:]).max())
+    assert (np.abs(got - exp) <= bound + floor).all()
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan], ids=str)
+@pytest.mark.parametrize("part", ["q", "k", "v"])
+def test_non_finite(hip, part, value):
+    heads, kd, hd = 1, 32, 64
+    qkv = synth.activations((1, 2 * kd + hd, 7, 9), 6)
+    qkv[0, {"q": 3, "k": kd + 3, "v": 2 * kd + 3}[part], 2, 5] = value
+    exp, _, _ = reference(qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    got, _, _ = run(hip, qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+    fine = np.isfinite(exp)
+    np.testing.assert_array_equal(got[~fine & ~np.isnan(exp)], exp[~fine & ~np.isnan(exp)])
+    np.testing.assert_allclose(got[fine], exp[fine], rtol=0, atol=1e-5)  # 63 products of order 1 in float32
+
+
+def test_wider_dims_keep_the_gemms(hip):
+    heads, kd, hd = 1, 40, 72
+    qkv = synth.activations((2, 2 * kd + hd, 9, 7), 7)
+    exp, bound, vexp = reference(qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    got, v, names = run(hip, qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    assert "attn_softmax" in names
+    np.testing.assert_array_equal(v, vexp.astype(np.float32))
+    assert (np.abs(got - exp) <= bound).all()
