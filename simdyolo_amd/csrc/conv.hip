@@ -2713,6 +2713,7 @@ static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo, int tile) {
   const int oc = p->oc, ic = p->ic, kh = p->kh, kw = p->kw;
   const float* W = p->host_w.data();
   if ((x3 && !p->w_x3) || (c3 && !p->w_c3)) {
+    SY_CHECK(p->finite, SY_EUNSUPPORTED, "the f16-split kernels take finite weights only");
     // Split weights in the GEMM's or the 3x3 patch kernel's operand order
     // (igemm.h), then the channels' inverse scales.
     const int taps = kh * kw, K = taps * ic, nkt = (K + 31) / 32, ng = (ic + 15) / 16, ocp = oc_pad(oc);
@@ -2722,8 +2723,7 @@ static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo, int tile) {
     for (int o = 0; o < oc; ++o) {
       const float* g = W + (size_t)o * K;
       float big = 0.f;
-      for (int i = 0; i < K; ++i)
-        if (std::isfinite(g[i])) big = std::max(big, std::fabs(g[i]));
+      for (int i = 0; i < K; ++i) big = std::max(big, std::fabs(g[i]));
       const float scale = x3_weight_scale(big);
       h[units * 4 + o] = 1.f / scale;
       for (int c = 0; c < ic; ++c)
@@ -2839,6 +2839,7 @@ int conv_prepare(sy_ctx* ctx, ConvPlan* p) {
            "convolution oc=%d ic=%d k=%dx%d groups=%d is not supported by the HIP backend", p->oc, p->ic, p->kh,
            p->kw, p->groups);
   p->algo = algo;
+  for (float w : p->host_w) p->finite = p->finite && std::isfinite(w);
   return pack_weights(ctx, p, algo, -1);
 }
 
@@ -3268,7 +3269,7 @@ static std::vector<ConvChoice> conv_candidates_all(const ConvPlan* p, const sy_t
   // against 58; 3x3 64 -> 64 at 80 x 80: 57 against 73; 3x3 stride 2 64 -> 128:
   // 38 against 82) and no other candidate is timed; smaller grids and shallow
   // products, where the in-workgroup split-K and row kernels can win, time all.
-  if (conv_supports(p, kIgemm) && M * p->oc < (1LL << 40)) {
+  if (conv_supports(p, kIgemm) && p->finite && M * p->oc < (1LL << 40)) {
     for (int i = 0; i < x3_num_tiles(); ++i) cand.push_back(ConvChoice{kIgemm, kX3Base + i});
     const long long wide = (M + 63) / 64 * ((p->oc + 63) / 64);
     if (conv3x3_s1(p)) {

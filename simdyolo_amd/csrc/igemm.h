@@ -177,9 +177,8 @@ extern const X3Tile kX3Tiles[];
 int x3_num_tiles();
 inline bool is_x3_tile(int t) { return t >= kX3Base && t < kX3Base + x3_num_tiles(); }
 const char* x3_name(int t, int mode);
-// hi and lo of a weight times its channel's scale (finite v: within 2^-23 of
-// it; otherwise hi alone holds it), and that power of two for the channel's
-// largest finite magnitude.
+// hi and lo of a (finite) weight times its channel's scale, within 2^-23 of it,
+// and that power of two for the channel's largest magnitude.
 void x3_split(float v, float scale, uint16_t out[2]);
 float x3_weight_scale(float largest);
 int launch_x3(sy_ctx* ctx, int t, int mode, const IgemmArgs& a);
@@ -200,9 +199,9 @@ struct C3Args {
   float* y;
   int ldy, OC, silu;
   int ng;  // groups of 16 input channels
-  // Tile shape, filled by launch_c3: TH x TW outputs, rows per image, tiles
+  // Filled by launch_c3: pixels; TH x TW outputs per tile, rows per image, tiles
   // per row, column blocks, 2^16 / TW and 2^16 / (TW + 2) rounded up.
-  int TH, TW, rpi, ntx, nblk, inv_tw, inv_pw;
+  int M, TH, TW, rpi, ntx, nblk, inv_tw, inv_pw;
 };
 constexpr int kC3Base = 96;  // tile ids kC3Base + i select the i-th form
 int c3_num_forms();

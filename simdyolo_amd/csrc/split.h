@@ -85,23 +85,18 @@ __device__ __forceinline__ void rescale(int se, int ne, f32x16 (&acc)[TM][TN], f
       }
 }
 
-// acc = the sums in true scale; whether one of them is not finite.  ws: the
-// lane's columns' inverse weight scales.
+// acc = the sums in true scale.  ws: the lane's columns' inverse weight scales.
 template <int TM, int TN>
-__device__ __forceinline__ bool unscale(const float (&ws)[TN], int se, f32x16 (&acc)[TM][TN],
+__device__ __forceinline__ void unscale(const float (&ws)[TN], int se, f32x16 (&acc)[TM][TN],
                                         const f32x16 (&crs)[TM][TN]) {
   const float xs = exp_float(254 - se);
-  float bad = 0.f;  // 0 * v is NaN for a non-finite v
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
+      for (int r = 0; r < 16; ++r)
         acc[i][j][r] = __builtin_fmaf(crs[i][j][r], 1.f / 2048, acc[i][j][r]) * xs * ws[j];
-        bad = __builtin_fmaf(acc[i][j][r], 0.f, bad);
-      }
-  return bad != bad;
 }
 
 }  // namespace sy

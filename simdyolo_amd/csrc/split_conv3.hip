@@ -44,6 +44,10 @@ constexpr int kC3BufWord3 = 0x00020000;  // raw buffer resource, word 3 (gfx9 fa
 // LDS pixels a patch may take for a tile of BM outputs.
 constexpr int c3_patch(int bm) { return bm == 64 ? 112 : 192; }
 
+// Low 32 bits of the product of two values below 2^24 (a full-rate instruction,
+// a 32-bit multiply is a quarter-rate one).
+__device__ __forceinline__ int mul24(int x, int y) { return (int)__umul24((unsigned)x, (unsigned)y); }
+
 // Pixel of a 32-pixel block that MFMA row r (lane r of a half wave) holds.
 __device__ __forceinline__ int c3_row(int r) { return ((0x73261540 >> (r & 28)) & 7) * 4 + (r & 3); }
 
@@ -52,15 +56,15 @@ __device__ __forceinline__ float c3_weight(const C3Args& a, int col, int ic, int
                       ((((long long)(col >> 5) * a.ng + (ic >> 4)) * 9 + tap) * 128 + ((ic >> 3) & 1) * 32 +
                        (col & 31)) * 8 + (ic & 7);
   const float hi = (float)e[0], lo = (float)e[512];
-  return (lo == 0.f ? hi : __builtin_fmaf(lo, 1.f / 2048, hi)) * a.ws[col];
+  return __builtin_fmaf(lo, 1.f / 2048, hi) * a.ws[col];
 }
 
-// Epilogue of a wave whose sums are not all finite: its elements again in
-// float32, from the input and the packed weights.
+// Epilogue of a workgroup that read a huge or infinite value: its elements
+// again in float32, from the input and the packed weights.
 __device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int pixels, int col0, int cols, int lane) {
   for (int i = lane; i < pixels * cols; i += 64) {
     const int pix = opix[i / cols], col = col0 + i % cols;
-    if (pix < 0 || col >= a.OC) continue;
+    if (pix >= a.M || col >= a.OC) continue;
     const int ox = pix % a.W, t = pix / a.W, oy = t % a.H, n = t / a.H;
     float v = 0.f;
     for (int tap = 0; tap < 9; ++tap) {
@@ -117,12 +121,12 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
     const bool cok = ch * (16 * G) + 4 * q4 < a.IC;
 #pragma unroll
     for (int i = 0; i < L_IT; ++i) {
-      const int px = px0 + i * (NT / (4 * G)), pr = (px * a.inv_pw) >> 16, ix = ox0 - 1 + px - pr * PW;
+      const int px = px0 + i * (NT / (4 * G)), pr = mul24(px, a.inv_pw) >> 16, ix = ox0 - 1 + px - mul24(pr, PW);
       const bool wrap = a.rpi > a.H && y0 - 1 + pr >= a.rpi;  // into the next image
       const int y = wrap ? y0 - 1 + pr - a.rpi : y0 - 1 + pr;
       const bool ok =
           cok && px < npx && nb + wrap < a.N && (unsigned)y < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-      const int off = ok ? 4 * ((wrap ? (int)img : 0) + (y * a.W + ix) * a.ldx + 4 * q4) : kC3Oob;
+      const int off = ok ? 4 * ((wrap ? (int)img : 0) + mul24(mul24(y, a.W) + ix, a.ldx) + 4 * q4) : kC3Oob;
       d[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, ch * (64 * G), 0));
     }
   };
@@ -170,19 +174,19 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
     bias[j] = col0 + j * 32 < a.OC ? a.bias[col0 + j * 32] : 0.f;
     ws[j] = a.ws[col0 + j * 32];
   }
-  // This tile's output pixels, by MFMA row.
+  // This tile's output pixels by MFMA row; M, past the output, for none.
   for (int p = tid; p < BM; p += NT) {
-    const int q = (p & ~31) + c3_row(p & 31), py = (q * a.inv_tw) >> 16, ox = ox0 + q - py * a.TW;
+    const int q = (p & ~31) + c3_row(p & 31), py = mul24(q, a.inv_tw) >> 16, ox = ox0 + q - mul24(py, a.TW);
     const bool wrap = y0 + py >= a.rpi;
     const int n = wrap ? nb + 1 : nb, oy = wrap ? y0 + py - a.rpi : y0 + py;
-    opix[p] = py < a.TH && n < a.N && oy < a.H && ox < a.W ? (n * a.H + oy) * a.W + ox : -1;
+    opix[p] = py < a.TH && n < a.N && oy < a.H && ox < a.W ? mul24(mul24(n, a.H) + oy, a.W) + ox : a.M;
   }
   // LDS offset (halves) of this lane's operand rows at tap (0, 0).
   int arow[TM];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int p = (wm * TM + i) * 32 + c3_row(r32), py = (p * a.inv_tw) >> 16;
-    arow[i] = (min(py, a.TH - 1) * PW + p - py * a.TW) * 8 + half * PL;
+    const int p = (wm * TM + i) * 32 + c3_row(r32), py = mul24(p, a.inv_tw) >> 16;
+    arow[i] = (mul24(min(py, a.TH - 1), PW) + p - mul24(py, a.TW)) * 8 + half * PL;
   }
   f32x16 acc[TM][TN], crs[TM][TN];
 #pragma unroll
@@ -256,12 +260,18 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
     }
   }
 
-  const bool bad = unscale<TM, TN>(ws, se, acc, crs);
   const int* po = opix + wm * TM * 32;
-  if (__any(bad) || big >= kSplitHuge) {
+  if (big >= kSplitHuge) {
     c3_exact(a, po, TM * 32, col0 - r32, TN * 32, lane);
     return;
   }
+  unscale<TM, TN>(ws, se, acc, crs);
+  // Buffer accesses: a pixel or channel past the output has an offset past the
+  // resource, whose load gives zero and whose store is dropped.
+  const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)a.y, (short)0, 4 * ((a.M - 1) * a.ldy + a.OC), kC3BufWord3);
+  const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)a.res, (short)0, a.res ? 4 * ((a.M - 1) * a.ldr + a.OC) : 0, kC3BufWord3);
   // D layout: lane holds column r32 of rows 8 (r / 4) + 4 half + r % 4.
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -270,24 +280,24 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
     for (int r = 0; r < 16; ++r) px[r] = po[i * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int col = col0 + j * 32;
-      if (col >= a.OC) continue;
-      float v[16];
+      const unsigned col = col0 + j * 32 < a.OC ? 4u * (col0 + j * 32) : 0x80000000u;
+      float v[16], rv[16];
+      if (a.res) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          rv[r] = __builtin_bit_cast(float,
+                                     __builtin_amdgcn_raw_buffer_load_b32(rr, mul24(px[r], 4 * a.ldr) + col, 0, 0));
+      }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         v[r] = acc[i][j][r] + bias[j];
         if (a.silu) v[r] = silu_fast(v[r]);
-      }
-      if (a.res) {
-        float rv[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) rv[r] = a.res[(unsigned)(max(px[r], 0) * a.ldr + col)];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = rv[r] + v[r];
+        if (a.res) v[r] = rv[r] + v[r];
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        if (px[r] >= 0) a.y[(unsigned)(px[r] * a.ldy + col)] = v[r];
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[r]), yr, mul24(px[r], 4 * a.ldy) + col, 0,
+                                              0);
     }
   }
 }
@@ -353,11 +363,12 @@ static bool pick_tile_shape(int bm, int N, int H, int W, int* th, int* tw, int* 
 }
 
 bool c3_fits(const C3Args& a) {
-  // 32-bit offsets: the two images a tile may span below the zero-read
-  // offset, every output and residual element below 2^31.
+  // 32-bit byte offsets: the two images a tile may span below the zero-read
+  // offset, outputs and residuals below 2^31; pixel counts for 24-bit multiplies.
   const long long img = 4LL * a.H * a.W * a.ldx, M = (long long)a.N * a.H * a.W;
-  return 2 * img < kC3Oob && M * a.ldy < (1LL << 31) && M * a.ldr < (1LL << 31) &&
-         (long long)a.N * (a.H + 64) < (1LL << 31) && (long long)a.ng * (9 * 128 * 16 * 4) < (1LL << 31);
+  return 2 * img < kC3Oob && 4 * M * a.ldy < (1LL << 31) && 4 * M * a.ldr < (1LL << 31) && M < (1LL << 24) &&
+         4LL * a.ldy < (1LL << 24) && 4LL * a.ldr < (1LL << 24) && a.ldx < (1LL << 24) &&
+         (long long)a.N * (a.H + 64) < (1LL << 24) && (long long)a.ng * (9 * 128 * 16 * 4) < (1LL << 31);
 }
 
 int launch_c3(sy_ctx* ctx, int f, C3Args a) {
@@ -366,6 +377,7 @@ int launch_c3(sy_ctx* ctx, int f, C3Args a) {
   long long tiles = 0;
   SY_CHECK(pick_tile_shape(bm, a.N, a.H, a.W, &a.TH, &a.TW, &a.rpi, &tiles, &a.ntx), SY_EUNSUPPORTED,
            "no tile for a %dx%d image", a.H, a.W);
+  a.M = a.N * a.H * a.W;
   a.nblk = ((a.OC + 31) / 32 + c.wn * c.tn - 1) / (c.wn * c.tn);
   a.inv_tw = 65536 / a.TW + 1;
   a.inv_pw = 65536 / (a.TW + 2) + 1;

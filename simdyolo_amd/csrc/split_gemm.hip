@@ -25,11 +25,11 @@
 // 32, against the float32 tiles: 1x1 384 -> 128 at 40 x 40 58 -> 30 us (105 MB
 // at 3.6 TB/s), 3x3 stride 2 64 -> 128 at 80 x 80 82 -> 38 us.
 //
-// Non-finite results: an infinite value becomes NaN in lo.  A wave whose
-// sums hold a non-finite value, and every wave of a workgroup that read a
-// magnitude of 2^100 or more (whose scale would leave nothing of the others),
-// computes its tile again in plain float32 from the same operands: infinities
-// and NaN propagate as they do in the float32 kernels.
+// Non-finite operands: an infinite value becomes NaN in lo, and a scale for
+// magnitudes of 2^100 or more would leave nothing of the others.  A workgroup
+// that reads such a value computes its tile again in plain float32 from the
+// same operands, and convolutions with non-finite weights are not routed here:
+// infinities and NaN propagate as they do in the float32 kernels.
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -65,14 +65,13 @@ __device__ __forceinline__ float x3_element(const IgemmArgs& a, int row, int col
     const _Float16* e =
         w + ((long long)(k >> 5) * kX3Units + ((k >> 4) & 1) * 128 + ((k >> 3) & 1) * 32 + (col & 31)) * 8 + (k & 7);
     const float hi = (float)e[0], lo = (float)e[512];
-    // An infinite or NaN weight sits in hi alone.
-    s = __builtin_fmaf(xv, (lo == 0.f ? hi : __builtin_fmaf(lo, 1.f / 2048, hi)) * ws, s);
+    s = __builtin_fmaf(xv, __builtin_fmaf(lo, 1.f / 2048, hi) * ws, s);
   }
   return s;
 }
 
-// Epilogue of a tile that holds non-finite sums: every element again in
-// float32, then bias, SiLU, residual and the store as in store_acc.
+// Epilogue of a workgroup that read a huge or infinite value: every element
+// again in float32, then bias, SiLU, residual and the store as in store_acc.
 template <int MODE>
 __device__ __forceinline__ void x3_exact_tile(const IgemmArgs& a, int row0, int rows, int col0, int cols, int lane) {
   for (int i = lane; i < rows * cols; i += 64) {
@@ -278,11 +277,11 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
   float ws[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) ws[j] = a.w3s[col0 + j * 32 + r32];
-  const bool bad = unscale<TM, TN>(ws, se, acc, crs);
-  if (__any(bad) || big >= kSplitHuge) {
+  if (big >= kSplitHuge) {
     x3_exact_tile<MODE>(a, row0, BM / WM, col0, BN / WN, lane);
     return;
   }
+  unscale<TM, TN>(ws, se, acc, crs);
   if (MODE == 2 && a.shuf > 0)
     store_shuf<TM, TN>(a, a.y, acc, row0 + 4 * half, col0 + r32);
   else
@@ -342,11 +341,6 @@ static inline float f16_value(uint16_t h) {
 }
 
 void x3_split(float v, float scale, uint16_t out[2]) {
-  if (!std::isfinite(v)) {
-    out[0] = std::isnan(v) ? 0x7e00 : v > 0 ? 0x7c00 : 0xfc00;
-    out[1] = 0;
-    return;
-  }
   const float s = v * scale;
   out[0] = f16_bits(s);
   out[1] = f16_bits((s - f16_value(out[0])) * 2048.f);

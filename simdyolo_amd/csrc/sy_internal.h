@@ -235,6 +235,7 @@ struct ConvPlan {
   // depthwise: [kh*kw][round_up(oc, 4)]
   float* w_dw = nullptr;
   float* bias = nullptr;  // [round_up(oc, 128)] zero padded
+  bool finite = true;  // every weight is finite
   std::vector<float> host_w, host_b;  // OIHW copy kept to repack on algo change
 };
 
