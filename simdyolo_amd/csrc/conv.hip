@@ -2661,17 +2661,18 @@ static bool fused_wino_fits(const sy_tensor* x) {
   return 4 * img * (31 / tpi + 2) < kFxOob;
 }
 
-// 3x3 stride-1 pad-1 undilated ungrouped convolution on whole float4s.
-static bool conv3x3_s1(const ConvPlan* p) {
-  return p->groups == 1 && p->kh == 3 && p->kw == 3 && p->sh == 1 && p->sw == 1 && p->dh == 1 && p->dw == 1 &&
-         p->pt == 1 && p->pl == 1 && p->pb == 1 && p->pr == 1 && p->ic % 4 == 0;
+// 3x3 pad-1 undilated ungrouped convolution of that stride on whole float4s.
+static bool conv3x3(const ConvPlan* p, int stride) {
+  return p->groups == 1 && p->kh == 3 && p->kw == 3 && p->sh == stride && p->sw == stride && p->dh == 1 &&
+         p->dw == 1 && p->pt == 1 && p->pl == 1 && p->pb == 1 && p->pr == 1 && p->ic % 4 == 0 && !p->up2;
 }
+static bool conv3x3_patch(const ConvPlan* p) { return conv3x3(p, 1) || conv3x3(p, 2); }
 
 bool conv_supports(const ConvPlan* p, int algo) {
   const bool g1 = p->groups == 1;
   switch (algo) {
     case kIgemm: return g1 && p->ic % 4 == 0;
-    case kWinograd: return conv3x3_s1(p) && p->oc % 4 == 0;
+    case kWinograd: return conv3x3(p, 1) && p->oc % 4 == 0;
     case kDirect: return g1 && p->kh * p->kw * p->ic <= 1024;
     case kWinograd3: return conv_supports(p, kWinograd);
     case kDepthwise: return p->groups == p->ic && p->ic == p->oc;
@@ -3040,20 +3041,21 @@ static int conv_exec(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tens
   if (algo == kIgemm && is_c3_tile(et)) {
     C3Args a{};
     a.x = x->data; a.N = x->n; a.H = x->h; a.W = x->w; a.IC = x->c; a.ldx = x->ldc;
+    a.S = p->sh; a.OH = oh; a.OW = ow;
     a.w = p->w_c3; a.ws = p->w_c3s; a.bias = p->bias;
     a.res = res ? res->data : nullptr; a.ldr = res ? res->ldc : 0;
     a.y = y->data; a.ldy = y->ldc; a.OC = p->oc; a.silu = p->silu; a.ng = (p->ic + 15) / 16;
-    if (!conv3x3_s1(p) || ctx->up_src || !c3_fits(a)) {
+    if (!conv3x3_patch(p) || ctx->up_src || !c3_fits(a)) {
       // Views past the kernel's 32-bit offsets (the tuned choice is kept by
       // shape, not by pitch) take the routing rule.
       SY_CHECK(ch.tile >= 0, SY_EUNSUPPORTED,
-               "the 3x3 patch kernel needs a 3x3 stride-1 pad-1 convolution of 32-bit extent");
+               "the 3x3 patch kernel needs a 3x3 stride-1 or -2 pad-1 convolution of 32-bit extent");
       return conv_exec(ctx, p, x, y, res, ConvChoice{p->algo, -1});
     }
     const double px = (double)x->n * oh * ow;
     const char* pn = c3_name(et - kC3Base);
     ProfScope prof(ctx, pn, 2.0 * 9 * px * p->ic * p->oc,
-                   4.0 * (px * p->ic + px * p->oc * (res ? 2 : 1) + 9.0 * p->ic * p->oc));
+                   4.0 * ((double)x->n * x->h * x->w * p->ic + px * p->oc * (res ? 2 : 1) + 9.0 * p->ic * p->oc));
     SY_TRY(launch_c3(ctx, et - kC3Base, a));
     return check_launch(pn);
   }
@@ -3266,13 +3268,13 @@ static std::vector<ConvChoice> conv_candidates_all(const ConvPlan* p, const sy_t
   // The f16-split kernels.  Where 64 x 64 output tiles fill the CUs twice over
   // they are the fastest of all at every layer shape of the YOLO families with
   // at least 64 multiplied channels (1x1 384 -> 128 at 40 x 40, batch 32: 30 us
-  // against 58; 3x3 64 -> 64 at 80 x 80: 57 against 73; 3x3 stride 2 64 -> 128:
+  // against 58; 3x3 64 -> 64 at 80 x 80: 52 against 73; 3x3 stride 2 64 -> 128:
   // 38 against 82) and no other candidate is timed; smaller grids and shallow
   // products, where the in-workgroup split-K and row kernels can win, time all.
   if (conv_supports(p, kIgemm) && p->finite && M * p->oc < (1LL << 40)) {
     for (int i = 0; i < x3_num_tiles(); ++i) cand.push_back(ConvChoice{kIgemm, kX3Base + i});
     const long long wide = (M + 63) / 64 * ((p->oc + 63) / 64);
-    if (conv3x3_s1(p)) {
+    if (conv3x3_patch(p)) {
       for (int i = 0; i < c3_num_forms(); ++i) cand.push_back(ConvChoice{kIgemm, kC3Base + i});
     }
     if (wide >= 512 && K >= 64 && p->ic >= 32) return cand;

@@ -185,12 +185,12 @@ int launch_x3(sy_ctx* ctx, int t, int mode, const IgemmArgs& a);
 
 // ------------------------------------------------------------ 3x3 from an LDS patch, f16 split
 
-// split_conv3.hip: 3x3 stride-1 pad-1 convolution.  Packed weights: channel o,
+// split_conv3.hip: 3x3 pad-1 convolution of stride S = 1 or 2.  Packed weights: channel o,
 // input channel c, tap, split s in f16 element c % 8 of 16-byte unit
 // (((o / 32) ng + c / 16) 9 + tap) 128 + 64 s + 32 ((c / 8) % 2) + o % 32.
 struct C3Args {
   const float* x;
-  int N, H, W, IC, ldx;
+  int N, H, W, IC, ldx, S, OH, OW;
   const void* w;
   const float* ws;    // per output channel: 1 / the weights' scale
   const float* bias;  // padded to whole column blocks
@@ -200,7 +200,8 @@ struct C3Args {
   int ldy, OC, silu;
   int ng;  // groups of 16 input channels
   // Filled by launch_c3: pixels; TH x TW outputs per tile, rows per image, tiles
-  // per row, column blocks, 2^16 / TW and 2^16 / (TW + 2) rounded up.
+  // per row, column blocks, reciprocals of TW (2^16) and of the patch width
+  // (2^16, at stride 2 2^20), rounded up.
   int M, TH, TW, rpi, ntx, nblk, inv_tw, inv_pw;
 };
 constexpr int kC3Base = 96;  // tile ids kC3Base + i select the i-th form

@@ -1,10 +1,11 @@
-// 3x3 stride-1 convolution on the f16 matrix cores, from an LDS patch.
+// 3x3 convolution, stride 1 or 2, on the f16 matrix cores, from an LDS patch.
 //
 // The arithmetic is split_gemm.hip's (float32 as scaled f16 pairs, three
 // products).  Its implicit GEMM stages and splits every input value once per
 // tap; here a workgroup stages the input patch of its output tile (TH x TW
-// outputs, (TH + 2) x (TW + 2) inputs) once, up to 64 channels at a time, and
-// the nine taps read it at shifted pixels.  All of a chunk's loads are issued
+// outputs, (TH + 2) x (TW + 2) inputs at stride 1, (2 TH + 1) x (2 TW + 1) at
+// stride 2) once, up to 64 channels at a time, and the nine taps read it at
+// shifted pixels.  All of a chunk's loads are issued
 // together: 16 channels at a time left too few bytes in flight, and every
 // wait for weights behind them (loads return in order) cost a memory latency.  Weights stream from L2 straight into MFMA
 // operands: their packed order makes each read of a wave 1 KiB contiguous, and
@@ -14,13 +15,16 @@
 // channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
 // MFMAs of 32 cycles.
 //
-// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 57 us,
+// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 52 us,
 // against 73 us for the fastest float32 Winograd form.  The matrix cores are
-// busy for a third of it at the 1.8 GHz the GPU holds under this load; a
-// 128-pixel workgroup's 31,000 cycles are 14,000 of taps, 8,000 of patch loads
-// and 7,000 of epilogue, and 1,600 of them on 256 CUs leave a thin last round.
+// busy for 46% of it at the 1.8 GHz the GPU holds under this load; the patch
+// loads (8,000 of a 128-pixel workgroup's 29,000 cycles), the epilogue (6,000)
+// and a thin last round of 1,600 workgroups on 256 CUs take the rest.
 // Workgroups that run through several tiles with the next patch loaded behind
 // the last taps measured the same, 16-channel double buffering 57 - 60 us.
+// Stride 2, batch 32, against the implicit GEMM of split_gemm.hip, which stages
+// every input per tap: 64 -> 128 at 80 x 80 42 -> 38 us, 32 -> 64 at 160 x 160
+// 49 -> 41, 16 -> 32 at 320 x 320 88 -> 75 (315 MB), 128 -> 128 at 40 x 40 33 -> 22.
 //
 // LDS holds the patch as planes of 8 channels, [split][8-channel block][pixel]
 // [8].  ds_read_b128 serves 16 lanes a cycle over 64 banks, lanes 0-3, 12-15,
@@ -42,7 +46,8 @@ constexpr int kC3Oob = 0x40000000;       // buffer offset past every record: the
 constexpr int kC3BufWord3 = 0x00020000;  // raw buffer resource, word 3 (gfx9 family)
 
 // LDS pixels a patch may take for a tile of BM outputs.
-constexpr int c3_patch(int bm) { return bm == 64 ? 112 : 192; }
+constexpr int c3_patch(int bm, int s) { return s == 1 ? (bm == 64 ? 112 : 192) : (bm == 64 ? 304 : 568); }
+constexpr int c3_extent(int n, int s) { return s * (n - 1) + 3; }  // inputs under n outputs
 
 // Low 32 bits of the product of two values below 2^24 (a full-rate instruction,
 // a 32-bit multiply is a quarter-rate one).
@@ -65,10 +70,10 @@ __device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int p
   for (int i = lane; i < pixels * cols; i += 64) {
     const int pix = opix[i / cols], col = col0 + i % cols;
     if (pix >= a.M || col >= a.OC) continue;
-    const int ox = pix % a.W, t = pix / a.W, oy = t % a.H, n = t / a.H;
+    const int ox = pix % a.OW, t = pix / a.OW, oy = t % a.OH, n = t / a.OH;
     float v = 0.f;
     for (int tap = 0; tap < 9; ++tap) {
-      const int iy = oy - 1 + tap / 3, ix = ox - 1 + tap % 3;
+      const int iy = oy * a.S - 1 + tap / 3, ix = ox * a.S - 1 + tap % 3;
       if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
       const float* x = a.x + (((long long)n * a.H + iy) * a.W + ix) * a.ldx;
       for (int c = 0; c < a.IC; ++c) v = __builtin_fmaf(x[c], c3_weight(a, col, c, tap), v);
@@ -80,11 +85,13 @@ __device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int p
   }
 }
 
-// G: 16-channel groups per chunk.
-template <int G, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G == 4 && WM * WN == 2) ? 2 : 4) void conv3_kernel(
+// S: stride.  G: 16-channel groups per chunk.  At stride 2 a patch row holds its
+// even columns, then the odd ones, so that the operand reads of neighbouring
+// outputs are neighbours at every tap.
+template <int S, int G, int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 || S == 2 ? 2 : 3) : (G == 4 || S == 2) && WM * WN == 2 ? 2 : S == 2 ? 3 : 4) void conv3_kernel(
     const C3Args a) {
-  constexpr int NW = WM * WN, NT = NW * 64, BM = WM * TM * 32, NPX = c3_patch(BM);
+  constexpr int NW = WM * WN, NT = NW * 64, BM = WM * TM * 32, NPX = c3_patch(BM, S);
   constexpr int PL = (NPX * 8 + 127) / 128 * 128 + 64 / G;  // halves per plane
   constexpr int L_IT = (NPX * 4 * G + NT - 1) / NT;         // float4 loads per thread and chunk
   __shared__ __attribute__((aligned(16))) _Float16 P[G * 4 * PL];
@@ -102,11 +109,11 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
   const int T = xcd * q8 + (xcd < rem ? xcd : rem) + (L >> 3);
   const int tile = T / a.nblk, ob0 = (T - tile * a.nblk) * (WN * TN) + wn * TN;
   const int trow = tile / a.ntx, ox0 = (tile - trow * a.ntx) * a.TW;
-  // Tile rows run over virtual rows, rpi per image: H + 1 with tiles that may
-  // span images (the row past H is the zero row between two images), or a
-  // multiple of TH with tiles inside one image.
+  // Tile rows run over virtual output rows, rpi per image: OH + 1 with tiles
+  // that may span images (the inputs of the row past OH are the zero rows
+  // between two images), or a multiple of TH with tiles inside one image.
   const int v0 = trow * a.TH, nb = v0 / a.rpi, y0 = v0 - nb * a.rpi;
-  const int PW = a.TW + 2, npx = (a.TH + 2) * PW;
+  const int PW = c3_extent(a.TW, S), npx = c3_extent(a.TH, S) * PW, odd = (PW + 1) >> 1;
 
   // Patch values this thread stages: its i-th float4 is channels 4 q4 .. + 3 of
   // the chunk, of patch pixel px0 + i NT / 4G.  Byte offsets from the tile's
@@ -116,14 +123,18 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(a.x + nb * img), (short)0, (int)min(span, (long long)kC3Oob), kC3BufWord3);
   const int q4 = tid % (4 * G), px0 = tid / (4 * G);
+  // Row of patch pixel px: at most 568 pixels, the quotient by a 2^16 or 2^20
+  // reciprocal is exact.
+  auto patch_row = [&](int px) { return mul24(px, a.inv_pw) >> (S == 1 ? 16 : 20); };
   f32x4 d[L_IT];
   auto xload = [&](int ch) {
     const bool cok = ch * (16 * G) + 4 * q4 < a.IC;
 #pragma unroll
     for (int i = 0; i < L_IT; ++i) {
-      const int px = px0 + i * (NT / (4 * G)), pr = mul24(px, a.inv_pw) >> 16, ix = ox0 - 1 + px - mul24(pr, PW);
-      const bool wrap = a.rpi > a.H && y0 - 1 + pr >= a.rpi;  // into the next image
-      const int y = wrap ? y0 - 1 + pr - a.rpi : y0 - 1 + pr;
+      const int px = px0 + i * (NT / (4 * G)), pr = patch_row(px), ix = S * ox0 - 1 + px - mul24(pr, PW);
+      const int row = S * y0 - 1 + pr;
+      const bool wrap = a.rpi > a.OH && row >= S * a.rpi;  // into the next image
+      const int y = wrap ? row - S * a.rpi : row;
       const bool ok =
           cok && px < npx && nb + wrap < a.N && (unsigned)y < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
       const int off = ok ? 4 * ((wrap ? (int)img : 0) + mul24(mul24(y, a.W) + ix, a.ldx) + 4 * q4) : kC3Oob;
@@ -139,8 +150,13 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
       const int px = px0 + i * (NT / (4 * G));
       u32x2 hi, lo;
       split4(d[i], s, hi, lo);
-      if (L_IT * NT == NPX * 4 * G || px < NPX) {
-        _Float16* dst = P + (q4 >> 1) * PL + px * 8 + (q4 & 1) * 4;
+      if (S == 2 ? px < npx : (L_IT * NT == NPX * 4 * G || px < NPX)) {
+        int at = px;
+        if (S == 2) {
+          const int row = mul24(patch_row(px), PW), c = px - row;
+          at = row + (c >> 1) + (c & 1 ? odd : 0);
+        }
+        _Float16* dst = P + (q4 >> 1) * PL + at * 8 + (q4 & 1) * 4;
         *(u32x2*)dst = hi;
         *(u32x2*)(dst + 2 * G * PL) = lo;
       }
@@ -179,14 +195,14 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
     const int q = (p & ~31) + c3_row(p & 31), py = mul24(q, a.inv_tw) >> 16, ox = ox0 + q - mul24(py, a.TW);
     const bool wrap = y0 + py >= a.rpi;
     const int n = wrap ? nb + 1 : nb, oy = wrap ? y0 + py - a.rpi : y0 + py;
-    opix[p] = py < a.TH && n < a.N && oy < a.H && ox < a.W ? mul24(mul24(n, a.H) + oy, a.W) + ox : a.M;
+    opix[p] = py < a.TH && n < a.N && oy < a.OH && ox < a.OW ? mul24(mul24(n, a.OH) + oy, a.OW) + ox : a.M;
   }
   // LDS offset (halves) of this lane's operand rows at tap (0, 0).
   int arow[TM];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int p = (wm * TM + i) * 32 + c3_row(r32), py = mul24(p, a.inv_tw) >> 16;
-    arow[i] = (mul24(min(py, a.TH - 1), PW) + p - mul24(py, a.TW)) * 8 + half * PL;
+    arow[i] = (S * mul24(min(py, a.TH - 1), PW) + p - mul24(py, a.TW)) * 8 + half * PL;
   }
   f32x16 acc[TM][TN], crs[TM][TN];
 #pragma unroll
@@ -230,7 +246,8 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 ? 2 : 3) : (G =
 #pragma unroll
         for (int p = 0; p < 2; ++p)
           av[tap & 1][i][p] =
-              *(const f16x8*)(pg + p * (2 * G * PL) + arow[i] + (tap / 3) * PW * 8 + (tap % 3) * 8);
+              *(const f16x8*)(pg + p * (2 * G * PL) + arow[i] +
+                              ((tap / 3) * PW + (S == 1 ? tap % 3 : tap % 3 == 1 ? odd : tap % 3 / 2)) * 8);
     };
     aload(0);
     // The barriers pin the order: operands of the next tap, this tap's MFMAs,
@@ -334,12 +351,13 @@ const char* c3_name(int f) {
 // Output tile of at most bm pixels whose patch fits, with the fewest tiles:
 // TW from 4 to bm columns (a multiple of 16 among equals: its operand reads are
 // free of bank conflicts), tiles inside one image or over virtual rows.
-static bool pick_tile_shape(int bm, int N, int H, int W, int* th, int* tw, int* rpi, long long* tiles, int* ntx) {
+static bool pick_tile_shape(int bm, const C3Args& a, int* th, int* tw, int* rpi, long long* tiles, int* ntx) {
+  const int S = a.S, N = a.N, H = a.OH, W = a.OW;
   long long best = -1;
-  int best_px = 0;
   for (int w = 4; w <= bm && w <= ((W + 3) & ~3); ++w) {
-    int h = std::min(bm / w, c3_patch(bm) / (w + 2) - 2);
-    if (h < 1) continue;
+    const int rows = c3_patch(bm, S) / c3_extent(w, S);
+    const int h = std::min(bm / w, (rows - 3) / S + 1);
+    if (rows < 3 || h < 1) continue;
     const int tx = (W + w - 1) / w;
     for (int span = 0; span < 2; ++span) {
       // A tile spans at most two images.
@@ -347,10 +365,8 @@ static bool pick_tile_shape(int bm, int N, int H, int W, int* th, int* tw, int* 
       if (hh < 1) continue;
       const int r = span ? H + 1 : (H + hh - 1) / hh * hh;
       const long long t = ((long long)N * r + hh - 1) / hh * tx;
-      const int px = (hh + 2) * (w + 2);
-      if (best < 0 || t < best || (t == best && (w % 16 == 0 || (*tw % 16 && px <= best_px)))) {
+      if (best < 0 || t < best || (t == best && w % 16 == 0)) {
         best = t;
-        best_px = px;
         *th = hh;
         *tw = w;
         *rpi = r;
@@ -365,9 +381,10 @@ static bool pick_tile_shape(int bm, int N, int H, int W, int* th, int* tw, int* 
 bool c3_fits(const C3Args& a) {
   // 32-bit byte offsets: the two images a tile may span below the zero-read
   // offset, outputs and residuals below 2^31; pixel counts for 24-bit multiplies.
-  const long long img = 4LL * a.H * a.W * a.ldx, M = (long long)a.N * a.H * a.W;
+  const long long img = 4LL * a.H * a.W * a.ldx, M = (long long)a.N * a.OH * a.OW;
   return 2 * img < kC3Oob && 4 * M * a.ldy < (1LL << 31) && 4 * M * a.ldr < (1LL << 31) && M < (1LL << 24) &&
          4LL * a.ldy < (1LL << 24) && 4LL * a.ldr < (1LL << 24) && a.ldx < (1LL << 24) &&
+         (long long)a.H * a.W < (1LL << 24) &&
          (long long)a.N * (a.H + 64) < (1LL << 24) && (long long)a.ng * (9 * 128 * 16 * 4) < (1LL << 31);
 }
 
@@ -375,19 +392,23 @@ int launch_c3(sy_ctx* ctx, int f, C3Args a) {
   const C3Form& c = kC3Forms[f];
   const int bm = c.wm * c.tm * 32;
   long long tiles = 0;
-  SY_CHECK(pick_tile_shape(bm, a.N, a.H, a.W, &a.TH, &a.TW, &a.rpi, &tiles, &a.ntx), SY_EUNSUPPORTED,
-           "no tile for a %dx%d image", a.H, a.W);
-  a.M = a.N * a.H * a.W;
+  SY_CHECK(pick_tile_shape(bm, a, &a.TH, &a.TW, &a.rpi, &tiles, &a.ntx), SY_EUNSUPPORTED, "no tile for a %dx%d image",
+           a.H, a.W);
+  a.M = a.N * a.OH * a.OW;
   a.nblk = ((a.OC + 31) / 32 + c.wn * c.tn - 1) / (c.wn * c.tn);
   a.inv_tw = 65536 / a.TW + 1;
-  a.inv_pw = 65536 / (a.TW + 2) + 1;
+  a.inv_pw = (a.S == 1 ? 1 << 16 : 1 << 20) / c3_extent(a.TW, a.S) + 1;
   SY_CHECK(tiles * a.nblk < (1LL << 31), SY_EUNSUPPORTED, "convolution grid too large");
   void (*k)(const C3Args) = nullptr;
-#define SY_C3_CASE(i, wm, wn, tm, tn)                 \
-  if (f == i)                                         \
-    k = a.ng == 1   ? conv3_kernel<1, wm, wn, tm, tn> \
-        : a.ng == 2 ? conv3_kernel<2, wm, wn, tm, tn> \
-                    : conv3_kernel<4, wm, wn, tm, tn>;
+  // Chunks of up to 64 channels for the wide forms at stride 1; 32 for the
+  // 32-channel forms (twice the workgroups per CU: 80 -> 80 at 80 x 80, batch 32,
+  // 104 against 119 us) and for stride 2 (four times the patch).
+#define SY_C3_CASE(i, wm, wn, tm, tn)                                                        \
+  if (f == i)                                                                                 \
+    k = a.S == 2    ? (a.ng == 1 ? conv3_kernel<2, 1, wm, wn, tm, tn> : conv3_kernel<2, 2, wm, wn, tm, tn>) \
+        : a.ng == 1 ? conv3_kernel<1, 1, wm, wn, tm, tn>                                      \
+        : a.ng == 2 || wn * tn == 1 ? conv3_kernel<1, 2, wm, wn, tm, tn>                      \
+                    : conv3_kernel<1, 4, wm, wn, tm, tn>;
   SY_C3_LIST(SY_C3_CASE)
 #undef SY_C3_CASE
   SY_CHECK(k != nullptr, SY_EINVAL, "no split 3x3 form %d", f);

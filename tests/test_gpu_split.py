@@ -123,6 +123,24 @@ def test_patch_forms(hip, monkeypatch, form, shape, res):
     near(got, exp, mag)
 
 
+# (n, ic, h, w, oc): odd and even extents, one pixel, tiles across images, three chunks.
+PATCH_S2 = [(1, 4, 1, 1, 1), (3, 16, 2, 5, 33), (5, 20, 20, 20, 24), (2, 32, 35, 66, 64), (1, 80, 45, 75, 96),
+            (2, 36, 9, 17, 40)]
+
+
+@pytest.mark.parametrize("res", [False, True], ids=["plain", "res"])
+@pytest.mark.parametrize("shape", PATCH_S2, ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("form", range(len(C3_FORMS)))
+def test_patch_forms_stride_2(hip, monkeypatch, form, shape, res):
+    n, ic, h, w, oc = shape
+    x, wt, b = data(n, ic, h, w, oc, 3, 250 + form)
+    r = synth.activations((n, oc, (h + 1) // 2, (w + 1) // 2), 9) if res else None
+    exp, mag = conv64(x, wt, b, 2, True, r)
+    got, names = run(hip, monkeypatch, C3_BASE + form, x, wt, b, 2, True, r)
+    assert names == {"conv3_x3_%dx%d_%d%d" % C3_FORMS[form]}
+    near(got, exp, mag)
+
+
 @pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3], ids=["gemm", "patch"])
 @pytest.mark.parametrize("scale", [0.0, 1e-30, 1e-6, 3e4, 1e30], ids=str)
 def test_scales(hip, monkeypatch, tile, scale):
