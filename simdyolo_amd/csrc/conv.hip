@@ -3275,7 +3275,12 @@ static std::vector<ConvChoice> conv_candidates_all(const ConvPlan* p, const sy_t
     for (int i = 0; i < x3_num_tiles(); ++i) cand.push_back(ConvChoice{kIgemm, kX3Base + i});
     const long long wide = (M + 63) / 64 * ((p->oc + 63) / 64);
     if (conv3x3_patch(p)) {
-      for (int i = 0; i < c3_num_forms(); ++i) cand.push_back(ConvChoice{kIgemm, kC3Base + i});
+      // Forms whose waves share out the channel groups: only while the plain
+      // ones leave most CUs idle, and with a group for most of the waves.
+      for (int i = 0; i < c3_num_forms(); ++i) {
+        const int kw = c3_form_groups(i);
+        if (kw == 1 || (wide < 256 && (p->ic + 15) / 16 * 4 >= 3 * kw)) cand.push_back(ConvChoice{kIgemm, kC3Base + i});
+      }
     }
     if (wide >= 512 && K >= 64 && p->ic >= 32) return cand;
   }

@@ -207,6 +207,7 @@ struct C3Args {
 constexpr int kC3Base = 96;  // tile ids kC3Base + i select the i-th form
 int c3_num_forms();
 inline bool is_c3_tile(int t) { return t >= kC3Base && t < kC3Base + c3_num_forms(); }
+int c3_form_groups(int f);  // waves that share out a block's channel groups (1: none)
 const char* c3_name(int f);
 bool c3_fits(const C3Args& a);
 int launch_c3(sy_ctx* ctx, int f, C3Args a);

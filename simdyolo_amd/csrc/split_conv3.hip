@@ -22,6 +22,9 @@
 // and a thin last round of 1,600 workgroups on 256 CUs take the rest.
 // Workgroups that run through several tiles with the next patch loaded behind
 // the last taps measured the same, 16-channel double buffering 57 - 60 us.
+// At batch 1 the chain of taps is the time: sharing a block's groups out over
+// four or eight waves (KW) takes 64 -> 64 at 40 x 40 from 6.3 to 5.0 us, 128 -> 128
+// at 20 x 20 from 9.3 to 6.0, 256 -> 64 at 20 x 20 from 15.5 to 8.1.
 // Stride 2, batch 32, against the implicit GEMM of split_gemm.hip, which stages
 // every input per tap: 64 -> 128 at 80 x 80 42 -> 38 us, 32 -> 64 at 160 x 160
 // 49 -> 41, 16 -> 32 at 320 x 320 88 -> 75 (315 MB), 128 -> 128 at 40 x 40 33 -> 22.
@@ -46,7 +49,9 @@ constexpr int kC3Oob = 0x40000000;       // buffer offset past every record: the
 constexpr int kC3BufWord3 = 0x00020000;  // raw buffer resource, word 3 (gfx9 family)
 
 // LDS pixels a patch may take for a tile of BM outputs.
-constexpr int c3_patch(int bm, int s) { return s == 1 ? (bm == 64 ? 112 : 192) : (bm == 64 ? 304 : 568); }
+constexpr int c3_patch(int bm, int s) {
+  return s == 1 ? (bm == 32 ? 72 : bm == 64 ? 112 : 192) : (bm == 32 ? 168 : bm == 64 ? 304 : 568);
+}
 constexpr int c3_extent(int n, int s) { return s * (n - 1) + 3; }  // inputs under n outputs
 
 // Low 32 bits of the product of two values below 2^24 (a full-rate instruction,
@@ -87,19 +92,23 @@ __device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int p
 
 // S: stride.  G: 16-channel groups per chunk.  At stride 2 a patch row holds its
 // even columns, then the odd ones, so that the operand reads of neighbouring
-// outputs are neighbours at every tap.
-template <int S, int G, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 || S == 2 ? 2 : 3) : (G == 4 || S == 2) && WM * WN == 2 ? 2 : S == 2 ? 3 : 4) void conv3_kernel(
+// outputs are neighbours at every tap.  KW > 1: the tile's channel groups shared
+// out over KW waves (small grids: a fourth or an eighth of the chain of taps),
+// their sums joined through LDS, each wave finishing 16 / KW of the rows.
+template <int S, int G, int WM, int WN, int TM, int TN, int KW>
+__global__ __launch_bounds__(WM* WN* KW * 64, KW > 1 ? 2 : TM * TN == 2 ? (G == 4 || S == 2 ? 2 : 3) : (G == 4 || S == 2) && WM * WN == 2 ? 2 : S == 2 ? 3 : 4) void conv3_kernel(
     const C3Args a) {
-  constexpr int NW = WM * WN, NT = NW * 64, BM = WM * TM * 32, NPX = c3_patch(BM, S);
+  constexpr int NW = WM * WN * KW, NT = NW * 64, BM = WM * TM * 32, NPX = c3_patch(BM, S);
   constexpr int PL = (NPX * 8 + 127) / 128 * 128 + 64 / G;  // halves per plane
   constexpr int L_IT = (NPX * 4 * G + NT - 1) / NT;         // float4 loads per thread and chunk
   __shared__ __attribute__((aligned(16))) _Float16 P[G * 4 * PL];
+  static_assert(KW == 1 || G * 4 * PL * 2 >= KW * 4096, "the partial sums fit the patch's memory");
   __shared__ __attribute__((aligned(16))) int opix[BM];
   __shared__ float red[NW];  // the waves' largest magnitudes
 
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wid / WN, wn = wid % WN;
+  static_assert(KW == 1 || (WM * WN * TM * TN == 1 && 16 % KW == 0), "split sums: one block per workgroup");
+  const int wk = wid % KW, wm = wid / KW / WN, wn = wid / KW % WN;
   const int half = lane >> 5, r32 = lane & 31;
   // Each XCD (workgroups L, L + 8, ...) takes a contiguous run of tiles, a
   // tile's channel blocks next to each other (they read the same patch) and
@@ -214,30 +223,34 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 || S == 2 ? 2 :
   int se = kSplitExpGuess;
   float big = 0.f;  // largest magnitude so far
 
-  for (int g = 0; g < a.ng; ++g) {
-    if (g % G == 0) {
-      if (g > 0) {
-        xload(g / G);
+  // KW waves take a group each per step (KW == G), so a chunk is one step.
+  static_assert(KW == 1 || KW == G, "a group per wave and chunk");
+  for (int gs = 0; gs < a.ng; gs += KW) {
+    if (gs % G == 0) {
+      if (gs > 0) {
+        xload(gs / G);
         __syncthreads();  // the last chunk's operand reads are done
       }
       stage(exp_float(se));
-      if (g == 0) {
+      if (gs == 0) {
 #pragma unroll
-        for (int t = 0; t < kRing; ++t) wload(0, t);
+        for (int t = 0; t < kRing; ++t) wload(wk, t);
       }
       __syncthreads();
 #pragma unroll
       for (int w = 0; w < NW; ++w) big = fmaxf(big, red[w]);
       int ne;
       if (!scale_fits(big, se, &ne)) {  // rare: the chunk again with another scale
-        if (g > 0) rescale<TM, TN>(se, ne, acc, crs);
+        if (gs > 0) rescale<TM, TN>(se, ne, acc, crs);
         se = ne;
-        xload(g / G);
+        xload(gs / G);
         __syncthreads();  // every wave has read the maxima
         stage(exp_float(se));
         __syncthreads();
       }
     }
+    const int g = gs + wk;
+    if (KW > 1 && g >= a.ng) continue;
     const _Float16* pg = P + (g % G) * (2 * PL);
     f16x8 av[2][TM][2];
     auto aload = [&](int tap) {
@@ -272,17 +285,33 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 || S == 2 ? 2 :
         for (int j = 0; j < TN; ++j)
           crs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i][0], w[j][1], crs[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      wload(tap + kRing < 9 ? g : g + 1, (tap + kRing) % 9);
+      wload(tap + kRing < 9 ? g : g + KW, (tap + kRing) % 9);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 
   const int* po = opix + wm * TM * 32;
   if (big >= kSplitHuge) {
-    c3_exact(a, po, TM * 32, col0 - r32, TN * 32, lane);
+    if (wk == 0) c3_exact(a, po, TM * 32, col0 - r32, TN * 32, lane);
     return;
   }
   unscale<TM, TN>(ws, se, acc, crs);
+  if (KW > 1) {
+    // Rows r of the sums belong to wave r KW / 16.
+    float* sums = (float*)P;
+    __syncthreads();  // the patch's reads are done
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sums[(wk * 16 + r) * 64 + lane] = acc[0][0][r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      if (r * KW / 16 != wk) continue;
+      float v = sums[r * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < KW; ++w) v += sums[(w * 16 + r) * 64 + lane];
+      acc[0][0][r] = v;
+    }
+  }
   // Buffer accesses: a pixel or channel past the output has an offset past the
   // resource, whose load gives zero and whose store is dropped.
   const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
@@ -294,7 +323,10 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 || S == 2 ? 2 :
   for (int i = 0; i < TM; ++i) {
     int px[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) px[r] = po[i * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
+    for (int r = 0; r < 16; ++r) {
+      px[r] = po[i * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
+      if (KW > 1 && r * KW / 16 != wk) px[r] = a.M;  // another wave's row
+    }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const unsigned col = col0 + j * 32 < a.OC ? 4u * (col0 + j * 32) : 0x80000000u;
@@ -319,17 +351,19 @@ __global__ __launch_bounds__(WM* WN * 64, TM * TN == 2 ? (G == 4 || S == 2 ? 2 :
   }
 }
 
-// Wave grid (pixels x channels) and 32 x 32 blocks per wave.
-#define SY_C3_LIST(X) \
-  X(0, 2, 2, 2, 1) X(1, 4, 1, 1, 1) X(2, 2, 1, 1, 1) X(3, 2, 2, 1, 1) X(4, 2, 3, 1, 1)
+// Wave grid (pixels x channels), 32 x 32 blocks per wave, waves per block.
+#define SY_C3_LIST(X)                                                                                 \
+  X(0, 2, 2, 2, 1, 1) X(1, 4, 1, 1, 1, 1) X(2, 2, 1, 1, 1, 1) X(3, 2, 2, 1, 1, 1) X(4, 2, 3, 1, 1, 1) \
+  X(5, 1, 1, 1, 1, 4) X(6, 1, 1, 1, 1, 8)
 
 struct C3Form {
-  int wm, wn, tm, tn;
+  int wm, wn, tm, tn, kw;
 };
-#define SY_C3_CFG(i, wm, wn, tm, tn) {wm, wn, tm, tn},
+#define SY_C3_CFG(i, wm, wn, tm, tn, kw) {wm, wn, tm, tn, kw},
 static const C3Form kC3Forms[] = {SY_C3_LIST(SY_C3_CFG)};
 #undef SY_C3_CFG
 static constexpr int kNumC3 = sizeof(kC3Forms) / sizeof(kC3Forms[0]);
+int c3_form_groups(int f) { return kC3Forms[f].kw; }
 int c3_num_forms() { return kNumC3; }
 
 const char* c3_name(int f) {
@@ -338,8 +372,9 @@ const char* c3_name(int f) {
     Names() {
       for (int i = 0; i < kNumC3; ++i) {
         char buf[48];
-        snprintf(buf, sizeof buf, "conv3_x3_%dx%d_%d%d", kC3Forms[i].wm * kC3Forms[i].tm * 32,
-                 kC3Forms[i].wn * kC3Forms[i].tn * 32, kC3Forms[i].wm, kC3Forms[i].wn);
+        const C3Form& c = kC3Forms[i];
+        int len = snprintf(buf, sizeof buf, "conv3_x3_%dx%d_%d%d", c.wm * c.tm * 32, c.wn * c.tn * 32, c.wm, c.wn);
+        if (c.kw > 1) snprintf(buf + len, sizeof buf - len, "_ks%d", c.kw);
         n[i] = buf;
       }
     }
@@ -388,6 +423,24 @@ bool c3_fits(const C3Args& a) {
          (long long)a.N * (a.H + 64) < (1LL << 24) && (long long)a.ng * (9 * 128 * 16 * 4) < (1LL << 31);
 }
 
+// Chunks of up to 64 channels for the wide forms at stride 1; 32 for the
+// 32-channel forms (twice the workgroups per CU: 80 -> 80 at 80 x 80, batch 32,
+// 104 against 119 us) and for stride 2 (four times the patch); a group per wave
+// where waves share a block out.
+template <int WM, int WN, int TM, int TN, int KW>
+static auto c3_pick(int stride, int ng) -> void (*)(const C3Args) {
+  if constexpr (KW > 1) {
+    return stride == 2 ? conv3_kernel<2, KW, WM, WN, TM, TN, KW> : conv3_kernel<1, KW, WM, WN, TM, TN, KW>;
+  } else {
+    if (stride == 2) return ng == 1 ? conv3_kernel<2, 1, WM, WN, TM, TN, 1> : conv3_kernel<2, 2, WM, WN, TM, TN, 1>;
+    if (ng == 1) return conv3_kernel<1, 1, WM, WN, TM, TN, 1>;
+    if constexpr (WN * TN == 1)
+      return conv3_kernel<1, 2, WM, WN, TM, TN, 1>;
+    else
+      return ng == 2 ? conv3_kernel<1, 2, WM, WN, TM, TN, 1> : conv3_kernel<1, 4, WM, WN, TM, TN, 1>;
+  }
+}
+
 int launch_c3(sy_ctx* ctx, int f, C3Args a) {
   const C3Form& c = kC3Forms[f];
   const int bm = c.wm * c.tm * 32;
@@ -400,19 +453,13 @@ int launch_c3(sy_ctx* ctx, int f, C3Args a) {
   a.inv_pw = (a.S == 1 ? 1 << 16 : 1 << 20) / c3_extent(a.TW, a.S) + 1;
   SY_CHECK(tiles * a.nblk < (1LL << 31), SY_EUNSUPPORTED, "convolution grid too large");
   void (*k)(const C3Args) = nullptr;
-  // Chunks of up to 64 channels for the wide forms at stride 1; 32 for the
-  // 32-channel forms (twice the workgroups per CU: 80 -> 80 at 80 x 80, batch 32,
-  // 104 against 119 us) and for stride 2 (four times the patch).
-#define SY_C3_CASE(i, wm, wn, tm, tn)                                                        \
-  if (f == i)                                                                                 \
-    k = a.S == 2    ? (a.ng == 1 ? conv3_kernel<2, 1, wm, wn, tm, tn> : conv3_kernel<2, 2, wm, wn, tm, tn>) \
-        : a.ng == 1 ? conv3_kernel<1, 1, wm, wn, tm, tn>                                      \
-        : a.ng == 2 || wn * tn == 1 ? conv3_kernel<1, 2, wm, wn, tm, tn>                      \
-                    : conv3_kernel<1, 4, wm, wn, tm, tn>;
+#define SY_C3_CASE(i, wm, wn, tm, tn, kw)                                                              \
+  if (f == i) k = c3_pick<wm, wn, tm, tn, kw>(a.S, a.ng);
   SY_C3_LIST(SY_C3_CASE)
 #undef SY_C3_CASE
   SY_CHECK(k != nullptr, SY_EINVAL, "no split 3x3 form %d", f);
-  hipLaunchKernelGGL(k, dim3((unsigned)(tiles * a.nblk)), dim3(c.wm * c.wn * 64), 0, ctx->stream, a);
+  hipLaunchKernelGGL(k, dim3((unsigned)(tiles * a.nblk)), dim3(c.wm * c.wn * c.kw * 64), 0,
+                     ctx->stream, a);
   return SY_OK;
 }
 

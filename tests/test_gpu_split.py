@@ -18,7 +18,14 @@ pytestmark = pytest.mark.gpu
 
 X3_BASE, C3_BASE = 64, 96
 X3_TILES = [(128, 128, 2, 2), (64, 64, 2, 2), (64, 128, 2, 2), (128, 32, 4, 1), (64, 32, 2, 1)]
-C3_FORMS = [(128, 64, 2, 2), (128, 32, 4, 1), (64, 32, 2, 1), (64, 64, 2, 2), (64, 96, 2, 3)]
+# (pixels, channels, wave grid, waves per block)
+C3_FORMS = [(128, 64, 2, 2, 1), (128, 32, 4, 1, 1), (64, 32, 2, 1, 1), (64, 64, 2, 2, 1), (64, 96, 2, 3, 1),
+            (32, 32, 1, 1, 4), (32, 32, 1, 1, 8)]
+
+
+def c3_name(form):
+    bm, bn, wm, wn, kw = C3_FORMS[form]
+    return f"conv3_x3_{bm}x{bn}_{wm}{wn}" + (f"_ks{kw}" if kw > 1 else "")
 
 
 def conv64(x, w, b, stride, silu, res):
@@ -119,7 +126,7 @@ def test_patch_forms(hip, monkeypatch, form, shape, res):
     r = synth.activations((n, oc, h, w), 8) if res else None
     exp, mag = conv64(x, wt, b, 1, True, r)
     got, names = run(hip, monkeypatch, C3_BASE + form, x, wt, b, 1, True, r)
-    assert names == {"conv3_x3_%dx%d_%d%d" % C3_FORMS[form]}
+    assert names == {c3_name(form)}
     near(got, exp, mag)
 
 
@@ -137,11 +144,11 @@ def test_patch_forms_stride_2(hip, monkeypatch, form, shape, res):
     r = synth.activations((n, oc, (h + 1) // 2, (w + 1) // 2), 9) if res else None
     exp, mag = conv64(x, wt, b, 2, True, r)
     got, names = run(hip, monkeypatch, C3_BASE + form, x, wt, b, 2, True, r)
-    assert names == {"conv3_x3_%dx%d_%d%d" % C3_FORMS[form]}
+    assert names == {c3_name(form)}
     near(got, exp, mag)
 
 
-@pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3], ids=["gemm", "patch"])
+@pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3, C3_BASE + 5], ids=["gemm", "patch", "patch_ks4"])
 @pytest.mark.parametrize("scale", [0.0, 1e-30, 1e-6, 3e4, 1e30], ids=str)
 def test_scales(hip, monkeypatch, tile, scale):
     """Magnitudes outside the first guess of the scale, the second half of the
@@ -157,7 +164,7 @@ def test_scales(hip, monkeypatch, tile, scale):
     near(got, exp, mag, 2.0 ** -38 * float(np.abs(x).max()) * np.abs(wt).sum(axis=(1, 2, 3)).max() + 1e-45)
 
 
-@pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3], ids=["gemm", "patch"])
+@pytest.mark.parametrize("tile", [X3_BASE + 1, C3_BASE + 3, C3_BASE + 5], ids=["gemm", "patch", "patch_ks4"])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38], ids=str)
 def test_non_finite_input(hip, monkeypatch, tile, value):
     """Infinities, NaN and the top of the float32 range give what float32
