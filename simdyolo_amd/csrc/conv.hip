@@ -2721,20 +2721,22 @@ static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo, int tile) {
     const size_t units = x3 ? (size_t)(ocp / 32) * nkt * kX3Units : (size_t)(ocp / 32) * ng * taps * 128;
     std::vector<float> h(units * 4 + ocp, 0.f);
     uint16_t* q = (uint16_t*)h.data();
+    std::vector<uint16_t> hi(K), lo(K);
     for (int o = 0; o < oc; ++o) {
       const float* g = W + (size_t)o * K;
       float big = 0.f;
       for (int i = 0; i < K; ++i) big = std::max(big, std::fabs(g[i]));
       const float scale = x3_weight_scale(big);
       h[units * 4 + o] = 1.f / scale;
+      x3_split(g, K, scale, hi.data(), lo.data());
       for (int c = 0; c < ic; ++c)
         for (int t = 0; t < taps; ++t) {
           const int k = x3 ? t * ic + c : c;
           const size_t unit = x3 ? ((size_t)(o >> 5) * nkt + (k >> 5)) * kX3Units + ((k >> 4) & 1) * 128
                                  : (((size_t)(o >> 5) * ng + (c >> 4)) * taps + t) * 128;
-          uint16_t part[2];
-          x3_split(g[(size_t)c * taps + t], scale, part);
-          for (int i = 0; i < 2; ++i) q[(unit + 64 * i + ((k >> 3) & 1) * 32 + (o & 31)) * 8 + (k & 7)] = part[i];
+          const size_t at = (unit + ((k >> 3) & 1) * 32 + (o & 31)) * 8 + (k & 7);
+          q[at] = hi[c * taps + t];
+          q[at + 512] = lo[c * taps + t];
         }
     }
     float* d = nullptr;
@@ -3372,15 +3374,18 @@ static int conv_tune(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tens
     rc = SY_EDEVICE;
     set_error("hipEventCreate failed");
   }
-  for (size_t i = 0; rc == SY_OK && i < cand.size(); ++i) {
-    rc = conv_exec(ctx, p, x, y, res, cand[i]);  // warm: packs weights, touches caches
-    if (rc != SY_OK) break;
-    // The better of two windows of three launches: one slow window (a clock
-    // change, another process's work) does not decide the pick.
-    constexpr int kReps = 3, kWindows = 2;
-    float ms = 1e30f;
-    for (int wdw = 0; rc == SY_OK && wdw < kWindows; ++wdw) {
-      if (hipEventRecord(e0, ctx->stream) != hipSuccess) rc = SY_EDEVICE;
+  // Rounds over all candidates, each timed over three launches and kept by its
+  // best: the clock moves with the load, so candidates next to each other in
+  // time are compared, not the first with the last.  After the first round only
+  // those within 30% of the best go on.
+  constexpr int kReps = 3, kRounds = 4;
+  std::vector<float> ms(cand.size(), 1e30f);
+  for (int round = 0; rc == SY_OK && round < kRounds; ++round) {
+    const float limit = 1.3f * best;
+    for (size_t i = 0; rc == SY_OK && i < cand.size(); ++i) {
+      if (round > 0 && ms[i] > limit) continue;
+      if (round == 0) rc = conv_exec(ctx, p, x, y, res, cand[i]);  // warm: packs weights, touches caches
+      if (rc == SY_OK && hipEventRecord(e0, ctx->stream) != hipSuccess) rc = SY_EDEVICE;
       for (int r = 0; rc == SY_OK && r < kReps; ++r) rc = conv_exec(ctx, p, x, y, res, cand[i]);
       if (rc != SY_OK) break;
       float w = 0.f;
@@ -3390,12 +3395,11 @@ static int conv_tune(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tens
         set_error("event timing failed while tuning a convolution");
         break;
       }
-      ms = std::min(ms, w);
-    }
-    if (rc != SY_OK) break;
-    if (ms < best) {
-      best = ms;
-      pick = cand[i];
+      ms[i] = std::min(ms[i], w);
+      if (ms[i] < best) {
+        best = ms[i];
+        pick = cand[i];
+      }
     }
   }
   if (e0) (void)hipEventDestroy(e0);

@@ -177,9 +177,9 @@ extern const X3Tile kX3Tiles[];
 int x3_num_tiles();
 inline bool is_x3_tile(int t) { return t >= kX3Base && t < kX3Base + x3_num_tiles(); }
 const char* x3_name(int t, int mode);
-// hi and lo of a (finite) weight times its channel's scale, within 2^-23 of it,
-// and that power of two for the channel's largest magnitude.
-void x3_split(float v, float scale, uint16_t out[2]);
+// hi and lo of n (finite) weights times their channel's scale, within 2^-23 of
+// them, and that power of two for the channel's largest magnitude.
+void x3_split(const float* v, int n, float scale, uint16_t* hi, uint16_t* lo);
 float x3_weight_scale(float largest);
 int launch_x3(sy_ctx* ctx, int t, int mode, const IgemmArgs& a);
 

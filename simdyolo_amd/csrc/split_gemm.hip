@@ -315,35 +315,33 @@ const char* x3_name(int t, int mode) {
 }
 
 // Nearest f16 (ties to even) of a float below 65520 in magnitude, and back.
-static inline uint16_t f16_bits(float v) {
-  uint32_t u;
+// Both branches are computed and one taken, so that loops vectorise.
+static inline uint32_t f16_bits(float v) {
+  uint32_t u, m;
   std::memcpy(&u, &v, 4);
   const uint32_t sign = (u >> 16) & 0x8000u;
   u &= 0x7fffffffu;
-  if (u < 0x38800000u) {  // below 2^-14: a multiple of 2^-24, rounded in the float addition
-    const float m = std::fabs(v) * 0x1p24f + 0x1p23f;
-    std::memcpy(&u, &m, 4);
-    return (uint16_t)(sign | (u & 0x7fffffu));
-  }
-  u += 0xfffu + ((u >> 13) & 1);
-  return (uint16_t)(sign | ((u - 0x38000000u) >> 13));
+  // Below 2^-14: a multiple of 2^-24, rounded in the float addition.
+  const float s = std::fabs(v) * 0x1p24f + 0x1p23f;
+  std::memcpy(&m, &s, 4);
+  const uint32_t n = (u + 0xfffu + ((u >> 13) & 1) - 0x38000000u) >> 13;
+  return sign | (u < 0x38800000u ? m & 0x7fffffu : n);
 }
-static inline float f16_value(uint16_t h) {
-  uint32_t u = h & 0x7fffu;
+static inline float f16_value(uint32_t h) {
+  const uint32_t u = h & 0x7fffu, n = (u << 13) + 0x38000000u;
   float v;
-  if (u < 0x400u) {
-    v = (float)u * 0x1p-24f;
-  } else {
-    u = (u << 13) + 0x38000000u;
-    std::memcpy(&v, &u, 4);
-  }
+  std::memcpy(&v, &n, 4);
+  v = u < 0x400u ? (float)(int)u * 0x1p-24f : v;
   return h & 0x8000u ? -v : v;
 }
 
-void x3_split(float v, float scale, uint16_t out[2]) {
-  const float s = v * scale;
-  out[0] = f16_bits(s);
-  out[1] = f16_bits((s - f16_value(out[0])) * 2048.f);
+void x3_split(const float* v, int n, float scale, uint16_t* hi, uint16_t* lo) {
+  for (int i = 0; i < n; ++i) {
+    const float s = v[i] * scale;
+    const uint32_t h = f16_bits(s);
+    hi[i] = (uint16_t)h;
+    lo[i] = (uint16_t)f16_bits((s - f16_value(h)) * 2048.f);
+  }
 }
 
 float x3_weight_scale(float largest) {
