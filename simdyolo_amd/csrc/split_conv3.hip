@@ -15,7 +15,7 @@
 // channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
 // MFMAs of 32 cycles.
 //
-// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 52 us,
+// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 51 us,
 // against 73 us for the fastest float32 Winograd form.  The matrix cores are
 // busy for 46% of it at the 1.8 GHz the GPU holds under this load; the patch
 // loads (8,000 of a 128-pixel workgroup's 29,000 cycles), the epilogue (6,000)
@@ -27,7 +27,7 @@
 // at 20 x 20 from 9.3 to 6.0, 256 -> 64 at 20 x 20 from 15.5 to 8.1.
 // Stride 2, batch 32, against the implicit GEMM of split_gemm.hip, which stages
 // every input per tap: 64 -> 128 at 80 x 80 42 -> 38 us, 32 -> 64 at 160 x 160
-// 49 -> 41, 16 -> 32 at 320 x 320 88 -> 75 (315 MB), 128 -> 128 at 40 x 40 33 -> 22.
+// 49 -> 41, 16 -> 32 at 320 x 320 88 -> 70 (315 MB), 128 -> 128 at 40 x 40 33 -> 22.
 //
 // LDS holds the patch as planes of 8 channels, [split][8-channel block][pixel]
 // [8].  ds_read_b128 serves 16 lanes a cycle over 64 banks, lanes 0-3, 12-15,
@@ -95,8 +95,19 @@ __device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int p
 // outputs are neighbours at every tap.  KW > 1: the tile's channel groups shared
 // out over KW waves (small grids: a fourth or an eighth of the chain of taps),
 // their sums joined through LDS, each wave finishing 16 / KW of the rows.
-template <int S, int G, int WM, int WN, int TM, int TN, int KW>
-__global__ __launch_bounds__(WM* WN* KW * 64, KW > 1 ? 2 : TM * TN == 2 ? (G == 4 || S == 2 ? 2 : 3) : (G == 4 || S == 2) && WM * WN == 2 ? 2 : S == 2 ? 3 : 4) void conv3_kernel(
+// ONE: all channels fit one chunk, whose staging registers are free again before
+// the sums exist.
+// Waves per SIMD the registers are allocated for (each measured without spills
+// that matter).
+constexpr int c3_waves(int s, int g, int nw, int blocks, int kw, bool one) {
+  if (kw > 1) return 2;
+  if (one) return blocks == 2 ? (s == 2 ? 2 : 3) : (s == 2 ? 3 : 4);
+  if (blocks == 2) return g == 4 || s == 2 ? 2 : 3;
+  return (g == 4 || s == 2) && nw == 2 ? 2 : s == 2 ? 3 : 4;
+}
+
+template <int S, int G, int WM, int WN, int TM, int TN, int KW, bool ONE>
+__global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, KW, ONE)) void conv3_kernel(
     const C3Args a) {
   constexpr int NW = WM * WN * KW, NT = NW * 64, BM = WM * TM * 32, NPX = c3_patch(BM, S);
   constexpr int PL = (NPX * 8 + 127) / 128 * 128 + 64 / G;  // halves per plane
@@ -136,7 +147,7 @@ __global__ __launch_bounds__(WM* WN* KW * 64, KW > 1 ? 2 : TM * TN == 2 ? (G == 
   // reciprocal is exact.
   auto patch_row = [&](int px) { return mul24(px, a.inv_pw) >> (S == 1 ? 16 : 20); };
   f32x4 d[L_IT];
-  auto xload = [&](int ch) {
+  auto xload = [&](int ch) __attribute__((always_inline)) {
     const bool cok = ch * (16 * G) + 4 * q4 < a.IC;
 #pragma unroll
     for (int i = 0; i < L_IT; ++i) {
@@ -150,7 +161,7 @@ __global__ __launch_bounds__(WM* WN* KW * 64, KW > 1 ? 2 : TM * TN == 2 ? (G == 
       d[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, ch * (64 * G), 0));
     }
   };
-  auto stage = [&](float s) {
+  auto stage = [&](float s) __attribute__((always_inline)) {
     float m = 0.f;
 #pragma unroll
     for (int i = 0; i < L_IT; ++i) {
@@ -181,7 +192,7 @@ __global__ __launch_bounds__(WM* WN* KW * 64, KW > 1 ? 2 : TM * TN == 2 ? (G == 
   const int wob = a.ng * (9 * 128 * 16);  // bytes per 32-channel block
   const char* wbase = (const char*)a.w + (long long)ob0 * wob;
   const unsigned wlane = lane * 16;
-  auto wload = [&](int g, int tap) {
+  auto wload = [&](int g, int tap) __attribute__((always_inline)) {
     const char* wg = wbase + min(g, a.ng - 1) * (9 * 128 * 16);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -213,41 +224,49 @@ __global__ __launch_bounds__(WM* WN* KW * 64, KW > 1 ? 2 : TM * TN == 2 ? (G == 
     const int p = (wm * TM + i) * 32 + c3_row(r32), py = mul24(p, a.inv_tw) >> 16;
     arow[i] = (S * mul24(min(py, a.TH - 1), PW) + p - mul24(py, a.TW)) * 8 + half * PL;
   }
-  f32x16 acc[TM][TN], crs[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = crs[i][j][r] = 0.f;
   int se = kSplitExpGuess;
   float big = 0.f;  // largest magnitude so far
+  f32x16 acc[TM][TN], crs[TM][TN];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = crs[i][j][r] = 0.f;
+  };
+  // Chunk ch (loaded already) into LDS.
+  auto enter = [&](int ch) __attribute__((always_inline)) {
+    stage(exp_float(se));
+    if (ch == 0) {
+#pragma unroll
+      for (int t = 0; t < kRing; ++t) wload(wk, t);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) big = fmaxf(big, red[w]);
+    int ne;
+    if (!scale_fits(big, se, &ne)) {  // rare: the chunk again with another scale
+      if (!ONE && ch > 0) rescale<TM, TN>(se, ne, acc, crs);
+      se = ne;
+      xload(ch);
+      __syncthreads();  // every wave has read the maxima
+      stage(exp_float(se));
+      __syncthreads();
+    }
+  };
+  if (ONE) enter(0);
+  clear();
 
   // KW waves take a group each per step (KW == G), so a chunk is one step.
   static_assert(KW == 1 || KW == G, "a group per wave and chunk");
   for (int gs = 0; gs < a.ng; gs += KW) {
-    if (gs % G == 0) {
+    if (!ONE && gs % G == 0) {
       if (gs > 0) {
         xload(gs / G);
         __syncthreads();  // the last chunk's operand reads are done
       }
-      stage(exp_float(se));
-      if (gs == 0) {
-#pragma unroll
-        for (int t = 0; t < kRing; ++t) wload(wk, t);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int w = 0; w < NW; ++w) big = fmaxf(big, red[w]);
-      int ne;
-      if (!scale_fits(big, se, &ne)) {  // rare: the chunk again with another scale
-        if (gs > 0) rescale<TM, TN>(se, ne, acc, crs);
-        se = ne;
-        xload(gs / G);
-        __syncthreads();  // every wave has read the maxima
-        stage(exp_float(se));
-        __syncthreads();
-      }
+      enter(gs / G);
     }
     const int g = gs + wk;
     if (KW > 1 && g >= a.ng) continue;
@@ -430,14 +449,18 @@ bool c3_fits(const C3Args& a) {
 template <int WM, int WN, int TM, int TN, int KW>
 static auto c3_pick(int stride, int ng) -> void (*)(const C3Args) {
   if constexpr (KW > 1) {
-    return stride == 2 ? conv3_kernel<2, KW, WM, WN, TM, TN, KW> : conv3_kernel<1, KW, WM, WN, TM, TN, KW>;
+    return stride == 2 ? conv3_kernel<2, KW, WM, WN, TM, TN, KW, false> : conv3_kernel<1, KW, WM, WN, TM, TN, KW, false>;
   } else {
-    if (stride == 2) return ng == 1 ? conv3_kernel<2, 1, WM, WN, TM, TN, 1> : conv3_kernel<2, 2, WM, WN, TM, TN, 1>;
-    if (ng == 1) return conv3_kernel<1, 1, WM, WN, TM, TN, 1>;
+    if (stride == 2)
+      return ng == 1   ? conv3_kernel<2, 1, WM, WN, TM, TN, 1, true>
+             : ng == 2 ? conv3_kernel<2, 2, WM, WN, TM, TN, 1, true>
+                       : conv3_kernel<2, 2, WM, WN, TM, TN, 1, false>;
+    if (ng == 1) return conv3_kernel<1, 1, WM, WN, TM, TN, 1, true>;
+    if (ng == 2) return conv3_kernel<1, 2, WM, WN, TM, TN, 1, true>;
     if constexpr (WN * TN == 1)
-      return conv3_kernel<1, 2, WM, WN, TM, TN, 1>;
+      return conv3_kernel<1, 2, WM, WN, TM, TN, 1, false>;
     else
-      return ng == 2 ? conv3_kernel<1, 2, WM, WN, TM, TN, 1> : conv3_kernel<1, 4, WM, WN, TM, TN, 1>;
+      return ng <= 4 ? conv3_kernel<1, 4, WM, WN, TM, TN, 1, true> : conv3_kernel<1, 4, WM, WN, TM, TN, 1, false>;
   }
 }
 
