@@ -5,11 +5,11 @@
 // tap; here a workgroup stages the input patch of its output tile (TH x TW
 // outputs, (TH + 2) x (TW + 2) inputs at stride 1, (2 TH + 1) x (2 TW + 1) at
 // stride 2) once, up to 64 channels at a time, and the nine taps read it at
-// shifted pixels.  All of a chunk's loads are issued
-// together: 16 channels at a time left too few bytes in flight, and every
-// wait for weights behind them (loads return in order) cost a memory latency.  Weights stream from L2 straight into MFMA
-// operands: their packed order makes each read of a wave 1 KiB contiguous, and
-// the workgroup's waves read the same ones.
+// shifted pixels.  All of a chunk's loads are issued together: 16 channels at a
+// time left too few bytes in flight, and every wait for weights behind them
+// (loads return in order) cost a memory latency.  Weights stream from L2
+// straight into MFMA operands: their packed order makes each read of a wave
+// 1 KiB contiguous, and the workgroup's waves read the same ones.
 //
 // A wave owns TM 32-pixel blocks x TN 32-channel blocks.  Per (tap, 16
 // channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
@@ -90,13 +90,6 @@ __device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int p
   }
 }
 
-// S: stride.  G: 16-channel groups per chunk.  At stride 2 a patch row holds its
-// even columns, then the odd ones, so that the operand reads of neighbouring
-// outputs are neighbours at every tap.  KW > 1: the tile's channel groups shared
-// out over KW waves (small grids: a fourth or an eighth of the chain of taps),
-// their sums joined through LDS, each wave finishing 16 / KW of the rows.
-// ONE: all channels fit one chunk, whose staging registers are free again before
-// the sums exist.
 // Waves per SIMD the registers are allocated for (each measured without spills
 // that matter).
 constexpr int c3_waves(int s, int g, int nw, int blocks, int kw, bool one) {
@@ -106,6 +99,13 @@ constexpr int c3_waves(int s, int g, int nw, int blocks, int kw, bool one) {
   return (g == 4 || s == 2) && nw == 2 ? 2 : s == 2 ? 3 : 4;
 }
 
+// S: stride.  G: 16-channel groups per chunk.  At stride 2 a patch row holds its
+// even columns, then the odd ones, so that the operand reads of neighbouring
+// outputs are neighbours at every tap.  KW > 1: the tile's channel groups shared
+// out over KW waves (small grids: a fourth or an eighth of the chain of taps),
+// their sums joined through LDS, each wave finishing 16 / KW of the rows.
+// ONE: all channels fit one chunk, whose staging registers are free again before
+// the sums exist.
 template <int S, int G, int WM, int WN, int TM, int TN, int KW, bool ONE>
 __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, KW, ONE)) void conv3_kernel(
     const C3Args a) {
