@@ -28,7 +28,7 @@ struct AttnArgs {
 };
 
 // Rows of the workgroup's queries in plain float32, one wave per query: what a
-// workgroup does that met a non-finite or huge operand (kSplitHuge).
+// workgroup does that met a non-finite or huge operand (kSplitHuge) or scale.
 __device__ __forceinline__ void attn_exact(const AttnArgs& a, const float* base, float* ob, int q0, int queries,
                                            int wave, int lane) {
   for (int q = wave; q < queries; q += 4) {
@@ -60,6 +60,17 @@ __device__ __forceinline__ void attn_exact(const AttnArgs& a, const float* base,
   }
 }
 
+// e^x for x up to a few units: 2^t of the hardware at t = x log2(e) rounded, times 1 plus the
+// first-order term of t's exact rounding error and of log2(e)'s.  Below -150,
+// where the result is under every float, 0; NaN stays.
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float kLog2e = 1.4426950408889634f, kLog2eLow = (float)(1.4426950408889634 - (double)kLog2e);
+  x = x < -150.f ? -150.f : x;
+  const float t = x * kLog2e, r = __builtin_fmaf(x, kLog2eLow, __builtin_fmaf(x, kLog2e, -t));
+  const float p = __builtin_amdgcn_exp2f(t);
+  return __builtin_fmaf(p, r * 0.69314718f, p);
+}
+
 // 32 queries of one head and image per workgroup.  Wave w takes the 32-key
 // tiles w, w + 4, ... with a running maximum, sum and output of its own; the
 // four are joined through LDS at the end.  Nothing else is shared: operands go
@@ -74,12 +85,18 @@ __device__ __forceinline__ void attn_exact(const AttnArgs& a, const float* base,
 // Both products are f16 splits (split_gemm.hip): queries, each key tile and the
 // values under scales from their largest magnitudes, probabilities under 2^11.
 //
-// Bound by VALU work (splitting K, V and P, the exponentials: about 750
+// The running maximum moves (and the sums with it) only where a score passes it
+// by kSlack: until then weights reach e^kSlack, and under 2^11 still fit f16.
+//
+// Bound by VALU work (splitting K, V and P, the exponentials: about 650
 // operations beside 18 MFMAs per tile) and, at 400 tokens, by the latency of its
 // few tiles.  Measured against two GEMMs, a softmax and a copy with the scores
-// in memory, us: 2 heads, 400 tokens, batch 16 74 -> 24, batch 1 25 -> 16;
-// 4 heads, 1,600 tokens, batch 8 858 -> 184.  64 queries per workgroup, which
-// would split each key tile for twice the work, spill registers: 214.
+// in memory, us: 2 heads, 400 tokens, batch 16 74 -> 23, batch 1 25 -> 14.6;
+// 4 heads, 1,600 tokens, batch 8 858 -> 156.  With expf, a maximum that moves in
+// every tile and per-lane row addresses these were 24.5, 15.5 and 184.  64
+// queries per workgroup, which would split each key tile for twice the work,
+// spill registers: 214.
+constexpr float kSlack = 2.5f;  // e^2.5 2^11 < 2^15
 __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
   constexpr int TQ = 1, NQ = 32 * TQ;  // 32-query blocks, queries
   __shared__ float O[4][NQ][65];
@@ -113,6 +130,44 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
     lo = __builtin_bit_cast(f16x8, u32x4{l0[0], l0[1], l1[0], l1[1]});
   };
 
+  // A tile's keys and values.  In a whole tile the rows' addresses are scalar, with
+  // one offset per lane; past the last key both read the last key's row.
+  f32x4 k[2][2];
+  float v[2][16];
+  const int krow = r32 * a.ldq + a.kd + 8 * half;
+  const int vrow = 4 * half * a.ldq + 2 * a.kd, vcol[2] = {min(r32, a.hd - 1), min(32 + r32, a.hd - 1)};
+  auto load = [&](int j0) __attribute__((always_inline)) {
+    if (j0 + 32 <= a.N) {
+      const float* tb = base + j0 * a.ldq;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int c = 16 * ks + 8 * half + 4 * i;
+          k[ks][i] = c < a.kd ? *(const f32x4*)(tb + (krow + 16 * ks + 4 * i)) : zero;
+        }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float* vr = tb + (16 * (e >> 3) + 8 * ((e >> 2) & 1) + (e & 3)) * a.ldq;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) v[d][e] = vr[(unsigned)(vrow + vcol[d])];
+      }
+      return;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) k[ks][i] = row4(j0 + r32, a.kd, ks, i);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int j = min(j0 + 16 * (e >> 3) + 8 * ((e >> 2) & 1) + 4 * half + (e & 3), a.N - 1);
+      const float* vr = base + j * a.ldq + 2 * a.kd;
+#pragma unroll
+      for (int d = 0; d < 2; ++d) v[d][e] = vr[vcol[d]];
+    }
+  };
+  const int tiles = (a.N + 31) / 32;
+
   f16x8 qh[TQ][2], ql[TQ][2];
   float huge = 0.f;
   int sq;
@@ -128,6 +183,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
           q[t][ks][i] = row4(q0 + 32 * t + r32, 0, ks, i);
           m = max4(m, q[t][ks][i]);
         }
+    load(min(wave, tiles - 1) * 32);
     m = readlane63(wave_max63(m));
     huge = m;
     sq = scale_exp(m);
@@ -153,24 +209,6 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
   int sv = kSplitExpGuess;
   float vbig = 0.f;
 
-  // A tile's keys and values; past the last key both read the last key's row.
-  f32x4 k[2][2];
-  float v[2][16];
-  auto load = [&](int j0) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) k[ks][i] = row4(j0 + r32, a.kd, ks, i);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int j = min(j0 + 16 * (e >> 3) + 8 * ((e >> 2) & 1) + 4 * half + (e & 3), a.N - 1);
-      const float* vr = base + j * a.ldq + 2 * a.kd;
-#pragma unroll
-      for (int d = 0; d < 2; ++d) v[d][e] = vr[min(32 * d + r32, a.hd - 1)];
-    }
-  };
-  const int tiles = (a.N + 31) / 32;
-  load(min(wave, tiles - 1) * 32);
   for (int kt = wave; kt < tiles; kt += 4) {
     const int j0 = kt * 32;
     float km = 0.f, vm = 0.f;
@@ -205,7 +243,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
     load(min(kt + 4, tiles - 1) * 32);  // the next tile (the last loads its own again)
 
     // 2^-(sq + sk) in two factors: their sum may pass the exponent range.
-    const float us = exp_float(254 - sq), uk = exp_float(254 - sk);
+    const float us = exp_float(254 - sq), uk = exp_float(254 - sk) * a.scale;
 #pragma unroll
     for (int t = 0; t < TQ; ++t) {
       f32x16 s, c;
@@ -217,36 +255,44 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
         s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks], qh[t][ks], s, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks], ql[t][ks], c, 0, 0, 0);
       }
-      float mx = mrun[t];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = j0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        s[r] = key < a.N ? __builtin_fmaf(c[r], 1.f / 2048, s[r]) * us * uk * a.scale : -INFINITY;
-        mx = fmaxf(mx, s[r]);
+      for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(c[r], 1.f / 2048, s[r]) * us * uk;
+      if (j0 + 32 > a.N) {
+        asm volatile("");  // a branch, not 16 selects in every tile
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (j0 + 8 * (r >> 2) + 4 * half + (r & 3) >= a.N) s[r] = -INFINITY;
       }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32));
-      // A maximum of -infinity: no weight yet, nothing to rescale.
-      const float alpha = mrun[t] == -INFINITY ? 0.f : expf(mrun[t] - mx);
-      mrun[t] = mx;
+      if (__any(mx > mrun[t] + kSlack)) {
+        mx = fmaxf(mx, mrun[t]);
+        const float f = exp_neg(mrun[t] - (mx == -INFINITY ? 0.f : mx));
+        mrun[t] = mx;
+        lrun[t] *= f;
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            acc[d][t][r] *= f;
+            crs[d][t][r] *= f;
+          }
+      }
+      const float from = mrun[t] == -INFINITY ? 0.f : mrun[t];  // no weight yet: all are 0
       float sum = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s[r] = s[r] == -INFINITY ? 0.f : expf(s[r] - mx);
+        s[r] = exp_neg(s[r] - from);
         sum += s[r];
       }
-      lrun[t] = __builtin_fmaf(lrun[t], alpha, sum);
+      lrun[t] += sum;
       f16x8 ph[2], pl[2];
 #pragma unroll
       for (int st = 0; st < 2; ++st)
         split8(f32x4{s[8 * st], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3]},
                f32x4{s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]}, 2048.f, ph[st], pl[st]);
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          acc[d][t][r] *= alpha;
-          crs[d][t][r] *= alpha;
-        }
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
@@ -273,7 +319,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
         O[wave][32 * t + r32][32 * d + 8 * (r >> 2) + 4 * half + (r & 3)] =
             __builtin_fmaf(crs[d][t][r], 1.f / 2048, acc[d][t][r]) * uv;
   }
-  if (lane == 0) wild[wave] = huge >= kSplitHuge;
+  // A scale past 2^20 might overflow its product with a key tile's factor.
+  if (lane == 0) wild[wave] = huge >= kSplitHuge || !(__builtin_fabsf(a.scale) <= 0x1p20f);
   // v of these rows, dense, for the positional conv: thread (row q, dim lane).
   float vd[NQ / 4];
 #pragma unroll

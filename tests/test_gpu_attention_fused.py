@@ -83,6 +83,32 @@ def test_operand_scales(hip, scales):
     assert (np.abs(got - exp) <= bound + floor).all()
 
 
+@pytest.mark.parametrize("step", [0.5, 2.0, 3.0, 60.0, -2.0])
+def test_creeping_maximum(hip, step):
+    """Scores that rise by `step` from one 32-key tile to the next: below, at about and far past the slack within
+    which a running maximum stays."""
+    heads, kd, hd = 1, 32, 64
+    qkv = synth.activations((1, 2 * kd + hd, 20, 24), 8)
+    qkv[:, :kd] = np.float32(1.0)
+    qkv[:, kd:2 * kd] *= np.float32(0.25)
+    qkv[:, kd] += (np.float32(step) * (np.arange(480) // 32)).reshape(20, 24).astype(np.float32)
+    exp, bound, _ = reference(qkv, heads, kd, hd, np.float32(1.0))
+    got, _, _ = run(hip, qkv, heads, kd, hd, np.float32(1.0))
+    assert (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
+
+
+@pytest.mark.parametrize("power", [20, 21, 60])
+def test_large_scale(hip, power):
+    """Past 2^20 the rows are computed in plain float32 (32 products: below the bound of the split)."""
+    heads, kd, hd = 2, 32, 64
+    qkv = synth.activations((1, heads, 2 * kd + hd, 5, 9), 9)
+    qkv[:, :, :kd] *= np.float32(2.0 ** -power)
+    qkv = qkv.reshape(1, -1, 5, 9)
+    exp, bound, _ = reference(qkv, heads, kd, hd, np.float32(2.0 ** power))
+    got, _, _ = run(hip, qkv, heads, kd, hd, np.float32(2.0 ** power))
+    assert (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
+
+
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan], ids=str)
 @pytest.mark.parametrize("part", ["q", "k", "v"])
 def test_non_finite(hip, part, value):
