@@ -29,7 +29,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-from bench import PEAK_FP32_MFMA_TFLOPS, PEAK_HBM_GBS, RIDGE  # noqa: E402
+from bench import PEAK_FP32_MFMA_TFLOPS, PEAK_HBM_GBS, matrix_peak  # noqa: E402
 
 
 def out(msg=""):
@@ -57,19 +57,20 @@ def kernels(ctx, fn, reps=3):
     return {k: (c // reps, 1e3 * ms / c, fl / c, by / c) for k, (c, ms, fl, by) in prof.items()}
 
 
-def roof(flops, nbytes, us):
+def roof(flops, nbytes, us, name=""):
     if us <= 0:
         return "-"
-    if flops > 0 and flops / max(nbytes, 1.0) > RIDGE:
+    peak = matrix_peak(name)
+    if flops > 0 and flops / max(nbytes, 1.0) > peak * 1e12 / (PEAK_HBM_GBS * 1e9):
         a = flops / (us * 1e-6) / 1e12
-        return f"{a:7.1f} TFLOP/s {100 * a / PEAK_FP32_MFMA_TFLOPS:5.1f}% mfma"
+        return f"{a:7.1f} TFLOP/s {100 * a / peak:5.1f}% mfma"
     a = nbytes / (us * 1e-6) / 1e9
     return f"{a:7.0f} GB/s    {100 * a / PEAK_HBM_GBS:5.1f}% hbm "
 
 
 def kernel_lines(prof, indent="    "):
     for k, (n, us, fl, by) in sorted(prof.items(), key=lambda kv: -kv[1][0] * kv[1][1]):
-        out(f"{indent}{k:<26} x{n:<3} {us:9.1f} us  {fl / 1e9:8.3f} GF {by / 1e6:9.2f} MB  {roof(fl, by, us)}")
+        out(f"{indent}{k:<26} x{n:<3} {us:9.1f} us  {fl / 1e9:8.3f} GF {by / 1e6:9.2f} MB  {roof(fl, by, us, k)}")
 
 
 # ------------------------------------------------------------------ layers
@@ -158,7 +159,7 @@ def model_line(hip, name, cfg, batch, size, steps):
         tot = sum(n * us for n, us, _, _ in prof.values())
         out(f"    eager kernel sum {tot / 1e3:.3f} ms; kernels by share:")
         for k, (n, us, fl, by) in sorted(prof.items(), key=lambda kv: -kv[1][0] * kv[1][1])[:10]:
-            out(f"    {k:<26} x{n:<3} {100 * n * us / tot:5.1f}%  avg {us:8.1f} us  {roof(fl, by, us)}")
+            out(f"    {k:<26} x{n:<3} {100 * n * us / tot:5.1f}%  avg {us:8.1f} us  {roof(fl, by, us, k)}")
     finally:
         det.close()
 
@@ -220,7 +221,7 @@ def section_route():
             out(f"    eager kernel sum {tot:.3f} ms; by kernel:")
             for k, (n, ms_, fl, by) in sorted(prof.items(), key=lambda kv: -kv[1][1])[:8]:
                 us = 1e3 * ms_ / n
-                out(f"    {k:<30} x{n:<4} {100 * ms_ / tot:5.1f}%  avg {us:8.1f} us  {roof(fl / n, by / n, us)}")
+                out(f"    {k:<30} x{n:<4} {100 * ms_ / tot:5.1f}%  avg {us:8.1f} us  {roof(fl / n, by / n, us, k)}")
         with DeviceRouteDetector(cfg, params) as det:
             for _ in range(2):
                 det.predict_raw(x)
@@ -691,7 +692,7 @@ def summarize_pmc_mfma(mfma_csv, bench_log):
             ag = a[1] / 1e9
             tf = ag / a_us * 1e3  # GFLOP per microsecond -> TFLOP/s
             out(f"{a[0]:<40} {n:8d} {ex:11.3f} {ag:8.3f} {ex / ag:5.2f} {a_us:9.2f} {busy_f:9.3f} {sq_f:7.2f} "
-                f"{tf:8.1f} {tf / PEAK_FP32_MFMA_TFLOPS:6.3f}")
+                f"{tf:8.1f} {tf / matrix_peak(a[0]):6.3f}")
         else:
             out(f"{_label(sym):<40} {n:8d} {ex:11.3f} {'-':>8} {'-':>5} {a_us:9.2f} {busy_f:9.3f} {sq_f:7.2f} "
                 f"{'-':>8} {'-':>6}")
