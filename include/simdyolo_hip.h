@@ -128,9 +128,11 @@ int sy_memcpy(sy_ctx* ctx, void* dst, const void* src, size_t bytes, int kind);
  * mirrors DeviceConv (src/SimdYolo/VulkanExecution.cs:337-350): depthwise;
  * low-channel stem -> direct; constant 3x3 s1 p1 d1 g1 with ic >= 16 ->
  * Winograd; else implicit GEMM.  On the first run of each input shape an
- * auto-routed conv times its candidates (implicit GEMM tiles, the
- * weight-stationary row kernel for 1x1 and Winograd planes, the 16-channel
- * 3x3 kernel, the three Winograd forms) with HIP events and keeps the fastest,
+ * auto-routed conv times its candidates (the f16-split implicit GEMM and 3x3
+ * patch kernels, float32 implicit GEMM tiles, the weight-stationary row kernel
+ * for 1x1 and Winograd planes, the 16-channel 3x3 kernel, the three Winograd
+ * forms; of these only the split kernels where they always win) with HIP
+ * events and keeps the fastest,
  * as the Vulkan backend's timestamp autotune does (VulkanWinograd.cs:83-117);
  * SIMDYOLO_HIP_AUTOTUNE=0 keeps the routing rule.  SIMDYOLO_HIP_WINOGRAD=0
  * disables Winograd (as SIMDYOLO_WINOGRAD does for Vulkan,
@@ -153,7 +155,8 @@ int sy_conv_transpose2x2_create(sy_ctx* ctx, const float* weight_iohw, const flo
                                 uint64_t* conv);
 /* Force an algorithm (SY_CONV_*); SY_EUNSUPPORTED when it cannot run this conv.
  * With a forced algorithm, SIMDYOLO_HIP_TILE=n also forces its n-th form: the
- * implicit-GEMM tile (or row-kernel width), the two-kernel Winograd's wave
+ * implicit-GEMM tile (from 64 the f16-split GEMM's, from 96 the 3x3 patch
+ * kernel's forms; or row-kernel width), the two-kernel Winograd's wave
  * layout (0 four waves, 1 eight), or the fused Winograd's form (0 four waves,
  * 1 warp-specialized, 2 two groups over 64 output channels). */
 int sy_conv_set_algo(sy_ctx* ctx, uint64_t conv, int algo);

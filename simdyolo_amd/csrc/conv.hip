@@ -1,4 +1,6 @@
-// Convolution: weight preparation, algorithm routing and the gfx950 kernels.
+// Convolution: weight preparation, algorithm routing and the gfx950 kernels,
+// but for the two that multiply float32 as f16 pairs, which most layers run:
+// split_gemm.hip (implicit GEMM) and split_conv3.hip (3x3 from an LDS patch).
 //
 //  * implicit GEMM on FP32 MFMA (v_mfma_f32_32x32x2f32): M = output pixels
 //    (NHWC rows), N = output channels, K = (ky, kx, ic).  A rows are gathered
