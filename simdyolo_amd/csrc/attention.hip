@@ -87,6 +87,8 @@ __device__ __forceinline__ float exp_neg(float x) {
 //
 // The running maximum moves (and the sums with it) only where a score passes it
 // by kSlack: until then weights reach e^kSlack, and under 2^11 still fit f16.
+// The test is on the difference, which is exact between floats this near: the
+// sum of maximum and slack rounds, from 2^23 on to more than the slack.
 //
 // Bound by VALU work (splitting K, V and P, the exponentials: about 650
 // operations beside 18 MFMAs per tile) and, at 400 tokens, by the latency of its
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32));
-      if (__any(mx > mrun[t] + kSlack)) {
+      if (__any(mx - mrun[t] > kSlack)) {
         mx = fmaxf(mx, mrun[t]);
         const float f = exp_neg(mrun[t] - (mx == -INFINITY ? 0.f : mx));
         mrun[t] = mx;

@@ -131,3 +131,25 @@ def test_wider_dims_keep_the_gemms(hip):
     assert "attn_softmax" in names
     np.testing.assert_array_equal(v, vexp.astype(np.float32))
     assert (np.abs(got - exp) <= bound).all()
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("step", [4.0, -4.0, 8.0])
+def test_large_scores(hip, sign, step):
+    """Scores of 2^25 magnitude, where floats lie 4 apart, in key tiles 0 and 4 (the same wave's): the step between
+    the tiles is larger than the slack of the running maximum, but not than the rounding of maximum plus slack."""
+    heads, kd, hd = 1, 32, 64
+    qkv = synth.activations((1, 2 * kd + hd, 8, 20), 10)
+    qkv[:, :kd] = np.float32(sign * 1024)
+    qkv[:, kd:2 * kd] = np.float32(1024)
+    late = (np.arange(160) >= 128).reshape(8, 20)
+    qkv[:, kd, late] += np.float32(sign * step / 1024)
+    got, _, _ = run(hip, qkv, heads, kd, hd, np.float32(1.0))
+    # Every product and sum of these scores is a float32: no error but the exponentials' and the weighted sum's.
+    t = qkv.astype(np.float64).reshape(2 * kd + hd, 160)
+    s = t[:kd].T @ t[kd:2 * kd]
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    exp, mag = t[2 * kd:] @ p.T, np.abs(t[2 * kd:]) @ p.T
+    err = np.abs(got.reshape(hd, 160) - exp)
+    assert np.isfinite(got).all() and (err <= 2.0 ** -18 * mag).all(), (err / mag).max()
