@@ -25,13 +25,41 @@ __device__ __forceinline__ void split4(const f32x4 v, float s, u32x2& hi, u32x2&
   }
 }
 
-// A workgroup that reads kSplitHuge or more (or infinity) uses plain float32.
-constexpr float kSplitHuge = 0x1p100f;
+// A workgroup that reads kSplitHuge or more (or infinity) multiplies in plain
+// float32: below it an element's error is at most 2^-32, however large its
+// neighbours are (networks that also run in f16 stay below 65,504 anyway).
+constexpr float kSplitHuge = 0x1p16f;
 // Exponent fields of the activations' power-of-two scale: its first guess
-// (largest values from 2^-2 to below 2^11 need no other) and its cap (the
-// inverse stays normal).
-constexpr int kSplitExpGuess = 127 + 4, kSplitExpMax = 250;
+// (largest values from 2^-2 to below 2^11 need no other) and its cap (every
+// normal float is 2^-13 or more under it).
+constexpr int kSplitExpGuess = 127 + 4, kSplitExpMax = 127 + 113;
+// Set in one of the bits of the top four exponent bits of an f16 (two packed)
+// of 2^-13 or more: its pair is within 2^-23 of the value.
+constexpr unsigned kSplitFull = 0x78007800u;
 __device__ __forceinline__ float exp_float(int e) { return __builtin_bit_cast(float, (unsigned)e << 23); }
+
+// v or'ed over aligned groups of 8 lanes.
+__device__ __forceinline__ unsigned or8(unsigned v) {
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false);          // lane ^ 1
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false);          // lane ^ 2
+  return v | (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false);  // 7 - lane
+}
+
+// Four elements' bits, without their signs.
+__device__ __forceinline__ unsigned magnitude_bits(const f32x4 v) {
+  const u32x4 b = __builtin_bit_cast(u32x4, v);
+  return (b[0] | b[1] | b[2] | b[3]) & 0x7fffffffu;
+}
+
+// Four weights from their pair (hi at w, lo 512 halves on) and inverse scale.
+__device__ __forceinline__ f32x4 join4(const _Float16* w, float ws) {
+  typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+  const f16x4 hi = *(const f16x4*)w, lo = *(const f16x4*)(w + 512);
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf((float)lo[e], 1.f / 2048, (float)hi[e]) * ws;
+  return v;
+}
 
 // One step of a wave reduction: m and the m that DPP control ctrl moves here.
 template <int ctrl, int rows>

@@ -5,17 +5,24 @@
 // and lo keeps 11 more significand bits, so the pair is within 2^-23 of v.  A
 // product is three f16 products, each exact in the float32 accumulators:
 // hi hi in one, hi lo + lo hi (2048 times too large) in the other.  The lo lo
-// left out is below 2^-22 of it, with either sign.  Against float64 the
-// result is closer than the float32 MFMA's, whose accumulator rounds once per
-// two terms: the main one here rounds once per sixteen.
+// left out is below 2^-22 of it, with either sign.  Where every operand has its
+// pair in full the result is closer to float64 than the float32 MFMA's, whose
+// accumulator rounds once per two terms: the main one here rounds once per
+// sixteen.
 //
 // Scales.  Weights: one power of two per output channel, chosen when they are
 // packed.  Activations: one per workgroup, from the largest magnitude of the
 // K tiles seen so far: 2^2 <= largest < 2^15 after scaling, so f16 does not
-// overflow, and the pair's absolute error is at most 2^-23 of the value or
-// 2^-38 of the largest.  The first guess, 16, suits largest values from 0.25
-// to 2047; a K tile that leaves the range is split again with another scale
-// (into [2^11, 2^12)) and the accumulators take the exact ratio.
+// overflow.  The first guess, 16, suits largest values from 0.25 to 2047; a K
+// tile that leaves the range is split again with another scale (into
+// [2^11, 2^12)) and the accumulators take the exact ratio.
+//
+// Range.  f16 ends at 2^-24: the pair of a scaled value is within 2^-23 of it down
+// to 2^-13, and within 2^-36 absolute below.  So that one row (pixel) does not pay
+// for another's magnitude, a workgroup in which a row has nonzero elements but
+// none of 2^-13 or more, or that reads a value of 2^16 or more, computes its tile
+// again in plain float32 from the same operands, at about the speed of the
+// float32 tiles.  What is left is, per element, 2^-23 of its row's largest.
 //
 // Why: v_mfma_f32_32x32x16_f16 multiplies 16 K steps in 32 cycles per SIMD,
 // three of them replace eight 64-cycle v_mfma_f32_32x32x2f32 (measured raw
@@ -25,11 +32,9 @@
 // 32, against the float32 tiles: 1x1 384 -> 128 at 40 x 40 58 -> 30 us (105 MB
 // at 3.6 TB/s), 3x3 stride 2 64 -> 128 at 80 x 80 82 -> 38 us.
 //
-// Non-finite operands: an infinite value becomes NaN in lo, and a scale for
-// magnitudes of 2^100 or more would leave nothing of the others.  A workgroup
-// that reads such a value computes its tile again in plain float32 from the
-// same operands, and convolutions with non-finite weights are not routed here:
-// infinities and NaN propagate as they do in the float32 kernels.
+// Non-finite operands: infinities take the plain path too, and convolutions with
+// non-finite weights are not routed here: infinities and NaN propagate as they do
+// in the float32 kernels.
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -42,51 +47,63 @@ namespace sy {
 // Four zeros: the source of elements outside the operand.
 __device__ const float kX3Zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
-// One element of the tile in float32, from the packed weights.
-template <int MODE>
-__device__ __forceinline__ float x3_element(const IgemmArgs& a, int row, int col) {
-  const _Float16* w = (const _Float16*)a.w3 + (long long)(col >> 5) * a.nkt * kX3Units * 8;
-  const float ws = a.w3s[col];
-  const int ox = row % a.OW, t = row / a.OW, oy = t % a.OH, n = t / a.OH;
-  float s = 0.f;
-  for (int k = 0; k < a.K; ++k) {
-    float xv = 0.f;
-    if (MODE == 2) {
-      xv = a.x[(long long)row * a.ldx + k];
-    } else if (MODE == 3) {
-      xv = k < a.ku ? a.xu[((long long)(n * (a.H >> 1) + (oy >> 1)) * (a.W >> 1) + (ox >> 1)) * a.ldxu + k]
-                    : a.x[(long long)row * a.ldx + (k - a.ku)];
-    } else {
-      const int tap = k / a.IC, ic = k - tap * a.IC, ky = tap / a.KW, kx = tap - ky * a.KW;
-      const int iy = oy * a.SH - a.PH + ky * a.DH, ix = ox * a.SW - a.PW + kx * a.DW;
-      if ((unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W)
-        xv = a.x[(((long long)n * a.H + iy) * a.W + ix) * a.ldx + ic];
-    }
-    const _Float16* e =
-        w + ((long long)(k >> 5) * kX3Units + ((k >> 4) & 1) * 128 + ((k >> 3) & 1) * 32 + (col & 31)) * 8 + (k & 7);
-    const float hi = (float)e[0], lo = (float)e[512];
-    s = __builtin_fmaf(xv, __builtin_fmaf(lo, 1.f / 2048, hi) * ws, s);
+// A wave's blocks in plain float32, on the float32 matrix cores, operands straight
+// from memory.  Lane half h takes k = 8 q + 4 h .. + 3 of its row and column.
+template <int MODE, int TM, int TN>
+__device__ __forceinline__ void x3_plain(const IgemmArgs& a, int row0, int col0, int lane, f32x16 (&acc)[TM][TN]) {
+  const int half = lane >> 5, r32 = lane & 31;
+  int m[TM], n[TM], oy[TM], ox[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    m[i] = row0 + i * 32 + r32;
+    const int t = m[i] / a.OW;
+    ox[i] = m[i] - t * a.OW;
+    n[i] = t / a.OH;
+    oy[i] = t - n[i] * a.OH;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   }
-  return s;
-}
-
-// Epilogue of a workgroup that read a huge or infinite value: every element
-// again in float32, then bias, SiLU, residual and the store as in store_acc.
-template <int MODE>
-__device__ __forceinline__ void x3_exact_tile(const IgemmArgs& a, int row0, int rows, int col0, int cols, int lane) {
-  for (int i = lane; i < rows * cols; i += 64) {
-    const int row = row0 + i / cols, col = col0 + i % cols;
-    if (row >= a.M || col >= a.OC) continue;
-    float v = x3_element<MODE>(a, row, col) + (a.bias ? a.bias[col] : 0.f);
-    if (a.silu) v = silu_fast(v);
-    long long at = (long long)row * a.ldy + col;
-    if (MODE == 2 && a.shuf > 0) {
-      const int hw = a.H * a.W, n = row / hw, rem = row - n * hw, yy = rem / a.W, xx = rem - yy * a.W;
-      const int q = col / a.shuf;
-      at = (((long long)n * 2 * a.H + 2 * yy + (q >> 1)) * (2 * a.W) + 2 * xx + (q & 1)) * a.ldy + (col - q * a.shuf);
+  const _Float16* w[TN];
+  float ws[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int col = col0 + j * 32 + r32;
+    w[j] = (const _Float16*)a.w3 + ((long long)(col >> 5) * a.nkt * kX3Units + (col & 31)) * 8;
+    ws[j] = a.w3s[col];
+  }
+  for (int k8 = 0; k8 < a.K; k8 += 8) {
+    const int k = k8 + 4 * half;
+    const int tap = k / a.IC, ic = k - tap * a.IC, ky = tap / a.KW, kx = tap - ky * a.KW;
+    f32x4 xv[TM], wv[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      bool ok = m[i] < a.M && k < a.K;
+      const float* x;
+      if (MODE == 2) {
+        x = a.x + (long long)m[i] * a.ldx + k;
+      } else if (MODE == 3) {
+        x = k < a.ku ? a.xu + ((long long)(n[i] * (a.H >> 1) + (oy[i] >> 1)) * (a.W >> 1) + (ox[i] >> 1)) * a.ldxu + k
+                     : a.x + (long long)m[i] * a.ldx + (k - a.ku);
+      } else {
+        const int iy = oy[i] * a.SH - a.PH + ky * a.DH, ix = ox[i] * a.SW - a.PW + kx * a.DW;
+        ok = ok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+        x = a.x + (((long long)n[i] * a.H + iy) * a.W + ix) * a.ldx + ic;
+      }
+      xv[i] = *(const f32x4*)(ok ? x : kX3Zeros);
     }
-    if (a.res) v = a.res[(long long)row * a.ldr + col] + v;
-    a.y[at] = v;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      wv[j] = join4(w[j] + ((long long)(k >> 5) * kX3Units + ((k >> 4) & 1) * 128 + ((k >> 3) & 1) * 32) * 8 + (k & 7),
+                    ws[j]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i][e], wv[j][e], acc[i][j], 0, 0, 0);
   }
 }
 
@@ -111,8 +128,10 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
   __shared__ __attribute__((aligned(16))) unsigned short As[2][BM][LDA];
   __shared__ __attribute__((aligned(16))) u32x4 Bs[BU];
   __shared__ float red[NW];
+  __shared__ int low;  // a row lies below the range of the workgroup's scale
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  if (tid == 0) low = 0;
   const int wm = wid / WN, wn = wid % WN;
   // Each XCD (workgroups L, L + 8, ...) takes a contiguous run of tiles, a
   // row block's column blocks next to each other: they share its A rows in
@@ -156,6 +175,7 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
 
   f32x4 ar[A_IT];
   u32x4 br[B_IT];
+  unsigned seen[A_IT] = {};  // hi parts of the thread's share of its rows, or'ed
   // Branch-free loads: an element outside the operand is read from the zeros.
   auto gload = [&](int kt) {
     const int k0 = kt * 32;
@@ -203,6 +223,7 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
     for (int i = 0; i < A_IT; ++i) {
       u32x2 hi, lo;
       split4(ar[i], s, hi, lo);
+      seen[i] |= hi[0] | hi[1];
       const int row = (tid + i * NT) / 8;
       *(u32x2*)&As[0][row][quad * 4] = hi;
       *(u32x2*)&As[1][row][quad * 4] = lo;
@@ -241,6 +262,8 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
     if (!scale_fits(big, se, &ne)) {
       if (kt > 0) rescale<TM, TN>(se, ne, acc, crs);
       se = ne;
+#pragma unroll
+      for (int i = 0; i < A_IT; ++i) seen[i] = 0;  // what counts is the rows under this scale
       stage(exp_float(se));
       __syncthreads();
     }
@@ -273,15 +296,33 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
     }
   }
 
-  const int row0 = m0 + wm * (BM / WM), col0 = n0 + wn * (BN / WN);
-  float ws[TN];
+  // Rows with no element in the pairs' full range, unless they are all zero.
+  unsigned below = 0;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) ws[j] = a.w3s[col0 + j * 32 + r32];
-  if (big >= kSplitHuge) {
-    x3_exact_tile<MODE>(a, row0, BM / WM, col0, BN / WN, lane);
-    return;
+  for (int i = 0; i < A_IT; ++i) below |= (a_ok[i] && !(or8(seen[i]) & kSplitFull)) << i;
+  if (__any(below != 0)) {
+    unsigned nz[A_IT] = {};
+    t_ic = t_ky = t_kx = 0;
+    for (int kt = 0; kt < nkt; ++kt) {
+      gload(kt);
+#pragma unroll
+      for (int i = 0; i < A_IT; ++i) nz[i] |= magnitude_bits(ar[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < A_IT; ++i)
+      if ((below >> i & 1) && nz[i]) low = 1;
   }
-  unscale<TM, TN>(ws, se, acc, crs);
+  __syncthreads();
+
+  const int row0 = m0 + wm * (BM / WM), col0 = n0 + wn * (BN / WN);
+  if (big >= kSplitHuge || low) {
+    x3_plain<MODE, TM, TN>(a, row0, col0, lane, acc);
+  } else {
+    float ws[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) ws[j] = a.w3s[col0 + j * 32 + r32];
+    unscale<TM, TN>(ws, se, acc, crs);
+  }
   if (MODE == 2 && a.shuf > 0)
     store_shuf<TM, TN>(a, a.y, acc, row0 + 4 * half, col0 + r32);
   else

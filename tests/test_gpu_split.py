@@ -258,3 +258,159 @@ def test_upsampled_part(hip, monkeypatch, tile):
         hip.end_frame()
     assert names == {"igemm_m3_x3_%dx%d_%d%d" % X3_TILES[tile]}
     near(got, exp, mag)
+
+
+def within(got, exp, mag):
+    """Float32-like: 2^-17 of the sum of the magnitudes that the output itself
+    reads (K <= 576 rounded float32 terms), whatever else its tile holds."""
+    off = np.abs(got.astype(np.float64) - exp)
+    assert np.isfinite(got).all() and (off <= 2.0 ** -17 * mag).all(), (off / (2.0 ** -17 * mag + 1e-300)).max()
+
+
+# kernel, (ic, h, w, oc, k, stride): every addressing mode of the GEMM.
+RANGE = [(X3_BASE + 1, (64, 12, 20, 40, 1, 1)), (X3_BASE + 3, (32, 9, 14, 24, 3, 1)), (X3_BASE + 4, (20, 9, 14, 24, 3, 2)),
+         (X3_BASE + 0, (96, 10, 13, 132, 1, 1))]
+RANGE_IDS = [f"{t}-" + "x".join(map(str, f)) for t, f in RANGE]
+
+
+def range_case(form, seed):
+    ic, h, w, oc, k, s = form
+    x, wt, b = data(2, ic, h, w, oc, k, seed)
+    r = synth.activations((2, oc, (h - 1) // s + 1, (w - 1) // s + 1), seed + 3)
+    return x, wt, b, s, r
+
+
+@pytest.mark.parametrize("value", [6e4, 1e10, 1e20], ids=str)
+@pytest.mark.parametrize("tile,form", RANGE, ids=RANGE_IDS)
+def test_outlier_leaves_other_outputs(hip, monkeypatch, tile, form, value):
+    """One large value in image 0: its own outputs, the other pixels of its
+    image and the other image are as close to float64 as float32 would be."""
+    x, wt, b, s, r = range_case(form, 700)
+    x[0, 3, 1, 1] = value
+    exp, mag = conv64(x, wt, b, s, True, r)
+    got, _ = run(hip, monkeypatch, tile, x, wt, b, s, True, r)
+    within(got, exp, mag)
+
+
+@pytest.mark.parametrize("small", [1e-4, 1e-7, 1e-30], ids=str)
+@pytest.mark.parametrize("large", [1.0, 1e3])
+@pytest.mark.parametrize("tile,form", RANGE, ids=RANGE_IDS)
+def test_images_of_far_apart_magnitudes(hip, monkeypatch, tile, form, large, small):
+    x, wt, b, s, _ = range_case(form, 800)
+    x[0] *= np.float32(large)
+    x[1] *= np.float32(small)
+    b *= np.float32(0)
+    exp, mag = conv64(x, wt, b, s, False, None)
+    got, _ = run(hip, monkeypatch, tile, x, wt, b, s, False)
+    within(got, exp, mag)
+
+
+@pytest.mark.parametrize("tile,form", RANGE, ids=RANGE_IDS)
+def test_small_pixels_among_zeros(hip, monkeypatch, tile, form):
+    """Pixels of 1e-9 in an image of zeros with one pixel of ordinary size."""
+    x, wt, b, s, _ = range_case(form, 900)
+    x[1] = 0
+    x[0, :, :, 4:] = 0
+    x[0, :, 2:] *= np.float32(1e-9)
+    b *= np.float32(0)
+    exp, mag = conv64(x, wt, b, s, False, None)
+    got, _ = run(hip, monkeypatch, tile, x, wt, b, s, False)
+    within(got, exp, mag)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan, 3.4e38], ids=str)
+@pytest.mark.parametrize("tile,form", RANGE, ids=RANGE_IDS)
+def test_non_finite_input_modes(hip, monkeypatch, tile, form, value):
+    x, wt, b, s, r = range_case(form, 1000)
+    x[1, 3, 2, 2] = value
+    exp, mag = conv64(x, wt, b, s, False, r)
+    exp = np.where(np.abs(exp) > np.finfo(np.float32).max, np.sign(exp) * np.inf, exp)
+    got, _ = run(hip, monkeypatch, tile, x, wt, b, s, False, r)
+    same_non_finite(got, exp)
+    fine = np.isfinite(exp)
+    assert (np.abs(got[fine] - exp[fine]) <= 2.0 ** -17 * mag[fine]).all()
+
+
+@pytest.mark.parametrize("value", [1e10, np.inf], ids=str)
+def test_transposed_conv_outlier(hip, monkeypatch, value):
+    monkeypatch.setenv("SIMDYOLO_HIP_TILE", str(X3_BASE + 1))
+    ic, oc, h, w = 36, 20, 7, 9
+    x = synth.activations((2, ic, h, w), 1100)
+    x[0, 5, 3, 2] = value
+    wt = synth.activations((ic, oc, 2, 2), 1101)
+    with np.errstate(invalid="ignore"):
+        exp = np.einsum("nchw,coij->nohiwj", x.astype(np.float64), wt).reshape(2, oc, 2 * h, 2 * w)
+    mag = np.einsum("nchw,coij->nohiwj", np.abs(x).astype(np.float64), np.abs(wt)).reshape(2, oc, 2 * h, 2 * w)
+    hip.begin_frame()
+    try:
+        conv = hip.conv_transpose2x2_create(wt, np.zeros(oc, np.float32))
+        hip.conv_set_algo(conv, CONV_IGEMM)
+        y = hip.alloc(2, oc, 2 * h, 2 * w)
+        hip.conv(conv, hip.upload(x), y)
+        got = hip.download(y)
+    finally:
+        hip.end_frame()
+    same_non_finite(got, exp)
+    fine = np.isfinite(exp)
+    assert (np.abs(got[fine] - exp[fine]) <= 2.0 ** -17 * mag[fine]).all()
+
+
+@pytest.mark.parametrize("part", ["upsampled", "rest"])
+@pytest.mark.parametrize("value", [1e10, np.inf], ids=str)
+def test_upsampled_part_outlier(hip, monkeypatch, value, part):
+    monkeypatch.setenv("SIMDYOLO_HIP_AUTOTUNE", "0")
+    monkeypatch.setenv("SIMDYOLO_HIP_TILE", str(X3_BASE + 1))
+    n, cu, c, h, w, oc = 2, 64, 20, 14, 18, 40
+    xu, x = synth.activations((n, cu, h // 2, w // 2), 1200), synth.activations((n, c, h, w), 1201)
+    (xu if part == "upsampled" else x)[0, 7, 3, 5] = value
+    _, wt, b = data(n, cu + c, h, w, oc, 1, 1202)
+    full = np.concatenate([xu.repeat(2, 2).repeat(2, 3), x], 1)
+    exp, mag = conv64(full, wt, b, 1, False, None)
+    hip.begin_frame()
+    try:
+        conv = hip.conv_create(wt, b)
+        xv = hip.alloc(n, cu + c, h, w)
+        hip.upload(x, xv.slice(cu, c))
+        yv = hip.alloc(n, oc, h, w)
+        hip.conv_upsampled(conv, hip.upload(xu), xv, yv)
+        got = hip.download(yv)
+    finally:
+        hip.end_frame()
+    same_non_finite(got, exp)
+    fine = np.isfinite(exp)
+    assert (np.abs(got[fine] - exp[fine]) <= 2.0 ** -17 * mag[fine]).all()
+
+
+# (ic, h, w, oc, kernel, strides, pads, dilation): forms that only the GEMM runs.
+GENERAL = [(16, 13, 17, 24, (3, 3), (1, 1), (2, 2, 2, 2), (2, 2)), (32, 11, 9, 40, (1, 3), (1, 1), (0, 1, 0, 1), (1, 1)),
+           (20, 12, 15, 33, (3, 2), (3, 1), (0, 1, 2, 0), (1, 1)), (64, 17, 18, 32, (5, 5), (4, 3), (2, 2, 2, 2), (1, 1))]
+
+
+@pytest.mark.parametrize("form", GENERAL, ids=lambda f: "x".join(map(str, f[:4])) + "k%dx%d" % f[4])
+@pytest.mark.parametrize("tile", range(len(X3_TILES)))
+def test_gemm_general_geometry(hip, monkeypatch, tile, form):
+    ic, h, w, oc, k, s, pads, d = form
+    monkeypatch.setenv("SIMDYOLO_HIP_TILE", str(X3_BASE + tile))
+    x = synth.activations((2, ic, h, w), 1300)
+    wt, b = synth.kaiming((oc, ic) + k, 1301), synth.activations((oc,), 1302) * np.float32(0.1)
+    top, left, bottom, right = pads
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (top, bottom), (left, right)))
+    oh, ow = [(n - e * (q - 1) - 1) // t + 1 for n, q, t, e in zip(xp.shape[2:], k, s, d)]
+    exp = np.zeros((2, oc, oh, ow)) + b[None, :, None, None]
+    mag = np.abs(exp)
+    for i in range(k[0]):
+        for j in range(k[1]):
+            t = xp[:, :, i * d[0]:i * d[0] + s[0] * (oh - 1) + 1:s[0], j * d[1]:j * d[1] + s[1] * (ow - 1) + 1:s[1]]
+            exp += np.einsum("nchw,oc->nohw", t, wt[:, :, i, j].astype(np.float64))
+            mag += np.einsum("nchw,oc->nohw", np.abs(t), np.abs(wt[:, :, i, j]).astype(np.float64))
+    hip.begin_frame()
+    try:
+        conv = hip.conv_create(wt, b, s, pads, d)
+        hip.conv_set_algo(conv, CONV_IGEMM)
+        assert hip.conv_out_size(conv, h, w) == (oh, ow)
+        y = hip.alloc(2, oc, oh, ow)
+        hip.conv(conv, hip.upload(x), y)
+        got = hip.download(y)
+    finally:
+        hip.end_frame()
+    near(got, exp, mag)
