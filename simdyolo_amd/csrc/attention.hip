@@ -10,6 +10,7 @@
 // 64) run in one kernel that keeps the scores in registers.  Other geometries
 // run both products on the FP32-MFMA GEMM (gemm_nt); S rows and V^T rows are
 // padded to N4 = round_up(N, 4) with zeros so K stays a multiple of 4.
+#include <cfloat>
 #include <cmath>
 
 #include "split.h"
@@ -27,37 +28,33 @@ struct AttnArgs {
   int ldv;
 };
 
-// Rows of the workgroup's queries in plain float32, one wave per query: what a
-// workgroup does that met a non-finite or huge operand (kSplitHuge) or scale.
-__device__ __forceinline__ void attn_exact(const AttnArgs& a, const float* base, float* ob, int q0, int queries,
-                                           int wave, int lane) {
-  for (int q = wave; q < queries; q += 4) {
-    if (q0 + q >= a.N) continue;
-    const float* qr = base + (long long)(q0 + q) * a.ldq;
-    auto score = [&](int j) {
-      if (j >= a.N) return -INFINITY;
-      const float* kr = base + (long long)j * a.ldq + a.kd;
-      float s = 0.f;
-      for (int c = 0; c < a.kd; ++c) s = __builtin_fmaf(qr[c], kr[c], s);
-      return s * a.scale;
-    };
-    float mx = -INFINITY;
-    for (int j = lane; j < a.N; j += 64) mx = fmaxf(mx, score(j));
+// One query's output in plain float32 by one wave: lane `lane`'s channel.  Weights
+// are normalised before they meet the values, so that no finite average overflows.
+__device__ __forceinline__ float attn_row(const AttnArgs& a, const float* base, int q, int lane) {
+  const float* qr = base + (long long)q * a.ldq;
+  auto score = [&](int j) {
+    if (j >= a.N) return -INFINITY;
+    const float* kr = base + (long long)j * a.ldq + a.kd;
+    float s = 0.f;
+    for (int c = 0; c < a.kd; ++c) s = __builtin_fmaf(qr[c], kr[c], s);
+    return s * a.scale;
+  };
+  float mx = -INFINITY, sum = 0.f, acc = 0.f;
+  for (int j = lane; j < a.N; j += 64) mx = fmaxf(mx, score(j));
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-    float sum = 0.f, acc = 0.f;
-    for (int j0 = 0; j0 < a.N; j0 += 64) {
-      const float e = j0 + lane < a.N ? expf(score(j0 + lane) - mx) : 0.f;
-      sum += e;
-      for (int t = 0; t < min(64, a.N - j0); ++t) {
-        const float et = __shfl(e, t);
-        if (lane < a.hd) acc = __builtin_fmaf(et, base[(long long)(j0 + t) * a.ldq + 2 * a.kd + lane], acc);
-      }
+  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+  for (int j = lane; j < a.N; j += 64) sum += expf(score(j) - mx);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  const float inv = 1.f / sum;
+  for (int j0 = 0; j0 < a.N; j0 += 64) {
+    const float e = j0 + lane < a.N ? expf(score(j0 + lane) - mx) * inv : 0.f;
+    for (int t = 0; t < min(64, a.N - j0); ++t) {
+      const float et = __shfl(e, t);
+      if (lane < a.hd) acc = __builtin_fmaf(et, base[(long long)(j0 + t) * a.ldq + 2 * a.kd + lane], acc);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    if (lane < a.hd) ob[(long long)(q0 + q) * a.ldo + lane] = acc / sum;
   }
+  return acc;
 }
 
 // e^x for x up to a few units: 2^t of the hardware at t = x log2(e) rounded, times 1 plus the
@@ -71,6 +68,40 @@ __device__ __forceinline__ float exp_neg(float x) {
   return __builtin_fmaf(p, r * 0.69314718f, p);
 }
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Eight floats as three bf16 parts each, v = p[0] + p[1] + p[2] exactly.
+__device__ __forceinline__ void parts8(const f32x4& x, const f32x4& y, bf16x8 (&p)[3]) {
+  u32x4 w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f32x2v v = i < 2 ? f32x2v{x[2 * i], x[2 * i + 1]} : f32x2v{y[2 * i - 4], y[2 * i - 3]};
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const unsigned b = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+      w[s][i] = b;
+      if (s < 2) {
+        v[0] -= __builtin_bit_cast(float, b << 16);
+        v[1] -= __builtin_bit_cast(float, b & 0xffff0000u);
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < 3; ++s) p[s] = __builtin_bit_cast(bf16x8, w[s]);
+}
+
+// main + rest += a b: the leading parts' product in main, the five next ones in
+// rest.
+__device__ __forceinline__ void mfma_parts(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x16& main, f32x16& rest) {
+  rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], rest, 0, 0, 0);
+  main = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], main, 0, 0, 0);
+  rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], rest, 0, 0, 0);
+  rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], rest, 0, 0, 0);
+  rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], rest, 0, 0, 0);
+  rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], rest, 0, 0, 0);
+}
+
 // 32 queries of one head and image per workgroup.  Wave w takes the 32-key
 // tiles w, w + 4, ... with a running maximum, sum and output of its own; the
 // four are joined through LDS at the end.  Nothing else is shared: operands go
@@ -82,28 +113,32 @@ __device__ __forceinline__ float exp_neg(float x) {
 // already the B operand of O^T = V^T P^T under the key order
 // 8 (e / 4) + 4 half + e % 4 of a 16-key step, in which V is loaded.
 //
-// Both products are f16 splits (split_gemm.hip): queries, each key tile and the
-// values under scales from their largest magnitudes, probabilities under 2^11.
+// Both products take float32 operands as three bf16 parts, which hold a float's 24
+// significand bits over its whole exponent range (parts below 2^-126, of values
+// below 2^-110, may be lost): no operand's precision depends on another's size, as
+// it would with f16 pairs under common scales.  Six of the nine part products are
+// taken, the rest is below 2^-24 of the product.  Where a part is not finite
+// (infinities, NaN, values that round to 2^128 in bf16) or a sum overflows, the
+// query's output is not finite either and is computed again in plain float32.
 //
-// The running maximum moves (and the sums with it) only where a score passes it
-// by kSlack: until then weights reach e^kSlack, and under 2^11 still fit f16.
-// The test is on the difference, which is exact between floats this near: the
-// sum of maximum and slack rounds, from 2^23 on to more than the slack.
+// The running maximum moves (and the sums with it) only where a score passes it by
+// kSlack; until then weights reach e^kSlack.  The test is on the difference, which
+// is exact between floats this near: the sum of maximum and slack rounds, from
+// 2^23 on to more than the slack.
 //
-// Bound by VALU work (splitting K, V and P, the exponentials: about 650
-// operations beside 18 MFMAs per tile) and, at 400 tokens, by the latency of its
-// few tiles.  Measured against two GEMMs, a softmax and a copy with the scores
-// in memory, us: 2 heads, 400 tokens, batch 16 74 -> 23, batch 1 25 -> 14.6;
-// 4 heads, 1,600 tokens, batch 8 858 -> 156.  With expf, a maximum that moves in
-// every tile and per-lane row addresses these were 24.5, 15.5 and 184.  64
-// queries per workgroup, which would split each key tile for twice the work,
-// spill registers: 214.
-constexpr float kSlack = 2.5f;  // e^2.5 2^11 < 2^15
+// Bound by VALU work (the parts of K, V and P 350 operations per tile, the
+// exponentials and sums about 220, beside 36 MFMAs) and, at 400 tokens, by the
+// latency of its few tiles.  Measured, us, against two GEMMs, a softmax and a copy
+// with the scores in memory / float32 MFMAs for both products / f16 pairs: 2 heads,
+// 400 tokens, batch 16 74 / 28 / 21.4 -> 19.9, batch 1 25 / 18 / 14.5 -> 13.5;
+// 4 heads, 1,600 tokens, batch 8 858 / 206 / 141 -> 144.  Error against float64 at
+// 400 tokens 1.4e-7 (1.9e-7 with f16 pairs, 2.0e-7 with float32 MFMAs summed tile by
+// tile).  Three waves per SIMD spill registers: 178 us at 1,600 tokens.
+constexpr float kSlack = 2.5f;
 __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
-  constexpr int TQ = 1, NQ = 32 * TQ;  // 32-query blocks, queries
+  constexpr int NQ = 32;  // queries
   __shared__ float O[4][NQ][65];
   __shared__ float M[4][NQ], Lsum[4][NQ];
-  __shared__ int wild[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, r32 = lane & 31;
   const int qt = blockIdx.x % a.qtiles, bh = blockIdx.x / a.qtiles, head = bh % a.heads, b = bh / a.heads;
@@ -118,36 +153,28 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
     const int c = 16 * ks + 8 * half + 4 * i;
     return c < a.kd ? *(const f32x4*)(base + min(row, a.N - 1) * a.ldq + at + c) : zero;
   };
-  auto max4 = [](float m, const f32x4& v) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) m = fmaxf(m, __builtin_fabsf(v[e]));
-    return m;
-  };
-  // Eight floats times s as operand halves.
-  auto split8 = [](const f32x4& x, const f32x4& y, float s, f16x8& hi, f16x8& lo) {
-    u32x2 h0, h1, l0, l1;
-    split4(x, s, h0, l0);
-    split4(y, s, h1, l1);
-    hi = __builtin_bit_cast(f16x8, u32x4{h0[0], h0[1], h1[0], h1[1]});
-    lo = __builtin_bit_cast(f16x8, u32x4{l0[0], l0[1], l1[0], l1[1]});
-  };
-
-  // A tile's keys and values.  In a whole tile the rows' addresses are scalar, with
-  // one offset per lane; past the last key both read the last key's row.
+  // A tile's keys and values; past the last key both read the last key's row.  Past
+  // kd the keys' last channels are read again, which the queries' zeros cancel.  In a
+  // whole tile the value rows' addresses are scalar, with one offset per lane.
   f32x4 k[2][2];
   float v[2][16];
-  const int krow = r32 * a.ldq + a.kd + 8 * half;
+  int kcol[2][2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) kcol[ks][i] = min(16 * ks + 8 * half + 4 * i, a.kd - 4);
   const int vrow = 4 * half * a.ldq + 2 * a.kd, vcol[2] = {min(r32, a.hd - 1), min(32 + r32, a.hd - 1)};
-  auto load = [&](int j0) __attribute__((always_inline)) {
+  auto load_k = [&](int j0) __attribute__((always_inline)) {
+    const float* tb = base + j0 * a.ldq + a.kd;
+    const int row = min(r32, a.N - 1 - j0) * a.ldq;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) k[ks][i] = *(const f32x4*)(tb + (unsigned)(row + kcol[ks][i]));
+  };
+  auto load_v = [&](int j0) __attribute__((always_inline)) {
     if (j0 + 32 <= a.N) {
       const float* tb = base + j0 * a.ldq;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int c = 16 * ks + 8 * half + 4 * i;
-          k[ks][i] = c < a.kd ? *(const f32x4*)(tb + (krow + 16 * ks + 4 * i)) : zero;
-        }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const float* vr = tb + (16 * (e >> 3) + 8 * ((e >> 2) & 1) + (e & 3)) * a.ldq;
@@ -156,10 +183,6 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
       }
       return;
     }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) k[ks][i] = row4(j0 + r32, a.kd, ks, i);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int j = min(j0 + 16 * (e >> 3) + 8 * ((e >> 2) & 1) + 4 * half + (e & 3), a.N - 1);
@@ -170,159 +193,97 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
   };
   const int tiles = (a.N + 31) / 32;
 
-  f16x8 qh[TQ][2], ql[TQ][2];
-  float huge = 0.f;
-  int sq;
+  bf16x8 q[2][3];
   {
-    f32x4 q[TQ][2][2];
-    float m = 0.f;
-#pragma unroll
-    for (int t = 0; t < TQ; ++t)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          q[t][ks][i] = row4(q0 + 32 * t + r32, 0, ks, i);
-          m = max4(m, q[t][ks][i]);
-        }
-    load(min(wave, tiles - 1) * 32);
-    m = readlane63(wave_max63(m));
-    huge = m;
-    sq = scale_exp(m);
-#pragma unroll
-    for (int t = 0; t < TQ; ++t)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) split8(q[t][ks][0], q[t][ks][1], exp_float(sq), qh[t][ks], ql[t][ks]);
-  }
-
-  f32x16 acc[2][TQ], crs[2][TQ];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int t = 0; t < TQ; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][t][r] = crs[j][t][r] = 0.f;
-  float mrun[TQ], lrun[TQ];
-#pragma unroll
-  for (int t = 0; t < TQ; ++t) {
-    mrun[t] = -INFINITY;
-    lrun[t] = 0.f;
-  }
-  int sv = kSplitExpGuess;
-  float vbig = 0.f;
-
-  for (int kt = wave; kt < tiles; kt += 4) {
-    const int j0 = kt * 32;
-    float km = 0.f, vm = 0.f;
+    f32x4 t[2][2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) km = max4(km, k[ks][i]);
+      for (int i = 0; i < 2; ++i) t[ks][i] = row4(q0 + r32, 0, ks, i);
+    load_k(min(wave, tiles - 1) * 32);
+    load_v(min(wave, tiles - 1) * 32);
 #pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) vm = fmaxf(vm, __builtin_fabsf(v[d][e]));
-    km = readlane63(wave_max63(km));
-    vbig = fmaxf(vbig, readlane63(wave_max63(vm)));
-    huge = fmaxf(huge, fmaxf(km, vbig));
-    const int sk = scale_exp(km);
-    f16x8 kh[2], kl[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) split8(k[ks][0], k[ks][1], exp_float(sk), kh[ks], kl[ks]);
-    int ne;
-    if (!scale_fits(vbig, sv, &ne)) {
-      rescale<2, TQ>(sv, ne, acc, crs);
-      sv = ne;
-    }
-    f16x8 vh[2][2], vl[2][2];  // [block of 32 dims][16-key step]
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int st = 0; st < 2; ++st)
-        split8(f32x4{v[d][8 * st], v[d][8 * st + 1], v[d][8 * st + 2], v[d][8 * st + 3]},
-               f32x4{v[d][8 * st + 4], v[d][8 * st + 5], v[d][8 * st + 6], v[d][8 * st + 7]}, exp_float(sv), vh[d][st],
-               vl[d][st]);
-    load(min(kt + 4, tiles - 1) * 32);  // the next tile (the last loads its own again)
-
-    // 2^-(sq + sk) in two factors: their sum may pass the exponent range.
-    const float us = exp_float(254 - sq), uk = exp_float(254 - sk) * a.scale;
-#pragma unroll
-    for (int t = 0; t < TQ; ++t) {
-      f32x16 s, c;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = c[r] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[ks], qh[t][ks], c, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks], qh[t][ks], s, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[ks], ql[t][ks], c, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(c[r], 1.f / 2048, s[r]) * us * uk;
-      if (j0 + 32 > a.N) {
-        asm volatile("");  // a branch, not 16 selects in every tile
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (j0 + 8 * (r >> 2) + 4 * half + (r & 3) >= a.N) s[r] = -INFINITY;
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      if (__any(mx - mrun[t] > kSlack)) {
-        mx = fmaxf(mx, mrun[t]);
-        const float f = exp_neg(mrun[t] - (mx == -INFINITY ? 0.f : mx));
-        mrun[t] = mx;
-        lrun[t] *= f;
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            acc[d][t][r] *= f;
-            crs[d][t][r] *= f;
-          }
-      }
-      const float from = mrun[t] == -INFINITY ? 0.f : mrun[t];  // no weight yet: all are 0
-      float sum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[r] = exp_neg(s[r] - from);
-        sum += s[r];
-      }
-      lrun[t] += sum;
-      f16x8 ph[2], pl[2];
-#pragma unroll
-      for (int st = 0; st < 2; ++st)
-        split8(f32x4{s[8 * st], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3]},
-               f32x4{s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]}, 2048.f, ph[st], pl[st]);
-#pragma unroll
-      for (int st = 0; st < 2; ++st)
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          crs[d][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[d][st], ph[st], crs[d][t], 0, 0, 0);
-          acc[d][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[d][st], ph[st], acc[d][t], 0, 0, 0);
-          crs[d][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[d][st], pl[st], crs[d][t], 0, 0, 0);
-        }
-    }
+    for (int ks = 0; ks < 2; ++ks) parts8(t[ks][0], t[ks][1], q[ks]);
   }
 
-  const float uv = exp_float(254 - sv) * (1.f / 2048);
+  f32x16 acc[2], rest[2];
 #pragma unroll
-  for (int t = 0; t < TQ; ++t) {
-    const float l = lrun[t] + __shfl_xor(lrun[t], 32);
-    if (half == 0) {
-      M[wave][32 * t + r32] = mrun[t];
-      Lsum[wave][32 * t + r32] = l;
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[d][r] = rest[d][r] = 0.f;
+  float mrun = -INFINITY, lrun = 0.f;
+
+  for (int kt = wave; kt < tiles; kt += 4) {
+    const int j0 = kt * 32;
+    const int jn = min(kt + 4, tiles - 1) * 32;  // the next tile (the last loads its own again)
+    f32x16 s, c;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = c[r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 kp[3];
+      parts8(k[ks][0], k[ks][1], kp);
+      mfma_parts(kp, q[ks], s, c);
     }
+    load_k(jn);
 #pragma unroll
-    for (int d = 0; d < 2; ++d)
+    for (int r = 0; r < 16; ++r) s[r] = (s[r] + c[r]) * a.scale;
+    if (j0 + 32 > a.N) {
+      asm volatile("");  // a branch, not 16 selects in every tile
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        O[wave][32 * t + r32][32 * d + 8 * (r >> 2) + 4 * half + (r & 3)] =
-            __builtin_fmaf(crs[d][t][r], 1.f / 2048, acc[d][t][r]) * uv;
+        if (j0 + 8 * (r >> 2) + 4 * half + (r & 3) >= a.N) s[r] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    if (__any(mx - mrun > kSlack)) {
+      mx = fmaxf(mx, mrun);
+      const float f = exp_neg(mrun - (mx == -INFINITY ? 0.f : mx));
+      mrun = mx;
+      lrun *= f;
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[d][r] *= f;
+          rest[d][r] *= f;
+        }
+    }
+    const float from = mrun == -INFINITY ? 0.f : mrun;  // no weight yet: all are 0
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = exp_neg(s[r] - from);
+      sum += s[r];
+    }
+    lrun += sum;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      bf16x8 p[3];
+      parts8(f32x4{s[8 * st], s[8 * st + 1], s[8 * st + 2], s[8 * st + 3]},
+             f32x4{s[8 * st + 4], s[8 * st + 5], s[8 * st + 6], s[8 * st + 7]}, p);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        bf16x8 vp[3];
+        parts8(f32x4{v[d][8 * st], v[d][8 * st + 1], v[d][8 * st + 2], v[d][8 * st + 3]},
+               f32x4{v[d][8 * st + 4], v[d][8 * st + 5], v[d][8 * st + 6], v[d][8 * st + 7]}, vp);
+        mfma_parts(vp, p, acc[d], rest[d]);
+      }
+    }
+    load_v(jn);
   }
-  // A scale past 2^20 might overflow its product with a key tile's factor.
-  if (lane == 0) wild[wave] = huge >= kSplitHuge || !(__builtin_fabsf(a.scale) <= 0x1p20f);
+
+  const float l = lrun + __shfl_xor(lrun, 32);
+  if (half == 0) {
+    M[wave][r32] = mrun;
+    Lsum[wave][r32] = l;
+  }
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) O[wave][r32][32 * d + 8 * (r >> 2) + 4 * half + (r & 3)] = acc[d][r] + rest[d][r];
   // v of these rows, dense, for the positional conv: thread (row q, dim lane).
   float vd[NQ / 4];
 #pragma unroll
@@ -332,11 +293,8 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
 #pragma unroll
   for (int i = 0; i < NQ / 4; ++i)
     if (q0 + wave + 4 * i < a.N && lane < a.hd) vb[(long long)(q0 + wave + 4 * i) * a.ldv + lane] = vd[i];
-  if (wild[0] | wild[1] | wild[2] | wild[3]) {
-    attn_exact(a, base, ob, q0, NQ, wave, lane);
-    return;
-  }
   // Joins the waves' partial outputs; a wave without keys weighs nothing.
+  unsigned again = 0;  // rows to compute in plain float32
 #pragma unroll
   for (int i = 0; i < NQ / 4; ++i) {
     const int q = wave + 4 * i;
@@ -350,7 +308,15 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
       l = __builtin_fmaf(Lsum[w][q], f, l);
       s = __builtin_fmaf(O[w][q][lane], f, s);
     }
-    if (q0 + q < a.N && lane < a.hd) ob[(long long)(q0 + q) * a.ldo + lane] = s / l;
+    const float y = s / l;
+    const bool here = q0 + q < a.N && lane < a.hd;
+    again |= (__any(here && !(__builtin_fabsf(y) <= FLT_MAX)) ? 1u : 0u) << i;
+    if (here) ob[(long long)(q0 + q) * a.ldo + lane] = y;
+  }
+  for (; again; again &= again - 1) {
+    const int row = q0 + wave + 4 * __builtin_ctz(again);
+    const float y = attn_row(a, base, row, lane);
+    if (lane < a.hd) ob[(long long)row * a.ldo + lane] = y;
   }
 }
 

@@ -2,9 +2,9 @@
 tiles over four waves, key and head dims below its 32 and 64), with non-finite
 and far-scaled operands, and the geometry past it that keeps the GEMMs.
 
-Bound: scores carry at most 2^-19 of sum |q||k| scale (f16-split products, as
-in the convolutions), a probability e^(s - m) that error twice, and the output
-2^-19 of the weighted sum of |v| more.
+Bound: scores carry at most 2^-19 of sum |q||k| scale (products within 2^-24,
+32 of them summed in float32), a probability e^(s - m) that error twice, and the
+output 2^-19 of the weighted sum of |v| more.
 """
 import numpy as np
 import pytest
@@ -153,3 +153,31 @@ def test_large_scores(hip, sign, step):
     exp, mag = t[2 * kd:] @ p.T, np.abs(t[2 * kd:]) @ p.T
     err = np.abs(got.reshape(hd, 160) - exp)
     assert np.isfinite(got).all() and (err <= 2.0 ** -18 * mag).all(), (err / mag).max()
+
+
+RANGES = {
+    # One query 2^29 times the others', whose own scores are of order 1.
+    "queries": lambda q, k, v: (np.where(np.arange(96) == 5, 3e4, 2.0 ** -14) * q, 2.0 ** 14 * k, v),
+    # Every query attends to key 40 alone, whose values are 10^-12 of the others'.
+    "value rows": lambda q, k, v: (q + 8, np.where(np.arange(96) == 40, 8.0, -1.0) + 0 * k,
+                                   np.where(np.arange(96) == 40, 1e-12, 1.0) * v),
+    # Channels from 1 down to 10^-20.
+    "value channels": lambda q, k, v: (q, k, np.logspace(0, -20, 64)[None, :, None] * v),
+    # One value of 10^20: only its channel and no other sees it.
+    "outlier": lambda q, k, v: (q, k, np.where((np.arange(96) == 70) & (np.arange(64) == 3)[:, None], 1e20, v)),
+    # A sum of 96 such values overflows, their average does not.
+    "largest": lambda q, k, v: (q, k, 1e37 * (1 + 0.1 * v)),
+}
+
+
+@pytest.mark.parametrize("name", RANGES)
+def test_precision_is_each_operands_own(hip, name):
+    """Operands of far-apart magnitudes: every output within the bound of its own products, no floor added."""
+    heads, kd, hd = 2, 32, 64
+    x = synth.activations((heads, 2 * kd + hd, 96), 11)
+    q, k, v = RANGES[name](x[:, :kd], x[:, kd:2 * kd], x[:, 2 * kd:])
+    qkv = np.concatenate([np.broadcast_to(t, (heads, d, 96)) for t, d in ((q, kd), (k, kd), (v, hd))], 1)
+    qkv = qkv.astype(np.float32).reshape(1, -1, 8, 12)
+    exp, bound, _ = reference(qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    got, _, _ = run(hip, qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    assert np.isfinite(got).all() and (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
