@@ -38,17 +38,27 @@ constexpr int kSplitExpGuess = 127 + 4, kSplitExpMax = 127 + 113;
 constexpr unsigned kSplitFull = 0x78007800u;
 __device__ __forceinline__ float exp_float(int e) { return __builtin_bit_cast(float, (unsigned)e << 23); }
 
-// v or'ed over aligned groups of 8 lanes.
-__device__ __forceinline__ unsigned or8(unsigned v) {
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false);          // lane ^ 1
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false);          // lane ^ 2
-  return v | (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false);  // 7 - lane
+// v or'ed over aligned groups of W lanes.
+template <int W>
+__device__ __forceinline__ unsigned or_lanes(unsigned v) {
+  static_assert(W == 4 || W == 8 || W == 16 || W == 32, "quads to half waves");
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false);               // lane ^ 1
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false);               // lane ^ 2
+  if (W > 4) v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false);  // 7 - lane
+  if (W > 8) v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false);  // 15 - lane
+  if (W > 16) v |= (unsigned)__shfl_xor((int)v, 16);
+  return v;
 }
 
 // Four elements' bits, without their signs.
 __device__ __forceinline__ unsigned magnitude_bits(const f32x4 v) {
   const u32x4 b = __builtin_bit_cast(u32x4, v);
   return (b[0] | b[1] | b[2] | b[3]) & 0x7fffffffu;
+}
+
+// Largest magnitude of four.
+__device__ __forceinline__ float max4(const f32x4 v) {
+  return fmaxf(fmaxf(__builtin_fabsf(v[0]), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
 }
 
 // Four weights from their pair (hi at w, lo 512 halves on) and inverse scale.

@@ -11,6 +11,15 @@
 // straight into MFMA operands: their packed order makes each read of a wave
 // 1 KiB contiguous, and the workgroup's waves read the same ones.
 //
+// Scales are split_gemm.hip's, by chunk instead of K tile.  A workgroup that reads
+// a value of 2^16 or more, or a pixel whose channels of a chunk are not all zero
+// but all below the pairs' full range, computes its tile again in plain float32, at
+// about the speed of the float32 tiles: an element's error is at most 2^-23 of its
+// pixel's largest of the chunk, whatever the other pixels hold.  The test costs two
+// operations per four values: 80 -> 80 at 80 x 80, batch 32, 103.2 -> 104.8 us,
+// 64 -> 64 52.2 -> 52.4, 64 -> 128 stride 2 39.5 -> 39.7, 80 -> 80 at 45 x 75, batch
+// 4, 11.0 -> 11.4.  Bits kept per pixel for all chunks took up to 10% (spills).
+//
 // A wave owns TM 32-pixel blocks x TN 32-channel blocks.  Per (tap, 16
 // channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
 // MFMAs of 32 cycles.
@@ -61,42 +70,65 @@ __device__ __forceinline__ int mul24(int x, int y) { return (int)__umul24((unsig
 // Pixel of a 32-pixel block that MFMA row r (lane r of a half wave) holds.
 __device__ __forceinline__ int c3_row(int r) { return ((0x73261540 >> (r & 28)) & 7) * 4 + (r & 3); }
 
-__device__ __forceinline__ float c3_weight(const C3Args& a, int col, int ic, int tap) {
-  const _Float16* e = (const _Float16*)a.w +
-                      ((((long long)(col >> 5) * a.ng + (ic >> 4)) * 9 + tap) * 128 + ((ic >> 3) & 1) * 32 +
-                       (col & 31)) * 8 + (ic & 7);
-  const float hi = (float)e[0], lo = (float)e[512];
-  return __builtin_fmaf(lo, 1.f / 2048, hi) * a.ws[col];
-}
+// Four zeros: the source of input outside the image.
+__device__ const float kC3Zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
-// Epilogue of a workgroup that read a huge or infinite value: its elements
-// again in float32, from the input and the packed weights.
-__device__ __forceinline__ void c3_exact(const C3Args& a, const int* opix, int pixels, int col0, int cols, int lane) {
-  for (int i = lane; i < pixels * cols; i += 64) {
-    const int pix = opix[i / cols], col = col0 + i % cols;
-    if (pix >= a.M || col >= a.OC) continue;
-    const int ox = pix % a.OW, t = pix / a.OW, oy = t % a.OH, n = t / a.OH;
-    float v = 0.f;
-    for (int tap = 0; tap < 9; ++tap) {
-      const int iy = oy * a.S - 1 + tap / 3, ix = ox * a.S - 1 + tap % 3;
-      if ((unsigned)iy >= (unsigned)a.H || (unsigned)ix >= (unsigned)a.W) continue;
-      const float* x = a.x + (((long long)n * a.H + iy) * a.W + ix) * a.ldx;
-      for (int c = 0; c < a.IC; ++c) v = __builtin_fmaf(x[c], c3_weight(a, col, c, tap), v);
+// A wave's blocks in plain float32, on the float32 matrix cores, operands straight
+// from memory: channel groups g0, g0 + gs, ...  Lane half h takes channels
+// 8 q + 4 h .. + 3 of its pixel and column.
+template <int TM, int TN>
+__device__ __forceinline__ void c3_plain(const C3Args& a, const int* opix, int ob0, int g0, int gs, int lane,
+                                         f32x16 (&acc)[TM][TN]) {
+  const int half = lane >> 5, r32 = lane & 31;
+  const float* img[TM];
+  int iy0[TM], ix0[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int pix = opix[i * 32 + r32], t = pix / a.OW, n = t / a.OH;
+    img[i] = a.x + (long long)n * a.H * a.W * a.ldx;
+    iy0[i] = pix < a.M ? (t - n * a.OH) * a.S - 1 : -4;  // -4: every tap is outside
+    ix0[i] = (pix - t * a.OW) * a.S - 1;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  }
+  float ws[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) ws[j] = a.ws[(ob0 + j) * 32 + r32];
+  for (int g = g0; g < a.ng; g += gs) {
+    for (int k = 0; k < 18; ++k) {
+      const int tap = k >> 1, h8 = k & 1, c = 16 * g + 8 * h8 + 4 * half;
+      f32x4 xv[TM], wv[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int iy = iy0[i] + tap / 3, ix = ix0[i] + tap % 3;
+        const bool ok = c < a.IC && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+        xv[i] = *(const f32x4*)(ok ? img[i] + ((long long)iy * a.W + ix) * a.ldx + c : kC3Zeros);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        wv[j] = join4((const _Float16*)a.w +
+                          ((((long long)(ob0 + j) * a.ng + g) * 9 + tap) * 128 + 32 * h8 + r32) * 8 + 4 * half,
+                      ws[j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i][e], wv[j][e], acc[i][j], 0, 0, 0);
     }
-    v += a.bias[col];
-    if (a.silu) v = silu_fast(v);
-    if (a.res) v = a.res[(long long)pix * a.ldr + col] + v;
-    a.y[(long long)pix * a.ldy + col] = v;
   }
 }
 
 // Waves per SIMD the registers are allocated for (each measured without spills
 // that matter).
 constexpr int c3_waves(int s, int g, int nw, int blocks, int kw, bool one) {
-  if (kw > 1) return 2;
+  if (kw > 1) return s == 1 ? 4 : 2;
   if (one) return blocks == 2 ? (s == 2 ? 2 : 3) : (s == 2 ? 3 : 4);
   if (blocks == 2) return g == 4 || s == 2 ? 2 : 3;
-  return (g == 4 || s == 2) && nw == 2 ? 2 : s == 2 ? 3 : 4;
+  return (g == 4 || s == 2) && nw == 2 ? 2 : 3;
 }
 
 // S: stride.  G: 16-channel groups per chunk.  At stride 2 a patch row holds its
@@ -115,7 +147,7 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
   __shared__ __attribute__((aligned(16))) _Float16 P[G * 4 * PL];
   static_assert(KW == 1 || G * 4 * PL * 2 >= KW * 4096, "the partial sums fit the patch's memory");
   __shared__ __attribute__((aligned(16))) int opix[BM];
-  __shared__ float red[NW];  // the waves' largest magnitudes
+  __shared__ float red[NW];  // the waves' largest magnitudes, negative: a pixel is below the scale's range
 
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   static_assert(KW == 1 || (WM * WN * TM * TN == 1 && 16 % KW == 0), "split sums: one block per workgroup");
@@ -161,12 +193,20 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
       d[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, ch * (64 * G), 0));
     }
   };
-  auto stage = [&](float s) __attribute__((always_inline)) {
+  // A chunk into LDS.  A pixel is below the scale's range if its channels of the
+  // chunk are not all zero and none is in the pairs' full range (2^-13 or more,
+  // scaled).  Few are: the first test is on any four channels of a thread.
+  static_assert(L_IT <= 32, "a bit per staged pixel");
+  auto stage = [&](int ch, int se) __attribute__((always_inline)) {
+    const float s = exp_float(se);
+    const unsigned range = (unsigned)(241 - se) << 23;  // bits of 2^-13 / s
     float m = 0.f;
+    unsigned least = ~0u;  // bits of the smallest nonzero maximum, less one
 #pragma unroll
     for (int i = 0; i < L_IT; ++i) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) m = fmaxf(m, __builtin_fabsf(d[i][e]));
+      const float mi = max4(d[i]);
+      m = fmaxf(m, mi);
+      least = min(least, __builtin_bit_cast(unsigned, mi) - 1);
       const int px = px0 + i * (NT / (4 * G));
       u32x2 hi, lo;
       split4(d[i], s, hi, lo);
@@ -182,6 +222,17 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
       }
     }
     m = wave_max63(m);
+    if (__builtin_expect(__any(least < range - 1), 0)) {
+      unsigned full = 0, some = 0;  // a bit per pixel
+      if (S == 2 && !ONE) xload(ch);  // their many registers are not kept until here
+#pragma unroll
+      for (int i = 0; i < L_IT; ++i) {
+        const float mi = max4(d[i]);
+        if (mi > 0.f) some |= 1u << i;
+        if (__builtin_bit_cast(unsigned, mi) >= range) full |= 1u << i;
+      }
+      if (__any(or_lanes<4 * G>(some) & ~or_lanes<4 * G>(full))) m = -m;
+    }
     if (lane == 63) red[wid] = m;
   };
   // Weights run kRing taps ahead of their use, across groups and chunks (the
@@ -235,25 +286,35 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = crs[i][j][r] = 0.f;
   };
+  int low = 0;  // negative: a chunk had a pixel below the range of its scale
+  auto maxima = [&]() __attribute__((always_inline)) {
+    int l = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      big = fmaxf(big, __builtin_fabsf(red[w]));
+      l |= __builtin_bit_cast(int, red[w]);
+    }
+    return __builtin_amdgcn_readfirstlane(l);
+  };
   // Chunk ch (loaded already) into LDS.
   auto enter = [&](int ch) __attribute__((always_inline)) {
-    stage(exp_float(se));
+    stage(ch, se);
     if (ch == 0) {
 #pragma unroll
       for (int t = 0; t < kRing; ++t) wload(wk, t);
     }
     __syncthreads();
-#pragma unroll
-    for (int w = 0; w < NW; ++w) big = fmaxf(big, red[w]);
-    int ne;
+    int l = maxima(), ne;
     if (!scale_fits(big, se, &ne)) {  // rare: the chunk again with another scale
       if (!ONE && ch > 0) rescale<TM, TN>(se, ne, acc, crs);
       se = ne;
       xload(ch);
       __syncthreads();  // every wave has read the maxima
-      stage(exp_float(se));
+      stage(ch, se);
       __syncthreads();
+      l = maxima();
     }
+    low |= l;
   };
   if (ONE) enter(0);
   clear();
@@ -310,11 +371,13 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
   }
 
   const int* po = opix + wm * TM * 32;
-  if (big >= kSplitHuge) {
-    if (wk == 0) c3_exact(a, po, TM * 32, col0 - r32, TN * 32, lane);
-    return;
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)(big >= kSplitHuge)) || low < 0, 0)) {
+    int l = lane;
+    asm volatile("" : "+v"(l));  // its addresses are not kept from the main loop's
+    c3_plain<TM, TN>(a, po, ob0, wk, KW, l, acc);
+  } else {
+    unscale<TM, TN>(ws, se, acc, crs);
   }
-  unscale<TM, TN>(ws, se, acc, crs);
   if (KW > 1) {
     // Rows r of the sums belong to wave r KW / 16.
     float* sums = (float*)P;

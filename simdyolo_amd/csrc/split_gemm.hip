@@ -299,7 +299,7 @@ __global__ __launch_bounds__(WM* WN * 64, (BM / WM) * (BN / WN) >= 3072   ? 2
   // Rows with no element in the pairs' full range, unless they are all zero.
   unsigned below = 0;
 #pragma unroll
-  for (int i = 0; i < A_IT; ++i) below |= (a_ok[i] && !(or8(seen[i]) & kSplitFull)) << i;
+  for (int i = 0; i < A_IT; ++i) below |= (a_ok[i] && !(or_lanes<8>(seen[i]) & kSplitFull)) << i;
   if (__any(below != 0)) {
     unsigned nz[A_IT] = {};
     t_ic = t_ky = t_kx = 0;

@@ -267,9 +267,12 @@ def within(got, exp, mag):
     assert np.isfinite(got).all() and (off <= 2.0 ** -17 * mag).all(), (off / (2.0 ** -17 * mag + 1e-300)).max()
 
 
-# kernel, (ic, h, w, oc, k, stride): every addressing mode of the GEMM.
+# kernel, (ic, h, w, oc, k, stride): every addressing mode of the GEMM; the patch kernel at both strides, with
+# one chunk of channels, several, and channel groups shared out over four and eight waves.
 RANGE = [(X3_BASE + 1, (64, 12, 20, 40, 1, 1)), (X3_BASE + 3, (32, 9, 14, 24, 3, 1)), (X3_BASE + 4, (20, 9, 14, 24, 3, 2)),
-         (X3_BASE + 0, (96, 10, 13, 132, 1, 1))]
+         (X3_BASE + 0, (96, 10, 13, 132, 1, 1)), (C3_BASE + 0, (64, 12, 20, 72, 3, 1)), (C3_BASE + 1, (48, 9, 14, 24, 3, 1)),
+         (C3_BASE + 4, (16, 9, 14, 40, 3, 1)), (C3_BASE + 0, (20, 17, 21, 24, 3, 2)), (C3_BASE + 3, (64, 12, 20, 40, 3, 2)),
+         (C3_BASE + 5, (64, 9, 14, 24, 3, 1)), (C3_BASE + 6, (60, 9, 14, 40, 3, 1)), (C3_BASE + 5, (64, 12, 20, 40, 3, 2))]
 RANGE_IDS = [f"{t}-" + "x".join(map(str, f)) for t, f in RANGE]
 
 
