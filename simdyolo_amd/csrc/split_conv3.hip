@@ -193,11 +193,28 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
       d[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, ch * (64 * G), 0));
     }
   };
+  // Weights run kRing taps ahead of their use, across groups and chunks (the
+  // last group loads its own first taps again): uniform base of the wave's
+  // channel blocks, 32-bit lane offset.
+  constexpr int kRing = 3;
+  f16x8 bv[kRing][TN][2];
+  const int wob = a.ng * (9 * 128 * 16);  // bytes per 32-channel block
+  const char* wbase = (const char*)a.w + (long long)ob0 * wob;
+  const unsigned wlane = lane * 16;
+  auto wload = [&](int g, int tap) __attribute__((always_inline)) {
+    const char* wg = wbase + min(g, a.ng - 1) * (9 * 128 * 16);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        bv[tap % kRing][j][p] = *(const f16x8*)(wg + (j * wob + (tap * 2 + p) * 1024) + wlane);
+  };
+
   // A chunk into LDS.  A pixel is below the scale's range if its channels of the
   // chunk are not all zero and none is in the pairs' full range (2^-13 or more,
   // scaled).  Few are: the first test is on any four channels of a thread.
   static_assert(L_IT <= 32, "a bit per staged pixel");
-  auto stage = [&](int ch, int se) __attribute__((always_inline)) {
+  auto stage = [&](int ch, int se, bool first) __attribute__((always_inline)) {
     const float s = exp_float(se);
     const unsigned range = (unsigned)(241 - se) << 23;  // bits of 2^-13 / s
     float m = 0.f;
@@ -221,6 +238,10 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
         *(u32x2*)(dst + 2 * G * PL) = lo;
       }
     }
+    if (first) {
+#pragma unroll
+      for (int t = 0; t < kRing; ++t) wload(wk, t);
+    }
     m = wave_max63(m);
     if (__builtin_expect(__any(least < range - 1), 0)) {
       unsigned full = 0, some = 0;  // a bit per pixel
@@ -235,23 +256,6 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
     }
     if (lane == 63) red[wid] = m;
   };
-  // Weights run kRing taps ahead of their use, across groups and chunks (the
-  // last group loads its own first taps again): uniform base of the wave's
-  // channel blocks, 32-bit lane offset.
-  constexpr int kRing = 3;
-  f16x8 bv[kRing][TN][2];
-  const int wob = a.ng * (9 * 128 * 16);  // bytes per 32-channel block
-  const char* wbase = (const char*)a.w + (long long)ob0 * wob;
-  const unsigned wlane = lane * 16;
-  auto wload = [&](int g, int tap) __attribute__((always_inline)) {
-    const char* wg = wbase + min(g, a.ng - 1) * (9 * 128 * 16);
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-        bv[tap % kRing][j][p] = *(const f16x8*)(wg + (j * wob + (tap * 2 + p) * 1024) + wlane);
-  };
-
   xload(0);
   // The epilogue's operands, loaded before they are waited for.
   const int col0 = ob0 * 32 + r32;
@@ -298,11 +302,7 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
   };
   // Chunk ch (loaded already) into LDS.
   auto enter = [&](int ch) __attribute__((always_inline)) {
-    stage(ch, se);
-    if (ch == 0) {
-#pragma unroll
-      for (int t = 0; t < kRing; ++t) wload(wk, t);
-    }
+    stage(ch, se, ch == 0);
     __syncthreads();
     int l = maxima(), ne;
     if (!scale_fits(big, se, &ne)) {  // rare: the chunk again with another scale
@@ -310,7 +310,7 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
       se = ne;
       xload(ch);
       __syncthreads();  // every wave has read the maxima
-      stage(ch, se);
+      stage(ch, se, false);
       __syncthreads();
       l = maxima();
     }
