@@ -2702,17 +2702,18 @@ static int auto_algo(const ConvPlan* p) {
   return -1;
 }
 
-// Packs (once) the device weights the given algorithm reads.
+// Whether the device weights the given algorithm reads are there.
+static bool weights_packed(const ConvPlan* p, int algo, int tile) {
+  if (algo == kIgemm) return (is_x3_tile(tile) ? p->w_x3 : is_c3_tile(tile) ? p->w_c3 : p->w_gemm) != nullptr;
+  if (algo == kDirect) return p->w_direct != nullptr;
+  if (algo == kDepthwise) return p->w_dw != nullptr;
+  return (algo == kWinograd2 || algo == kWinograd ? p->w_wino_b : p->w_wino) != nullptr;
+}
+
+// Packs them (once).
 static int pack_weights(sy_ctx* ctx, ConvPlan* p, int algo, int tile) {
   const bool x3 = algo == kIgemm && is_x3_tile(tile), c3 = algo == kIgemm && is_c3_tile(tile);
-  SY_CHECK(!ctx->capturing || (x3 ? p->w_x3 != nullptr
-                               : c3 ? p->w_c3 != nullptr
-                               : algo == kIgemm ? p->w_gemm != nullptr
-                               : algo == kDirect ? p->w_direct != nullptr
-                               : algo == kDepthwise ? p->w_dw != nullptr
-                               : algo == kWinograd2 || algo == kWinograd ? p->w_wino_b != nullptr
-                                                                          : p->w_wino != nullptr),
-           SY_ESTATE, "weight packing during graph capture");
+  SY_CHECK(!ctx->capturing || weights_packed(p, algo, tile), SY_ESTATE, "weight packing during graph capture");
   const int oc = p->oc, ic = p->ic, kh = p->kh, kw = p->kw;
   const float* W = p->host_w.data();
   if ((x3 && !p->w_x3) || (c3 && !p->w_c3)) {
@@ -3457,7 +3458,10 @@ int conv_run(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tensor* y, c
           if (c.algo == rec->second.algo && c.tile == rec->second.tile && c.split == rec->second.split)
             reused = true;
       }
-      if (reused) {
+      if (reused && ctx->capturing && !weights_packed(p, rec->second.algo, rec->second.tile)) {
+        // A first run inside a capture, which cannot upload: the routing rule,
+        // whose weights are there from the start, for this call alone.
+      } else if (reused) {
         ch = rec->second;
         p->tuned[key] = ch;
       } else if (!ctx->capturing) {

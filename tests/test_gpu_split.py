@@ -417,3 +417,43 @@ def test_gemm_general_geometry(hip, monkeypatch, tile, form):
     finally:
         hip.end_frame()
     near(got, exp, mag)
+
+
+# (n, ic, h, w, oc, k, stride): sizes that only the split kernels are timed at.
+@pytest.mark.parametrize("form", [(8, 36, 76, 80, 32, 1, 1), (8, 36, 150, 146, 40, 3, 2)], ids=["1x1", "3x3s2"])
+def test_capture_with_the_choice_of_another_conv(hip, form):
+    """A convolution that runs first inside a capture, of a shape that another
+    one tuned: its split weights are not packed yet, and packing uploads."""
+    n, ic, h, w, oc, k, s = form
+    x, wt, b = data(n, ic, h, w, oc, k, 1400)
+    w2 = synth.kaiming((oc, ic, k, k), 1410)
+    xs = [x] + [synth.activations(x.shape, 1411 + i) for i in range(2)]
+    hip.begin_frame()
+    try:
+        first, second = (hip.conv_create(t, b, (s, s), (k // 2,) * 4) for t in (wt, w2))
+        xv = hip.upload(x)
+        yv = hip.alloc(n, oc, *hip.conv_out_size(first, h, w))
+        hip.conv(first, xv, yv)
+        near(hip.download(yv), *conv64(x, wt, b, s, False, None))
+        hip.graph_begin()
+        try:
+            hip.conv(second, xv, yv)
+        finally:
+            g = hip.graph_end()
+        for x in xs:
+            hip.upload(x, xv)
+            hip.graph_launch(g)
+            near(hip.download(yv), *conv64(x, w2, b, s, False, None))
+        # Outside the capture it takes the recorded choice.
+        hip.profile_enable(True)
+        hip.profile_read()
+        try:
+            hip.conv(second, xv, yv)
+            hip.flush()
+            names = set(hip.profile_read())
+        finally:
+            hip.profile_enable(False)
+        assert all("_x3_" in name for name in names), names
+        near(hip.download(yv), *conv64(xs[-1], w2, b, s, False, None))
+    finally:
+        hip.end_frame()
