@@ -3219,10 +3219,18 @@ static std::string tune_key(const ConvPlan* p, const sy_tensor* x, const sy_tens
   return k;
 }
 
+// What the tile numbers of a saved table mean: the form lists' sizes and bases.
+static std::string tune_header() {
+  char h[80];
+  snprintf(h, sizeof h, "simdyolo_hip tune3 %d %d %d %d %d %d", kNumTiles, kPwBase, kX3Base, x3_num_tiles(), kC3Base,
+           c3_num_forms());
+  return h;
+}
+
 int tune_save(const sy_ctx* ctx, const char* path) {
   FILE* f = fopen(path, "w");
   SY_CHECK(f != nullptr, SY_EINVAL, "cannot open %s for writing", path);
-  fprintf(f, "simdyolo_hip tune2 %d %d\n", kNumTiles, kPwBase);
+  fprintf(f, "%s\n", tune_header().c_str());
   for (const auto& kv : ctx->tune_table)
     fprintf(f, "%s %d %d %d\n", kv.first.c_str(), kv.second.algo, kv.second.tile, kv.second.split);
   const bool ok = fclose(f) == 0;
@@ -3233,9 +3241,10 @@ int tune_save(const sy_ctx* ctx, const char* path) {
 int tune_load(sy_ctx* ctx, const char* path) {
   FILE* f = fopen(path, "r");
   SY_CHECK(f != nullptr, SY_EINVAL, "cannot open %s", path);
-  int nt = -1, pb = -1;
-  const bool head = fscanf(f, "simdyolo_hip tune2 %d %d", &nt, &pb) == 2;
-  if (!head || nt != kNumTiles || pb != kPwBase) {
+  char line[128] = "";
+  const bool head = fgets(line, sizeof line, f) != nullptr;
+  line[strcspn(line, "\r\n")] = 0;
+  if (!head || line != tune_header()) {
     fclose(f);
     SY_CHECK(false, SY_EINVAL, "%s is not a tuning table of this library build", path);
   }

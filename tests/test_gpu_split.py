@@ -12,7 +12,7 @@ that largest instead.
 import numpy as np
 import pytest
 
-from simdyolo_amd import CONV_IGEMM, synth
+from simdyolo_amd import CONV_IGEMM, SyError, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -457,3 +457,20 @@ def test_capture_with_the_choice_of_another_conv(hip, form):
         near(hip.download(yv), *conv64(xs[-1], w2, b, s, False, None))
     finally:
         hip.end_frame()
+
+
+def test_tuning_tables_of_other_forms_are_refused(hip, tmp_path):
+    """A saved table numbers the kernels: one whose lists were of another
+    length, or from before the split kernels, would name others."""
+    table, other = tmp_path / "table.txt", tmp_path / "other.txt"
+    hip.tune_save(str(table))
+    hip.tune_load(str(table))
+    head, *rows = table.read_text().splitlines()
+    kind, fields = head.split()[:2], head.split()[2:]
+    changed = [kind + fields[:i] + [str(int(fields[i]) + 1)] + fields[i + 1:] for i in range(len(fields))]
+    for old in changed + [[kind[0], "tune2"] + fields[:2]]:
+        other.write_text("\n".join([" ".join(old)] + rows) + "\n")
+        with pytest.raises(SyError):
+            hip.tune_load(str(other))
+    other.write_text("\r\n".join([head] + rows) + "\r\n")
+    hip.tune_load(str(other))
