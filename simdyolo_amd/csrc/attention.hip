@@ -7,9 +7,10 @@
 // (VulkanExecution.cs:499-541, tensor.comp:62-68).
 //
 // Key dims up to 32 and head dims up to 64 (every YOLO11 / YOLO26 block: 32 and
-// 64) run in one kernel that keeps the scores in registers.  Other geometries
-// run both products on the FP32-MFMA GEMM (gemm_nt); S rows and V^T rows are
-// padded to N4 = round_up(N, 4) with zeros so K stays a multiple of 4.
+// 64) run in one kernel that keeps the scores in registers.  Other geometries,
+// and outputs that overlap the input or each other, run both products on the
+// FP32-MFMA GEMM (gemm_nt); S rows and V^T rows are padded to N4 = round_up(N, 4)
+// with zeros so K stays a multiple of 4.
 #include <cfloat>
 #include <cmath>
 
@@ -320,10 +321,12 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const AttnArgs a) {
   }
 }
 
-// The fused kernel's geometries: operands in its 32-channel steps, row offsets
-// within an image in 32 bits.
-static bool attention_fused(const sy_tensor* qkv, int kd, int hd) {
-  return kd <= 32 && hd <= 64 && (long long)qkv->h * qkv->w * qkv->ldc < (1LL << 31);
+// What the fused kernel takes: operands in its 32-channel steps, row offsets
+// within an image in 32 bits, outputs of their own (its workgroups write them
+// while others still read qkv; the GEMMs copy v and form all scores first).
+static bool attention_fused(const sy_tensor* qkv, int kd, int hd, const sy_tensor* o, const sy_tensor* v) {
+  return kd <= 32 && hd <= 64 && (long long)qkv->h * qkv->w * qkv->ldc < (1LL << 31) && !views_overlap(o, qkv) &&
+         !views_overlap(v, qkv) && !views_overlap(o, v);
 }
 
 // One wavefront per row: y = softmax(x * scale) over n entries (max-subtracted),
@@ -390,7 +393,7 @@ int op_attention(sy_ctx* ctx, const sy_tensor* qkv, int heads, int kd, int hd, f
            "attention needs key/head dims that are multiples of 4");
   SY_CHECK(((uintptr_t)qkv->data & 15) == 0 && qkv->ldc % 4 == 0, SY_EINVAL,
            "attention qkv view must be 16-byte aligned with ldc %% 4 == 0");
-  if (attention_fused(qkv, kd, hd)) {
+  if (attention_fused(qkv, kd, hd, o, v)) {
     AttnArgs a{qkv->data, qkv->ldc, N, heads, kd, hd, (N + 31) / 32, scale, o->data, o->ldc, v->data, v->ldc};
     const long long grid = (long long)B * heads * a.qtiles;
     SY_CHECK(grid < (1LL << 31), SY_EUNSUPPORTED, "attention grid too large");

@@ -3422,8 +3422,7 @@ static int conv_tune(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tens
   return SY_OK;
 }
 
-// Byte ranges of two views intersect (dense NCHW or strided NHWC).
-static bool views_overlap(const sy_tensor* a, const sy_tensor* b) {
+bool views_overlap(const sy_tensor* a, const sy_tensor* b) {
   auto span = [](const sy_tensor* t) {
     const size_t px = (size_t)t->n * t->h * t->w;
     const size_t floats = t->layout == SY_LAYOUT_NCHW ? px * t->c : (px - 1) * t->ldc + t->c;

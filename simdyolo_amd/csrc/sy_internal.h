@@ -242,6 +242,8 @@ struct ConvPlan {
 int conv_prepare(sy_ctx* ctx, ConvPlan* p);
 bool conv_supports(const ConvPlan* p, int algo);
 int conv_run(sy_ctx* ctx, ConvPlan* p, const sy_tensor* x, const sy_tensor* y, const sy_tensor* res);
+// Two views share memory (dense NCHW or strided NHWC; true where in doubt).
+bool views_overlap(const sy_tensor* a, const sy_tensor* b);
 // A 1x1 conv whose input x is concat(upsample2x(xu), rest): channels
 // [0, xu->c) of x are the 2x nearest upsample of xu and need not be written;
 // the GEMM reads them from xu at half resolution.  Shapes the kernel cannot

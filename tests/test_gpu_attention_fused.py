@@ -155,6 +155,26 @@ def test_large_scores(hip, sign, step):
     assert np.isfinite(got).all() and (err <= 2.0 ** -18 * mag).all(), (err / mag).max()
 
 
+@pytest.mark.parametrize("where", ["o in qkv", "o in v"])
+def test_output_over_an_operand(hip, where):
+    """The output over the query channels of its own input, or over v's copy, is written after all reads."""
+    heads, kd, hd = 2, 32, 32
+    c = heads * (2 * kd + hd)
+    qkv = synth.activations((2, c, 9, 40), 12)
+    exp, bound, _ = reference(qkv, heads, kd, hd, np.float32(kd ** -0.5))
+    hip.begin_frame()
+    try:
+        x, v = hip.alloc(2, c, 9, 40), hip.alloc(2, heads * hd, 9, 40)
+        o = x.slice(0, heads * hd) if where == "o in qkv" else v
+        for _ in range(2):
+            hip.upload(qkv, x)
+            hip.attention(x, heads, kd, hd, float(np.float32(kd ** -0.5)), o, v)
+            got = hip.download(o)
+            assert (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
+    finally:
+        hip.end_frame()
+
+
 RANGES = {
     # One query 2^29 times the others', whose own scores are of order 1.
     "queries": lambda q, k, v: (np.where(np.arange(96) == 5, 3e4, 2.0 ** -14) * q, 2.0 ** 14 * k, v),
