@@ -26,12 +26,14 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3  # MI355X dense FP32 matrix
 PEAK_SPLIT_TFLOPS = 2500.0 / 3  # dense f16 matrix over the three products of a split float32 one
+PEAK_PARTS_TFLOPS = 2500.0 / 6  # dense bf16 matrix over the six of a float32 one in three parts
 PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 RIDGE = PEAK_FP32_MFMA_TFLOPS * 1e12 / (PEAK_HBM_GBS * 1e9)  # FLOP/B
 METRIC = "images/s YOLOv8n 640\u00b2 FP32 bs1/bs32; % FP32-MFMA peak & % HBM peak per kernel"
 # HBM bytes per launch from the rocprofv3 FETCH_SIZE / WRITE_SIZE passes,
-# scaled by the plain-copy calibration (see the file's header).
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_yolov8n_640_b32.txt")
+# scaled by the plain-copy calibration (see the files' headers): the float32
+# kernels', then the split kernels', which count where both name a kernel.
+TRAFFIC_FILES = [os.path.join(ROOT, "profiles", f"hbm_traffic{kind}_yolov8n_640_b32.txt") for kind in ("", "_split")]
 
 # Library profile names -> the kernel symbols rocprofv3 reports.
 SYMBOLS = {"wino_input": "sy::wino_in_kernel<4>", "wino_input_blk": "sy::wino_in_blk_kernel",
@@ -58,7 +60,8 @@ SYMBOLS = {"wino_input": "sy::wino_in_kernel<4>", "wino_input_blk": "sy::wino_in
 def symbol(name):
     """rocprofv3 symbol of a library profile name: igemm_m<mode>_<bm>x<bn>_<wm><wn>_k<bk>[_p<pf>] or
     wino_gemm_<bm>x<bn>_<wm><wn>_k<bk>[_p<pf>] (pf: K tiles loaded ahead, 1 when absent),
-    igemm_m<mode>_x3_<bm>x<bn>_<wm><wn> and conv3_x3_<pixels>x<channels>_<waves> (f16-split kernels),
+    igemm_m<mode>_x3_<bm>x<bn>_<wm><wn> and conv3_x3_<bm>x<bn>_<wm><wn>[_ks<waves per block>] (f16-split
+    kernels; the latter's stride, chunk and single-chunk template arguments depend on the layer, written *),
     pw_gemm_n<32*NW> / wino_pw_n<32*NW> (the K-chunk template argument depends on the layer,
     written *), or a fixed kernel."""
     m = re.fullmatch(r"(igemm_m(\d)|wino_gemm)_(\d+)x(\d+)_(\d)(\d)_k(\d+)(?:_p(\d))?", name)
@@ -70,8 +73,10 @@ def symbol(name):
     m = re.fullmatch(r"igemm_m(\d)_x3_(\d+)x(\d+)_(\d)(\d)", name)
     if m:
         return "sy::x3_kernel<" + ", ".join(m.groups()) + ">"
-    if name.startswith("conv3_x3_"):
-        return "sy::conv3_kernel<*>"
+    m = re.fullmatch(r"conv3_x3_(\d+)x(\d+)_(\d)(\d)(?:_ks(\d))?", name)
+    if m:
+        bm, bn, wm, wn, kw = (int(g or 1) for g in m.groups())
+        return f"sy::conv3_kernel<*, *, {wm}, {wn}, {bm // 32 // wm}, {bn // 32 // wn}, {kw}, *>"
     m = re.fullmatch(r"(pw_gemm|wino_pw)_n(\d+)", name)
     if m:
         return f"sy::pw_kernel<{int(m.group(2)) // 32}, *>"
@@ -79,8 +84,11 @@ def symbol(name):
 
 
 def matrix_peak(name):
-    """TFLOP/s that a kernel's float32-equivalent products can reach: f16 triples or float32 matrix cores."""
-    return PEAK_SPLIT_TFLOPS if "_x3_" in name or name == "attention" else PEAK_FP32_MFMA_TFLOPS
+    """TFLOP/s that a kernel's float32-equivalent products can reach: f16 triples, bf16 sextuples or float32
+    matrix cores."""
+    if name == "attention":
+        return PEAK_PARTS_TFLOPS
+    return PEAK_SPLIT_TFLOPS if "_x3_" in name else PEAK_FP32_MFMA_TFLOPS
 
 
 def log(msg):
@@ -105,18 +113,17 @@ def kernel_table(prof, steps):
 
 
 def load_traffic():
-    """{profile name: HBM bytes per launch} from the committed PMC summary."""
+    """{profile name: HBM bytes per launch} from the committed PMC summaries."""
     out = {}
-    if not os.path.exists(TRAFFIC_FILE):
-        return out
-    with open(TRAFFIC_FILE) as f:
-        for line in f:
-            parts = line.split()
-            if len(parts) >= 2 and not line.startswith("#") and symbol(parts[0]):
-                try:
-                    out[parts[0]] = float(parts[-1])
-                except ValueError:
-                    pass
+    for path in filter(os.path.exists, TRAFFIC_FILES):
+        with open(path) as f:
+            for line in f:
+                parts = line.split()
+                if len(parts) >= 2 and not line.startswith("#") and symbol(parts[0]):
+                    try:
+                        out[parts[0]] = float(parts[-1])
+                    except ValueError:
+                        pass
     return out
 
 
@@ -376,8 +383,9 @@ def main():
         "timing": f"median of {args.windows} windows of {args.steps} graph replays, HIP events on the library "
                   f"stream; inputs resident in HBM",
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp32", "arithmetic": "float32 in and out; most convolutions and the attention multiply each "
-                                       "float32 as a scaled f16 pair (three matrix products, float32 sums)",
+        "dtype": "fp32", "arithmetic": "float32 in and out; most convolutions multiply each float32 as a scaled f16 "
+                                       "pair (three matrix products, float32 sums; plain float32 where a pixel is "
+                                       "out of the pairs' range)",
         "data": "synthetic (seeded random-init YOLOv8 weights, uniform u8 pixels / 255)",
         "config": {"workload": f"YOLOv8{args.scale} detect forward {S}x{S}, batch {B}, "
                                f"{'eager launches' if args.eager else 'hipGraph replay'}",

@@ -5,7 +5,7 @@ Segment models) and the post-processing kernels (end-to-end top-k, mask
 decode, NMS candidates, device letterbox).  All inputs are synthetic and
 seeded; every figure is HIP-event time on the library stream.
 
-    python bench_suite.py --section layers|models|post|bandwidth|route
+    python bench_suite.py --section layers|models|post|bandwidth|route|gemm1x1|split
     rocprofv3 --kernel-trace --output-format csv -d DIR -o bw -- python bench_suite.py --section bandwidth > LOG
     python bench_suite.py --trace DIR/bw_kernel_trace.csv LOG
     rocprofv3 --kernel-trace --output-format csv -d DIR -o kt -- python bench.py --eager ... > BENCH_LOG
@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import argparse
 import ctypes
+import fnmatch
 import os
 import sys
 
@@ -522,7 +523,7 @@ def summarize_trace(trace_csv, log):
             else:
                 for lib_name, (_, b) in case["kernels"].items():
                     sym = symbol(lib_name)
-                    if sym and (sym == k or ("*" in sym and k.startswith(sym.split("<")[0]))):
+                    if sym and fnmatch.fnmatchcase(k, sym):
                         nbytes = b
             med = statistics.median(d)
             line = f"    {k:<56} {len(d) // reps:8d} {med:10.2f}"
@@ -530,6 +531,12 @@ def summarize_trace(trace_csv, log):
                 gbs = nbytes / (med * 1e-6) / 1e9
                 line += f" {nbytes / 1e6:9.2f} {gbs:8.0f} {100 * gbs / PEAK_HBM_GBS:9.1f}%"
             out(line)
+
+
+def join_symbol(kernel, symbols):
+    """The symbol of `symbols` (with * for template arguments that a profile name leaves open) that names this
+    kernel, else the kernel itself: the kernels of one profile name count together, as in the bench's rows."""
+    return next((s for s in symbols if fnmatch.fnmatchcase(kernel, s)), kernel)
 
 
 def summarize_forward_trace(trace_csv, steps, bench_log):
@@ -548,9 +555,6 @@ def summarize_forward_trace(trace_csv, steps, bench_log):
     if len(ends) <= steps:
         raise SystemExit(f"the trace holds {len(ends)} forwards, fewer than {steps} + 1")
     seg = rows[ends[-steps - 1] + 1:ends[-1] + 1]
-    agg = collections.defaultdict(list)
-    for r in seg:
-        agg[name(r)].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
     bench = {}
     with open(bench_log) as f:
         for line in f:
@@ -559,6 +563,9 @@ def summarize_forward_trace(trace_csv, steps, bench_log):
                     sym = symbol(k["kernel"])
                     if sym:
                         bench[sym] = (k["avg_launch_us"], k["kernel"])
+    agg = collections.defaultdict(list)
+    for r in seg:
+        agg[join_symbol(name(r), bench)].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
     total = sum(sum(v) for v in agg.values()) / steps
     out(f"# {steps} steady-state forwards of eager launches; total kernel time per forward {total / 1e3:.3f} ms")
     out(f"# {'symbol':<52} {'calls/step':>10} {'ms/step':>8} {'avg us':>8} {'share %':>8} {'bench avg us':>13}"
@@ -604,8 +611,16 @@ def _bench_kernels(bench_log):
             if line.startswith("{") and '"kernels"' in line:
                 for k in json.loads(line)["kernels"]:
                     sym = symbol(k["kernel"])
-                    if sym and "*" not in sym:
+                    if sym:
                         out_[sym] = (k["kernel"], k["flops_per_launch"], k["bytes_per_launch"])
+    return out_
+
+
+def _joined(counter, algo):
+    """The counter's values with the kernels of one profile name together."""
+    out_ = {}
+    for kernel, vals in counter.items():
+        out_.setdefault(join_symbol(kernel, algo), []).extend(vals)
     return out_
 
 
@@ -641,7 +656,7 @@ def summarize_pmc_traffic(fetch_csv, write_csv, bench_log):
     out("#")
     out(f"# {'kernel (bench name or symbol)':<38} {'dispatches':>10} {'FETCH KiB':>12} {'WRITE KiB':>12} "
         f"{'algo_bytes':>14} {'ratio':>6} {'hbm_bytes':>14}")
-    fd, wd = fwd_f["FETCH_SIZE"], fwd_w["WRITE_SIZE"]
+    fd, wd = _joined(fwd_f["FETCH_SIZE"], algo), _joined(fwd_w["WRITE_SIZE"], algo)
     rows = []
     for sym, vals in fd.items():
         f = sum(vals) / len(vals)
@@ -659,18 +674,23 @@ def summarize_pmc_traffic(fetch_csv, write_csv, bench_log):
 
 def summarize_pmc_mfma(mfma_csv, bench_log):
     """MFMA work, matrix-pipe busy fraction and achieved rate per kernel from
-    SQ_INSTS_VALU_MFMA_MOPS_F32, SQ_VALU_MFMA_BUSY_CYCLES and GRBM_GUI_ACTIVE."""
+    SQ_INSTS_VALU_MFMA_MOPS_F32 (and _F16, _BF16), SQ_VALU_MFMA_BUSY_CYCLES and GRBM_GUI_ACTIVE."""
     fwd, _, nf = _pmc_forwards(mfma_csv)
     algo = _bench_kernels(bench_log)
-    mops, busy, act = fwd["SQ_INSTS_VALU_MFMA_MOPS_F32"], fwd["SQ_VALU_MFMA_BUSY_CYCLES"], fwd["GRBM_GUI_ACTIVE"]
-    sqb = fwd.get("SQ_BUSY_CYCLES", {})
+    busy, act = _joined(fwd["SQ_VALU_MFMA_BUSY_CYCLES"], algo), _joined(fwd["GRBM_GUI_ACTIVE"], algo)
+    sqb = _joined(fwd.get("SQ_BUSY_CYCLES", {}), algo)
+    mops = {}
+    for kind in ("F32", "F16", "BF16"):
+        for sym, v in _joined(fwd.get("SQ_INSTS_VALU_MFMA_MOPS_" + kind, {}), algo).items():
+            mops[sym] = [x + y for x, y in zip(mops.get(sym, [0.0] * len(v)), v)]
     out(f"# {nf} forward passes after the first; per launch averages.")
-    out("# executed_GF = SQ_INSTS_VALU_MFMA_MOPS_F32 * 512 FLOP (MFMA work including tile padding);")
+    out("# executed_GF = SQ_INSTS_VALU_MFMA_MOPS_F32 + _F16 + _BF16, * 512 FLOP (MFMA work including tile padding;")
+    out("#   three f16 products for each float32 one in the _x3_ kernels);")
     out("# algo_GF = the library's algorithmic FLOPs per launch (unpadded), from the bench's eager pass;")
     out("# active_us = GRBM_GUI_ACTIVE / 8 XCDs / 2.4 GHz (the counter sums the 8 XCDs; under counter collection);")
     out("# mfma_busy = SQ_VALU_MFMA_BUSY_CYCLES / (GRBM_GUI_ACTIVE / 8 * 256 CUs * 4 SIMDs): the fraction of")
     out("#   SIMD-cycles the matrix pipe was busy while the kernel ran (one v_mfma_f32_32x32x2f32 = 64 busy cycles);")
-    out("# achieved = algo_GF / active_us, frac = achieved / 157.3 TFLOP/s (MI355X dense FP32 matrix).")
+    out("# achieved = algo_GF / active_us, frac = achieved / 157.3 TFLOP/s (MI355X dense FP32 matrix; _x3_: 2,500 / 3).")
     out("# sq_busy = SQ_BUSY_CYCLES / GRBM_GUI_ACTIVE, each summed over its hardware instances as the counter")
     out("#   reports it: the sequencers' busy share while the kernel ran, in units of GRBM instances.")
     out("#")
@@ -748,9 +768,72 @@ def section_gemm1x1():
             f" | " + ", ".join(f"t{tt} {u:.1f}" for u, tt in res[1:7]))
 
 
+def section_split():
+    """The tuner's cut: at grids of 512 and more 64 x 64 output tiles, K >= 64
+    and 32 input channels it times the f16-split kernels alone.  Here every
+    float32 form runs beside them on the layers of YOLOv8n, s and m at 640."""
+    from simdyolo_amd import synth, CONV_IGEMM, CONV_WINOGRAD, CONV_WINOGRAD2, CONV_WINOGRAD3, SyError
+    from simdyolo_amd.device import HipContext
+    hip = HipContext(0)
+    out(f"# device: {hip.name}")
+    out("# bias + SiLU; each candidate forced, HIP-event average of 10 back-to-back calls after 2 warm ones, best of two.")
+    out(f"# {'layer':<34} {'split us':>9} {'':<22} {'float32 us':>10} {'':<22} {'ratio':>6}")
+    ones = [(32, 32, 160), (48, 32, 160), (64, 64, 160), (96, 64, 160), (96, 96, 160), (192, 96, 160), (64, 64, 80),
+            (128, 64, 80), (192, 64, 80), (64, 80, 80), (80, 80, 80), (128, 128, 80), (384, 128, 80), (192, 192, 80),
+            (128, 128, 40), (192, 128, 40), (256, 128, 40), (384, 128, 40), (256, 256, 40), (576, 384, 40),
+            (256, 256, 20), (384, 256, 20), (512, 512, 20), (576, 576, 20)]
+    threes = [(32, 32, 160), (48, 48, 160), (32, 32, 80), (64, 64, 80), (64, 80, 80), (80, 80, 80), (96, 96, 80),
+              (128, 128, 80), (64, 64, 40), (128, 64, 40), (128, 128, 40), (192, 192, 40), (128, 128, 20),
+              (256, 64, 20), (256, 256, 20)]
+    downs = [(32, 64, 160), (48, 96, 160), (64, 128, 160), (64, 64, 80), (64, 128, 80), (96, 192, 80), (128, 256, 80),
+             (128, 128, 40), (128, 256, 40), (192, 384, 40)]
+    for batch in (1, 4, 8, 32):
+        for k, s, shapes in ((1, 1, ones), (3, 1, threes), (3, 2, downs)):
+            for ic, oc, hw in shapes:
+                px = batch * (hw // s) ** 2
+                if (px + 63) // 64 * ((oc + 63) // 64) < 512:
+                    continue
+                hip.begin_frame()
+                try:
+                    conv = hip.conv_create(synth.kaiming((oc, ic, k, k), 2), synth.activations((oc,), 3), (s, s),
+                                           (k // 2,) * 4, silu=True)
+                    x = hip.upload(synth.activations((batch, ic, hw, hw), 1))
+                    y = hip.alloc(batch, oc, hw // s, hw // s)
+                    best = {}
+                    cands = [(CONV_IGEMM, t) for t in [*range(24), *range(32, 36), *range(64, 69), *range(96, 103)]]
+                    if k == 3 and s == 1:
+                        cands += [(CONV_WINOGRAD, t) for t in range(3)] + [(CONV_WINOGRAD2, t) for t in range(2)]
+                        cands += [(CONV_WINOGRAD3, t) for t in [*range(24), *range(32, 36)]]
+                    for algo, t in cands:
+                        if k == 1 and (t >= 96) or k == 3 and algo == CONV_IGEMM and 32 <= t < 36:
+                            continue
+                        os.environ["SIMDYOLO_HIP_TILE"] = str(t)
+                        try:
+                            hip.conv_set_algo(conv, algo)
+                            for _ in range(2):
+                                hip.conv(conv, x, y)
+                        except SyError:
+                            continue  # a form that does not take this shape
+                        us = []
+                        for _ in range(2):
+                            hip.timer_start()
+                            for _ in range(10):
+                                hip.conv(conv, x, y)
+                            us.append(hip.timer_stop() * 100)
+                        side = "split" if algo == CONV_IGEMM and t >= 64 else "float32"
+                        best[side] = min(best.get(side, (1e30,)), (min(us), f"algo {algo} tile {t}"))
+                    os.environ.pop("SIMDYOLO_HIP_TILE")
+                finally:
+                    hip.end_frame()
+                a, b = best["split"], best["float32"]
+                out(f"{k}x{k} s{s} {ic:>3} -> {oc:<3} @{hw:<3} batch {batch:<2}{'':<8} {a[0]:9.1f} {a[1]:<22} {b[0]:10.1f} "
+                    f"{b[1]:<22} {b[0] / a[0]:6.2f}")
+    hip.close()
+
+
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--section", choices=["layers", "models", "post", "bandwidth", "route", "gemm1x1"])
+    ap.add_argument("--section", choices=["layers", "models", "post", "bandwidth", "route", "gemm1x1", "split"])
     ap.add_argument("--trace", nargs=2, metavar=("KERNEL_TRACE_CSV", "BANDWIDTH_LOG"),
                     help="summarise a rocprofv3 kernel trace of a --section bandwidth run")
     ap.add_argument("--forward-trace", nargs=3, metavar=("KERNEL_TRACE_CSV", "STEPS", "BENCH_LOG"),
@@ -774,7 +857,7 @@ def main():
         summarize_forward_trace(csv_path, int(steps), log)
         return
     {"layers": section_layers, "models": section_models, "post": section_post,
-     "bandwidth": section_bandwidth, "route": section_route, "gemm1x1": section_gemm1x1}[args.section]()
+     "bandwidth": section_bandwidth, "route": section_route, "gemm1x1": section_gemm1x1, "split": section_split}[args.section]()
 
 
 if __name__ == "__main__":

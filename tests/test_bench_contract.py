@@ -56,3 +56,19 @@ def test_committed_profiles_cover_the_roofline_kernel():
         trace = f.read()
     assert bench.symbol("wino_gemm_out") in trace
     assert "rocprofv3 --kernel-trace --stats" in trace
+
+
+def test_split_kernels_join_their_symbols():
+    """Profile names of the f16-split kernels against rocprofv3's symbols: a patch kernel's name leaves template
+    arguments open, and its variants count together."""
+    import bench_suite
+    assert bench.symbol("igemm_m2_x3_64x128_22") == "sy::x3_kernel<2, 64, 128, 2, 2>"
+    wide, split = bench.symbol("conv3_x3_128x64_22"), bench.symbol("conv3_x3_32x32_11_ks8")
+    assert wide == "sy::conv3_kernel<*, *, 2, 2, 2, 1, 1, *>" and split == "sy::conv3_kernel<*, *, 1, 1, 1, 1, 8, *>"
+    assert bench.symbol("conv3_x3_64x96_23") == "sy::conv3_kernel<*, *, 2, 3, 1, 1, 1, *>"
+    for kernel in ("sy::conv3_kernel<1, 4, 2, 2, 2, 1, 1, true>", "sy::conv3_kernel<2, 2, 2, 2, 2, 1, 1, false>"):
+        assert bench_suite.join_symbol(kernel, [split, wide]) == wide
+    other = "sy::conv3_kernel<1, 4, 2, 2, 1, 1, 1, true>"
+    assert bench_suite.join_symbol(other, [split, wide]) == other
+    assert bench.matrix_peak("conv3_x3_128x64_22") == pytest.approx(2500.0 / 3)
+    assert bench.matrix_peak("attention") == pytest.approx(2500.0 / 6)
