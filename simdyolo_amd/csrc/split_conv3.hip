@@ -16,18 +16,19 @@
 // but all below the pairs' full range, computes its tile again in plain float32, at
 // about the speed of the float32 tiles: an element's error is at most 2^-23 of its
 // pixel's largest of the chunk, whatever the other pixels hold.  The test costs two
-// operations per four values: 80 -> 80 at 80 x 80, batch 32, 103.2 -> 104.8 us,
-// 64 -> 64 52.2 -> 52.4, 64 -> 128 stride 2 39.5 -> 39.7, 80 -> 80 at 45 x 75, batch
-// 4, 11.0 -> 11.4.  Bits kept per pixel for all chunks took up to 10% (spills).
+// operations per four values: 80 -> 80 at 80 x 80, batch 32, 98.7 -> 100.5 us, at
+// 45 x 75, batch 4, 10.5 -> 10.7, 64 -> 64 at 40 x 40, batch 1, 5.0 -> 5.1, at 80 x 80,
+// batch 32, 53.8 -> 53.6.  Bits kept per pixel for all chunks took up to 10% (spills).
 //
 // A wave owns TM 32-pixel blocks x TN 32-channel blocks.  Per (tap, 16
 // channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
 // MFMAs of 32 cycles.
 //
-// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 51 us,
-// against 73 us for the fastest float32 Winograd form.  The matrix cores are
-// busy for 46% of it at the 1.8 GHz the GPU holds under this load; the patch
-// loads (8,000 of a 128-pixel workgroup's 29,000 cycles), the epilogue (6,000)
+// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 54 us on
+// normal random inputs (44 on smaller ones: the clock follows the power), against
+// 73 us for the fastest float32 Winograd form.  The matrix cores are busy for 38%
+// of its cycles (SQ_VALU_MFMA_BUSY_CYCLES over GRBM_GUI_ACTIVE); the patch loads
+// (8,000 of a 128-pixel workgroup's 29,000 cycles), the epilogue (6,000)
 // and a thin last round of 1,600 workgroups on 256 CUs take the rest.
 // Workgroups that run through several tiles with the next patch loaded behind
 // the last taps measured the same, 16-channel double buffering 57 - 60 us.
@@ -372,9 +373,11 @@ __global__ __launch_bounds__(WM* WN * KW * 64, c3_waves(S, G, WM * WN, TM * TN, 
 
   const int* po = opix + wm * TM * 32;
   if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)(big >= kSplitHuge)) || low < 0, 0)) {
+    // Lane and arguments read anew: the rare path keeps no register of the main one.
     int l = lane;
-    asm volatile("" : "+v"(l));  // its addresses are not kept from the main loop's
-    c3_plain<TM, TN>(a, po, ob0, wk, KW, l, acc);
+    auto p = (const __attribute__((address_space(4))) C3Args*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+v"(l), "+s"(p));
+    c3_plain<TM, TN>(*(const C3Args*)p, po, ob0, wk, KW, l, acc);
   } else {
     unscale<TM, TN>(ws, se, acc, crs);
   }
