@@ -16,6 +16,21 @@
  * input (dense NCHW, layout = SY_LAYOUT_NCHW) and the joined head output
  * ([B, nc+4, anchors], channels first) keep the reference's layouts.
  *
+ * Precision.  Inputs, outputs and sums are float32.  Most tuned convolutions
+ * multiply on the f16 matrix cores, each operand as a pair of f16 values under
+ * a common power of two: an input within 2^-23 of the largest magnitude of its
+ * pixel (1x1 and strided forms: of its GEMM row; 3x3: of the chunk of 16 to 128
+ * channels that holds it), a weight within 2^-23 of itself, or 2^-47 of its
+ * output channel's largest where that is more, and the product of the two low
+ * halves left out.  Tiles with values of 65,536 and more, or with pixels too
+ * small for the tile's scale, and convolutions with non-finite weights are
+ * multiplied in float32.  Over ordinary layers the result is nearer to float64
+ * than the float32 kernels' (0.35 to 0.97 of their error).  Plain float32
+ * products throughout: SIMDYOLO_HIP_AUTOTUNE=0, or an algorithm forced with
+ * sy_conv_set_algo.  sy_attention's fused kernel takes operands as three bf16
+ * parts, which hold all 24 bits whatever else is in the tile, and leaves out
+ * products below 2^-24 of the leading one.
+ *
  * Errors.  Every int-returning call returns SY_OK (0) or one of the SY_E*
  * codes; sy_last_error() returns a thread-local message.  The C# binding maps
  * SY_EINVAL -> ArgumentException, SY_EUNSUPPORTED -> NotSupportedException and
@@ -112,7 +127,7 @@ int sy_memcpy(sy_ctx* ctx, void* dst, const void* src, size_t bytes, int kind);
 /* ---------------------------------------------------------- convolution */
 
 #define SY_CONV_AUTO 0
-#define SY_CONV_IGEMM 1    /* implicit-GEMM on FP32 MFMA */
+#define SY_CONV_IGEMM 1    /* implicit GEMM, on FP32 MFMA when forced */
 #define SY_CONV_WINOGRAD 2  /* fused Winograd F(4x4,3x3): transforms + 36-plane MFMA GEMM in one kernel */
 #define SY_CONV_DIRECT 3    /* direct low-channel conv (stem; NCHW input allowed) */
 #define SY_CONV_WINOGRAD3 4 /* Winograd F(4x4,3x3) as three kernels (transform, batched GEMM, inverse) */
@@ -131,10 +146,11 @@ int sy_memcpy(sy_ctx* ctx, void* dst, const void* src, size_t bytes, int kind);
  * auto-routed conv times its candidates (the f16-split implicit GEMM and 3x3
  * patch kernels, float32 implicit GEMM tiles, the weight-stationary row kernel
  * for 1x1 and Winograd planes, the 16-channel 3x3 kernel, the three Winograd
- * forms; of these only the split kernels where they always win) with HIP
- * events and keeps the fastest,
- * as the Vulkan backend's timestamp autotune does (VulkanWinograd.cs:83-117);
- * SIMDYOLO_HIP_AUTOTUNE=0 keeps the routing rule.  SIMDYOLO_HIP_WINOGRAD=0
+ * forms; only the split kernels at 512 and more 64 x 64 output tiles) with HIP
+ * events and keeps the fastest, as the Vulkan backend's timestamp autotune
+ * does (VulkanWinograd.cs:83-117); SIMDYOLO_HIP_AUTOTUNE=0 keeps the routing
+ * rule, and so does a first run inside a graph capture whose recorded choice
+ * reads weights not packed yet.  SIMDYOLO_HIP_WINOGRAD=0
  * disables Winograd (as SIMDYOLO_WINOGRAD does for Vulkan,
  * VulkanWinograd.cs:16-35) and SIMDYOLO_HIP_WINO_FUSED=1 makes the routing
  * rule pick the fused kernel (SY_CONV_WINOGRAD) instead of the three-kernel
@@ -291,7 +307,9 @@ int sy_matmul(sy_ctx* ctx, const float* a, const float* b, float* c, int m, int 
  * conv output viewed as [B, heads, 2*key_dim + head_dim, H*W] (per pixel:
  * head-major q | k | v channels).  Writes o = v softmax(q^T k * scale)^T as
  * the NHWC view o [B, heads*head_dim, H, W] and a dense copy of v into the
- * view v (same shape) for the depthwise positional conv. */
+ * view v (same shape) for the depthwise positional conv.  o may overlap qkv
+ * or v: such calls keep the scores in scratch memory, as key dims above 32
+ * and head dims above 64 do. */
 int sy_attention(sy_ctx* ctx, const sy_tensor* qkv, int heads, int key_dim,
                  int head_dim, float scale, const sy_tensor* o, const sy_tensor* v);
 

@@ -3279,12 +3279,13 @@ static std::vector<ConvChoice> conv_candidates_all(const ConvPlan* p, const sy_t
   conv_out_size(p, x->h, x->w, &oh, &ow);
   const long long M = (long long)x->n * oh * ow;
   const int K = p->kh * p->kw * p->ic;
-  // The f16-split kernels.  Where 64 x 64 output tiles fill the CUs twice over
-  // they are the fastest of all at every layer shape of the YOLO families with
-  // at least 64 multiplied channels (1x1 384 -> 128 at 40 x 40, batch 32: 30 us
-  // against 58; 3x3 64 -> 64 at 80 x 80: 52 against 73; 3x3 stride 2 64 -> 128:
-  // 38 against 82) and no other candidate is timed; smaller grids and shallow
-  // products, where the in-workgroup split-K and row kernels can win, time all.
+  // The f16-split kernels.  Where 64 x 64 output tiles fill the CUs twice over,
+  // no other candidate is timed: of 98 such layers of YOLOv8n, s and m at 640
+  // (batch 1 to 32) they are the fastest at 97, by 1.02 to 2.5 times (1x1 384 ->
+  // 128 at 40 x 40, batch 32: 30 us against 58; 3x3 64 -> 64 at 80 x 80: 52 against
+  // 73; 3x3 stride 2 64 -> 128: 38 against 82), and 1% behind at one (1x1 48 -> 32
+  // at 160 x 160, bound by memory).  Smaller grids and shallow products, where the
+  // in-workgroup split-K and row kernels can win, time all.
   if (conv_supports(p, kIgemm) && p->finite && M * p->oc < (1LL << 40)) {
     for (int i = 0; i < x3_num_tiles(); ++i) cand.push_back(ConvChoice{kIgemm, kX3Base + i});
     const long long wide = (M + 63) / 64 * ((p->oc + 63) / 64);

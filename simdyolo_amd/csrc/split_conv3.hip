@@ -24,10 +24,9 @@
 // channels) it reads 2 TM KiB from LDS and 2 TN KiB from L1 / L2 for 3 TM TN
 // MFMAs of 32 cycles.
 //
-// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 54 us on
-// normal random inputs (44 on smaller ones: the clock follows the power), against
-// 73 us for the fastest float32 Winograd form.  The matrix cores are busy for 38%
-// of its cycles (SQ_VALU_MFMA_BUSY_CYCLES over GRBM_GUI_ACTIVE); the patch loads
+// Measured at 64 -> 64 channels, 80 x 80, batch 32 (15.1 GFLOP direct): 52 - 54 us on
+// random inputs (41 - 44 on zeros: the clock follows the power), against 73 us for the fastest float32 Winograd form.  The matrix cores are busy for 38% of its
+// cycles (SQ_VALU_MFMA_BUSY_CYCLES over GRBM_GUI_ACTIVE); the patch loads
 // (8,000 of a 128-pixel workgroup's 29,000 cycles), the epilogue (6,000)
 // and a thin last round of 1,600 workgroups on 256 CUs take the rest.
 // Workgroups that run through several tiles with the next patch loaded behind
