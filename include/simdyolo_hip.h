@@ -28,8 +28,8 @@
  * than the float32 kernels' (0.35 to 0.97 of their error).  Plain float32
  * products throughout: SIMDYOLO_HIP_AUTOTUNE=0, or an algorithm forced with
  * sy_conv_set_algo.  sy_attention's fused kernel takes operands as three bf16
- * parts, which hold all 24 bits whatever else is in the tile, and leaves out
- * products below 2^-24 of the leading one.
+ * parts, which hold all 24 bits (of values of 2^-110 and more) whatever else
+ * is in the tile, and leaves out products below 2^-24 of the leading one.
  *
  * Errors.  Every int-returning call returns SY_OK (0) or one of the SY_E*
  * codes; sy_last_error() returns a thread-local message.  The C# binding maps

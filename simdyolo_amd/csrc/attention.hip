@@ -114,25 +114,26 @@ __device__ __forceinline__ void mfma_parts(const bf16x8 (&a)[3], const bf16x8 (&
 // already the B operand of O^T = V^T P^T under the key order
 // 8 (e / 4) + 4 half + e % 4 of a 16-key step, in which V is loaded.
 //
-// Both products take float32 operands as three bf16 parts, which hold a float's 24
-// significand bits over its whole exponent range (parts below 2^-126, of values
-// below 2^-110, may be lost): no operand's precision depends on another's size, as
-// it would with f16 pairs under common scales.  Six of the nine part products are
-// taken, the rest is below 2^-24 of the product.  Where a part is not finite
-// (infinities, NaN, values that round to 2^128 in bf16) or a sum overflows, the
-// query's output is not finite either and is computed again in plain float32.
+// Both products take float32 operands as three bf16 parts (Henry, Tang and
+// Heinecke, 2019), which hold a float's 24 significand bits over its whole exponent
+// range (parts below 2^-126, of values below 2^-110, may be lost): no operand's
+// precision depends on another's size, as it would with f16 pairs under common
+// scales.  Six of the nine part products are taken, the rest is below 2^-24 of the
+// product.  Where a part is not finite (infinities, NaN, values that round to 2^128
+// in bf16) or a sum overflows, the query's output is not finite either and is
+// computed again in plain float32.
 //
-// The running maximum moves (and the sums with it) only where a score passes it by
-// kSlack; until then weights reach e^kSlack.  The test is on the difference, which
-// is exact between floats this near: the sum of maximum and slack rounds, from
-// 2^23 on to more than the slack.
+// The running maximum (online softmax: Milakov and Gimelshein, 2018) moves, and the
+// sums with it, only where a score passes it by kSlack; until then weights reach
+// e^kSlack.  The test is on the difference, which is exact between floats this near:
+// the sum of maximum and slack rounds, from 2^23 on to more than the slack.
 //
 // Bound by VALU work (the parts of K, V and P 350 operations per tile, the
 // exponentials and sums about 220, beside 36 MFMAs) and, at 400 tokens, by the
 // latency of its few tiles.  Measured, us, against two GEMMs, a softmax and a copy
 // with the scores in memory / float32 MFMAs for both products / f16 pairs: 2 heads,
-// 400 tokens, batch 16 74 / 28 / 21.4 -> 19.9, batch 1 25 / 18 / 14.5 -> 13.5;
-// 4 heads, 1,600 tokens, batch 8 858 / 206 / 141 -> 144.  Error against float64 at
+// 400 tokens, batch 16 74 / 28 / 21.6 -> 19.6, batch 1 25 / 18 / 14.5 -> 13.0;
+// 4 heads, 1,600 tokens, batch 8 858 / 206 / 141 -> 145.  Error against float64 at
 // 400 tokens 1.4e-7 (1.9e-7 with f16 pairs, 2.0e-7 with float32 MFMAs summed tile by
 // tile).  Three waves per SIMD spill registers: 178 us at 1,600 tokens.
 constexpr float kSlack = 2.5f;

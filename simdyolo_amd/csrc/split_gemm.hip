@@ -1,4 +1,5 @@
-// Float32 implicit GEMM on the f16 matrix cores.
+// Float32 implicit GEMM on the f16 matrix cores, with error-corrected products
+// (Ootomo and Yokota, 2022).
 //
 // Every float32 operand, scaled by a power of two (exact), is written as
 // hi + lo / 2048 with hi = f16(v) and lo = f16(2048 (v - hi)): v - hi is exact
